@@ -192,6 +192,19 @@ ENTRY_POINTS = {
         [C.c_void_p, C.c_int32, C.c_void_p, C.POINTER(C.c_float), C.POINTER(C.c_float), C.c_void_p, C.c_void_p,
          C.c_int32, C.c_int32, C.c_void_p, C.c_size_t, C.c_void_p],
     ),
+    "adop_bounding_box_size": (C.c_size_t, []),
+    "adop_bounding_box": (C.c_int, [C.c_void_p, C.c_int32, C.c_void_p, C.c_void_p]),
+    "adop_gather_points": (C.c_int, [C.c_void_p, C.c_int32, C.c_void_p, C.c_int32, C.c_void_p, C.c_void_p]),
+    "adop_shuffle_points": (
+        C.c_int,
+        [C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, C.c_int32, C.c_int32, C.c_void_p, C.c_void_p, C.c_void_p,
+         C.c_void_p],
+    ),
+    "adop_radius_blocks": (
+        C.c_int,
+        [C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, C.c_int32, C.c_void_p, C.c_void_p, C.c_void_p,
+         C.c_void_p, C.c_void_p],
+    ),
     "adop_profile_enable": (C.c_int, [C.c_int32]),
     "adop_profile_read": (C.c_int32, [C.POINTER(StageTime), C.c_int32]),
     "adop_last_error_string": (C.c_char_p, []),

@@ -1235,6 +1235,58 @@ adop_status adop_morton_codes(const float* position, int32_t num_points, const f
     return ADOP_OK;
 }
 
+size_t adop_bounding_box_size(void)
+{
+    return sizeof(float) * bounding_box_floats();
+}
+
+adop_status adop_bounding_box(const float* position, int32_t num_points, float* box, void* hip_stream)
+{
+    if (!position || !box) return fail(ADOP_INVALID_ARG, "null argument");
+    if (num_points < 1) return fail(ADOP_INVALID_ARG, "empty cloud");
+    launch_bounding_box((const float4*)position, num_points, box, (hipStream_t)hip_stream);
+    ADOP_HIP_CHECK(hipGetLastError());
+    return ADOP_OK;
+}
+
+adop_status adop_gather_points(const float* position, int32_t num_points, const int64_t* index, int32_t count,
+                               float* out_position, void* hip_stream)
+{
+    if (!position || !index || !out_position || num_points < 0 || count < 0) return fail(ADOP_INVALID_ARG, "null argument");
+    if (count == 0) return ADOP_OK;
+    launch_gather_rows((const float4*)position, num_points, (const long long*)index, count, (float4*)out_position,
+                       (hipStream_t)hip_stream);
+    ADOP_HIP_CHECK(hipGetLastError());
+    return ADOP_OK;
+}
+
+adop_status adop_shuffle_points(const float* position, const int32_t* normal, const int64_t* order,
+                                const int64_t* block_order, int32_t num_points, int32_t block_size, float* out_position,
+                                int32_t* out_normal, int32_t* out_id, void* hip_stream)
+{
+    if (!position || !order || !out_position || !out_id || (!normal) != (!out_normal))
+        return fail(ADOP_INVALID_ARG, "null argument");
+    if (num_points < 1 || block_size < 1) return fail(ADOP_INVALID_ARG, "empty cloud or block");
+    if (num_points >= block_size && !block_order) return fail(ADOP_INVALID_ARG, "null argument");
+    launch_shuffle_gather((const float4*)position, normal, (const long long*)order, (const long long*)block_order, num_points,
+                          block_size, (float4*)out_position, out_normal, out_id, (hipStream_t)hip_stream);
+    ADOP_HIP_CHECK(hipGetLastError());
+    return ADOP_OK;
+}
+
+adop_status adop_radius_blocks(const float* position, const int32_t* normal, const int32_t* id, const float* distance,
+                               const double* uniform, int32_t num_points, float* out_position, int32_t* out_normal,
+                               float* out_data, int64_t* out_order, void* hip_stream)
+{
+    if (!position || !id || !distance || !uniform || !out_position || !out_data || !out_order || (!normal) != (!out_normal))
+        return fail(ADOP_INVALID_ARG, "null argument");
+    if (num_points < 1) return fail(ADOP_INVALID_ARG, "empty cloud");
+    launch_radius_blocks((const float4*)position, normal, id, distance, uniform, num_points, (float4*)out_position,
+                         out_normal, (float4*)out_data, (long long*)out_order, (hipStream_t)hip_stream);
+    ADOP_HIP_CHECK(hipGetLastError());
+    return ADOP_OK;
+}
+
 adop_status adop_profile_enable(int32_t enable)
 {
     g_profile = enable != 0;

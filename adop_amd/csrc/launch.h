@@ -42,6 +42,14 @@ void launch_camera_distance(const float4* position, int n, const ViewConst* view
                             hipStream_t st);
 void launch_close_points(const float4* sorted, int n, const KnnGrid* g, const uint32_t* offset, const float* radius,
                          int32_t* state, uint32_t* round_count, int round, hipStream_t st);
+size_t bounding_box_floats();  // the box and the partial boxes behind it
+void launch_bounding_box(const float4* position, int n, float* box, hipStream_t st);
+void launch_gather_rows(const float4* src, int rows, const long long* index, int n, float4* dst, hipStream_t st);
+void launch_shuffle_gather(const float4* position, const int32_t* normal, const long long* order, const long long* perm,
+                           int n, int block, float4* out_position, int32_t* out_normal, int32_t* out_id, hipStream_t st);
+void launch_radius_blocks(const float4* position, const int32_t* normal, const int32_t* id, const float* distance,
+                          const double* uniform, int n, float4* out_position, int32_t* out_normal, float4* out_data,
+                          long long* out_order, hipStream_t st);
 void launch_morton(const float4* position, int n, const float* mn, const float* scale, unsigned long long* code,
                    hipStream_t st);
 // The launchers take the tuning switches of the call as an argument (one snapshot per call: adop_forward / adop_backward).

@@ -14,39 +14,64 @@ from . import _capi
 from .render import _check, _stream_ptr
 
 
+def _ptr(t):
+    return None if t is None else C.c_void_p(t.data_ptr())
+
+
+def _checked_position(position):
+    assert position.is_cuda and position.dtype == torch.float32 and position.dim() == 2 and position.shape[1] == 4
+    return position.contiguous()
+
+
+_RADIUS_BLOCK = 256  # the block size of adop_radius_blocks
+
+
 def _bbox(position):
-    lo, hi = torch.aminmax(position, dim=0)  # one pass over the contiguous [N,4] array
-    both = torch.stack([lo[:3], hi[:3]]).cpu()
-    return (C.c_float * 3)(*both[0].tolist()), (C.c_float * 3)(*both[1].tolist())
+    lib = _capi.load_library()
+    box = torch.empty(int(lib.adop_bounding_box_size()) // 4, dtype=torch.float32, device=position.device)
+    _check(lib.adop_bounding_box(_ptr(position), int(position.shape[0]), _ptr(box), _stream_ptr()), lib)
+    host = box[:6].tolist()
+    return (C.c_float * 3)(*host[:3]), (C.c_float * 3)(*host[3:])
+
+
+def _knn_distance(position, rank, box):
+    n = int(position.shape[0])
+    lib = _capi.load_library()
+    out = torch.empty(n, dtype=torch.float32, device=position.device)
+    ws = torch.empty(int(lib.adop_knn_workspace_size(n)), dtype=torch.uint8, device=position.device)
+    rc = lib.adop_knn_distance(_ptr(position), n, int(rank), *box, _ptr(out), _ptr(ws), int(ws.numel()), _stream_ptr())
+    _check(rc, lib)
+    return out
+
+
+def _morton_codes(position, box):
+    lib = _capi.load_library()
+    codes = torch.empty(int(position.shape[0]), dtype=torch.int64, device=position.device)
+    _check(lib.adop_morton_codes(_ptr(position), int(position.shape[0]), *box, _ptr(codes), _stream_ptr()), lib)
+    return codes
+
+
+def _gather_points(position, index):
+    """position[index] for rows of 4 floats (torch's own gather takes ten times as long, and its rows come back wrong
+    from 2^26 on)."""
+    lib = _capi.load_library()
+    out = torch.empty(int(index.shape[0]), 4, dtype=torch.float32, device=position.device)
+    _check(lib.adop_gather_points(_ptr(position), int(position.shape[0]), _ptr(index), int(index.shape[0]), _ptr(out),
+                                  _stream_ptr()), lib)
+    return out
 
 
 def KNearestNeighbourDistance(position, rank=4):
     """Distance of every point to its ``rank``-th nearest other point: ``data[i](0)`` of ComputeRadius
     (SceneData.cpp:441-463).  position: [N,4] f32 on the device."""
-    assert position.is_cuda and position.dtype == torch.float32 and position.dim() == 2 and position.shape[1] == 4
-    position = position.contiguous()
-    n = int(position.shape[0])
-    lib = _capi.load_library()
-    out = torch.empty(n, dtype=torch.float32, device=position.device)
-    ws = torch.empty(int(lib.adop_knn_workspace_size(n)), dtype=torch.uint8, device=position.device)
-    mn, mx = _bbox(position)
-    rc = lib.adop_knn_distance(C.c_void_p(position.data_ptr()), n, int(rank), mn, mx, C.c_void_p(out.data_ptr()),
-                               C.c_void_p(ws.data_ptr()), int(ws.numel()), _stream_ptr())
-    _check(rc, lib)
-    return out
+    position = _checked_position(position)
+    return _knn_distance(position, rank, _bbox(position))
 
 
 def MortonCodes(position):
     """63-bit Morton code of every point inside the cloud's bounding box (the key of ReorderMorton64)."""
-    assert position.is_cuda and position.dtype == torch.float32 and position.dim() == 2 and position.shape[1] == 4
-    position = position.contiguous()
-    n = int(position.shape[0])
-    lib = _capi.load_library()
-    codes = torch.empty(n, dtype=torch.int64, device=position.device)
-    mn, mx = _bbox(position)
-    rc = lib.adop_morton_codes(C.c_void_p(position.data_ptr()), n, mn, mx, C.c_void_p(codes.data_ptr()), _stream_ptr())
-    _check(rc, lib)
-    return codes
+    position = _checked_position(position)
+    return _morton_codes(position, _bbox(position))
 
 
 def PointDistanceToCamera(position, poses_se3, intrinsics, frames):
@@ -160,17 +185,38 @@ def PreprocessPointCloud(position, normal=None, rank=4, block_size=256, seed=0):
     w, normal, data [N,4], order) where ``order`` maps new to original point ids."""
     gen = torch.Generator(device="cpu").manual_seed(int(seed))
     gen_dev = torch.Generator(device=position.device).manual_seed(int(seed))  # the per-point numbers are drawn on the device
-    position = position.contiguous()
-    order = ReorderMorton64(position)
-    order = order[RandomBlockShuffle(int(position.shape[0]), block_size, gen)]
-    position = position[order].contiguous()
-    data = ComputeRadius(position, rank, gen_dev)
-    by_radius = SortBlocksByRadius(data[:, 3], block_size)
-    order = order[by_radius]
-    position = position[by_radius].clone()
-    data = data[by_radius].contiguous()
-    position[:, 3] = data[:, 3]
-    return position, (None if normal is None else normal[order].contiguous()), data, order
+    position = _checked_position(position)
+    n = int(position.shape[0])
+    if block_size != _RADIUS_BLOCK or (normal is not None and (normal.dtype != torch.int32 or normal.numel() != n)):
+        order = ReorderMorton64(position)
+        order = order[RandomBlockShuffle(n, block_size, gen)]
+        position = _gather_points(position, order)
+        data = ComputeRadius(position, rank, gen_dev)
+        by_radius = SortBlocksByRadius(data[:, 3], block_size)
+        order = order[by_radius]
+        position = _gather_points(position, by_radius)
+        data = _gather_points(data, by_radius)
+        position[:, 3] = data[:, 3]
+        return position, (None if normal is None else normal[order].contiguous()), data, order
+    # The same steps in passes over whole points: one gather along both permutations, one kernel for the radii and the
+    # order inside the blocks.  One bounding box serves the codes and the search: the points stay the same.
+    lib = _capi.load_library()
+    shape = None if normal is None else normal.shape
+    normal = None if normal is None else normal.contiguous()
+    box = _bbox(position)
+    order = torch.sort(_morton_codes(position, box), stable=True).indices
+    blocks = torch.randperm(n // block_size, generator=gen, device="cpu").to(position.device)
+    shuffled, ids = torch.empty_like(position), torch.empty(n, dtype=torch.int32, device=position.device)
+    shuffled_normal = None if normal is None else torch.empty_like(normal)
+    _check(lib.adop_shuffle_points(_ptr(position), _ptr(normal), _ptr(order), _ptr(blocks), n, block_size, _ptr(shuffled),
+                                   _ptr(shuffled_normal), _ptr(ids), _stream_ptr()), lib)
+    distance = _knn_distance(shuffled, rank, box)
+    uniform = torch.rand(n, generator=gen_dev, dtype=torch.float64, device=position.device)
+    out, data = torch.empty_like(position), torch.empty_like(position)
+    out_normal = None if normal is None else torch.empty(shape, dtype=torch.int32, device=position.device)
+    _check(lib.adop_radius_blocks(_ptr(shuffled), _ptr(shuffled_normal), _ptr(ids), _ptr(distance), _ptr(uniform), n,
+                                  _ptr(out), _ptr(out_normal), _ptr(data), _ptr(order), _stream_ptr()), lib)
+    return out, out_normal, data, order
 
 
 def AttachDropOutRadii(hs, rank=4, block_size=256, seed=0):

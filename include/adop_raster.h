@@ -347,6 +347,28 @@ adop_status adop_close_points(const float* position, int32_t num_points, const f
 adop_status adop_morton_codes(const float* position, int32_t num_points, const float* bbox_min, const float* bbox_max,
                               uint64_t* out_codes, void* hip_stream);
 
+/* The passes of SceneData's initial processing (SceneData.cpp:101-104) that move the cloud.
+ * adop_bounding_box: box [adop_bounding_box_size() bytes, device] starts with min x, y, z, max x, y, z (not a number on an
+ * axis where a coordinate is not), scratch behind them.
+ * adop_gather_points: out_position[i] = position[index[i]], rows of 4 floats; an index that names no point gives zeros.
+ * adop_shuffle_points: the cloud along `order` (a permutation of its N points) with its blocks of block_size points
+ * shuffled (RandomBlockShuffle, :102): point i of the result is point order[block_order[i / block_size] * block_size +
+ * i % block_size]; the points behind the last whole block keep their place in `order`.  out_id receives the point ids;
+ * normal / out_normal may be NULL.
+ * adop_radius_blocks: ComputeRadius' radii (:462-483) from the neighbour distance d of every point and a uniform number u
+ * of (0, 1), data = (d, 0, sqrt(1 / u), d * sqrt(1 / u)), and SortBlocksByRadius (:671-684) for blocks of 256 points
+ * (stable, a last shorter block keeps its order): position with the radius in w, normals, data and ids in that order. */
+size_t adop_bounding_box_size(void);
+adop_status adop_bounding_box(const float* position, int32_t num_points, float* box, void* hip_stream);
+adop_status adop_gather_points(const float* position, int32_t num_points, const int64_t* index, int32_t count,
+                               float* out_position, void* hip_stream);
+adop_status adop_shuffle_points(const float* position, const int32_t* normal, const int64_t* order,
+                                const int64_t* block_order, int32_t num_points, int32_t block_size, float* out_position,
+                                int32_t* out_normal, int32_t* out_id, void* hip_stream);
+adop_status adop_radius_blocks(const float* position, const int32_t* normal, const int32_t* id, const float* distance,
+                               const double* uniform, int32_t num_points, float* out_position, int32_t* out_normal,
+                               float* out_data, int64_t* out_order, void* hip_stream);
+
 /* Stage timers.  The reference wraps each stage in SAIGA_OPTIONAL_TIME_MEASURE(name, info->timer_system)
  * (PointRenderer.cu:906,913,919,1095,1414,1430,1447,1565,1594,1602,1610); here HIP events are recorded on the
  * caller's stream around each stage while profiling is enabled on the calling thread.  Stage names are the

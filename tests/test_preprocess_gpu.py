@@ -250,3 +250,46 @@ def test_knn_distance_with_far_outliers():
     assert np.allclose(got[check], want, rtol=2e-6, atol=1e-9)
     print("seconds", seconds)
     assert seconds < 1.0, seconds  # (~0.01 s; with the grid over the bounding box, all in one cell: 2.6 s)
+
+
+@pytest.mark.parametrize("n", [5, 255, 256, 257, 1024, 4099])
+def test_fused_preparation_equals_the_single_steps(n):
+    """PreprocessPointCloud moves the cloud in fused passes; the steps one by one give the same bits.  Sizes around the
+    256-point block and the 1024 rows of a gather workgroup; ties in the radius (coincident points) keep their order."""
+    import torch
+    from adop_amd import preprocess as pp
+
+    announce(f"PreprocessPointCloud, fused passes, N={n}")
+    g = np.random.default_rng(n)
+    p = torch.from_numpy(g.random((n, 4)).astype(np.float32)).cuda()
+    p[n // 2:, :3] = p[0, :3] if n > 1024 else p[n // 2:, :3]
+    normal = torch.arange(n, dtype=torch.int32, device="cuda").reshape(-1, 1)
+    got = pp.PreprocessPointCloud(p, normal, seed=7)
+    order = pp.ReorderMorton64(p)[pp.RandomBlockShuffle(n, 256, torch.Generator().manual_seed(7))]
+    moved = p[order]
+    data = pp.ComputeRadius(moved, 4, torch.Generator(device="cuda").manual_seed(7))
+    by_radius = pp.SortBlocksByRadius(data[:, 3])
+    want = moved[by_radius]
+    want[:, 3] = data[by_radius, 3]
+    for a, b in zip(got, (want, normal[order[by_radius]], data[by_radius], order[by_radius])):
+        assert a.shape == b.shape and a.dtype == b.dtype and torch.equal(a, b)
+    one = pp.PreprocessPointCloud(p, None, block_size=64, seed=7)
+    assert one[1] is None and torch.equal(one[0][:, :3], p[one[3], :3])
+
+
+@pytest.mark.parametrize("n", [1, 64, 1023, 1025, 300_001])
+def test_bounding_box_and_gather(n):
+    import torch
+    from adop_amd import preprocess as pp
+
+    announce(f"bounding box, gather of rows, N={n}")
+    g = np.random.default_rng(n)
+    p = torch.from_numpy(g.standard_normal((n, 4)).astype(np.float32)).cuda()
+    lo, hi = pp._bbox(p)
+    assert np.array_equal(np.float32(list(lo)), p[:, :3].amin(0).cpu().numpy())
+    assert np.array_equal(np.float32(list(hi)), p[:, :3].amax(0).cpu().numpy())
+    index = torch.from_numpy(g.integers(0, n, n + 3)).cuda()
+    assert torch.equal(pp._gather_points(p, index), p[index])
+    p[n - 1, 1] = float("nan")
+    with pytest.raises(RuntimeError, match="not finite"):
+        pp.MortonCodes(p)
