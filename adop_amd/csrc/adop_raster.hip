@@ -994,71 +994,62 @@ adop_status adop_apply_tangent(double* tangent, double* poses_se3, int32_t num_p
     return ADOP_OK;
 }
 
-// Grids of the nearest-neighbour search: both are sized on the device (preprocess_kernels.hip), the second one within a
-// budget of cells that grows with the cloud.
-static uint32_t knn_max_cells(int32_t num_points)
+// Bricks of the search grid: the grid is sized on the device (preprocess_kernels.hip) within a budget that grows with the
+// cloud.
+static size_t knn_max_bricks(int32_t num_points)
 {
-    size_t want = (size_t)(num_points > 0 ? num_points : 0) * 16;
-    if (want < ((size_t)1 << 22)) want = (size_t)1 << 22;  // > kKnnCoarseDim^3
-    if (want > ((size_t)1 << 27)) want = (size_t)1 << 27;
-    return (uint32_t)want;
+    const size_t want = (size_t)(num_points > 0 ? num_points : 0) / 8;  // 16 cells per point
+    return want < 32768 ? 32768 : (want > kKnnMaxBricks ? kKnnMaxBricks : want);
 }
 
-constexpr uint32_t kKnnFirstCells = 160u * 160u * 160u;  // the first grid has at most 160 cells per axis
+constexpr uint32_t kKnnFirstCells = 160u * 160u * 160u;  // the coarse grid has at most 160 cells per axis
 
 struct KnnWorkspace
 {
-    KnnGrid *grid, *grid0;  // second (search) grid and first grid, device
+    KnnGrid *grid, *grid0;  // search grid and coarse grid, device
     float* sample;
-    uint32_t *count, *offset, *chunk;  // second grid
-    uint32_t *count0, *offset0;        // first grid
-    float4 *sorted, *sorted0;
+    KnnBricks bricks;
+    uint32_t *count0, *start0;  // coarse grid
     uint32_t *list, *list2, *counts;
     size_t total;
+    KnnView view() const { return KnnView{grid, bricks.sorted, bricks.slot, bricks.cell_start}; }
 };
 
 static KnnWorkspace knn_layout(void* workspace, int32_t num_points)
 {
-    const uint32_t cells = knn_max_cells(num_points);
-    const size_t n       = (size_t)(num_points > 0 ? num_points : 0);
-    size_t o             = 0;
-    auto take            = [&](size_t bytes) {
+    const size_t bricks = knn_max_bricks(num_points);
+    const size_t n      = (size_t)(num_points > 0 ? num_points : 0);
+    const size_t slots  = bricks < n ? bricks : n;
+    size_t o            = 0;
+    auto take           = [&](size_t bytes) {
         const size_t at = o;
         o               = align_up(o + bytes, 256);
-        return at;
+        return (void*)((uintptr_t)workspace + at);
     };
-    const size_t o_grid = take(sizeof(KnnGrid)), o_grid0 = take(sizeof(KnnGrid));
-    const size_t o_sample  = take(sizeof(float) * 2048);
-    const size_t o_counts  = take(sizeof(uint32_t) * 2);
-    const size_t o_count   = take(sizeof(uint32_t) * (size_t)cells);
-    const size_t o_offset  = take(sizeof(uint32_t) * ((size_t)cells + 1));
-    const size_t o_chunk   = take(sizeof(uint32_t) * knn_chunk_words(cells));
-    const size_t o_count0  = take(sizeof(uint32_t) * (size_t)kKnnFirstCells);
-    const size_t o_offset0 = take(sizeof(uint32_t) * ((size_t)kKnnFirstCells + 1));
-    const size_t o_sorted  = take(sizeof(float4) * n);
-    const size_t o_sorted0 = take(sizeof(float4) * n);
-    const size_t o_list    = take(sizeof(uint32_t) * n);
-    const size_t o_list2   = take(sizeof(uint32_t) * n);
     KnnWorkspace w;
     memset(&w, 0, sizeof(w));
-    w.total = o;
-    if (workspace)
-    {
-        char* base = (char*)workspace;
-        w.grid     = (KnnGrid*)(base + o_grid);
-        w.grid0    = (KnnGrid*)(base + o_grid0);
-        w.sample   = (float*)(base + o_sample);
-        w.counts   = (uint32_t*)(base + o_counts);
-        w.count    = (uint32_t*)(base + o_count);
-        w.offset   = (uint32_t*)(base + o_offset);
-        w.chunk    = (uint32_t*)(base + o_chunk);
-        w.count0   = (uint32_t*)(base + o_count0);
-        w.offset0  = (uint32_t*)(base + o_offset0);
-        w.sorted   = (float4*)(base + o_sorted);
-        w.sorted0  = (float4*)(base + o_sorted0);
-        w.list     = (uint32_t*)(base + o_list);
-        w.list2    = (uint32_t*)(base + o_list2);
-    }
+    w.grid   = (KnnGrid*)take(sizeof(KnnGrid));
+    w.grid0  = (KnnGrid*)take(sizeof(KnnGrid));
+    w.sample = (float*)take(sizeof(float) * 1024);
+    w.counts = (uint32_t*)take(sizeof(uint32_t) * 4);  // three list counters, the number of slots
+    KnnBricks& b = w.bricks;
+    b.grid       = w.grid;
+    b.max_bricks = bricks;
+    b.num_slots  = w.counts + 3;
+    b.chunk_sum  = (unsigned long long*)take(sizeof(uint32_t) * knn_chunk_words());
+    b.count      = (uint32_t*)take(sizeof(uint32_t) * bricks);
+    b.start      = (uint32_t*)take(sizeof(uint32_t) * bricks);
+    b.slot       = (uint32_t*)take(sizeof(uint32_t) * bricks);
+    b.slot_brick = (uint32_t*)take(sizeof(uint32_t) * slots);
+    b.cell_start = (uint32_t*)take(sizeof(uint32_t) * (slots * kBrickCells + 1));
+    b.rank       = (uint32_t*)take(sizeof(uint32_t) * n);
+    b.scratch    = (float4*)take(sizeof(float4) * n);  // (also the points in the order of the coarse grid)
+    b.sorted     = (float4*)take(sizeof(float4) * n);
+    w.count0     = (uint32_t*)take(sizeof(uint32_t) * (size_t)kKnnFirstCells);
+    w.start0     = (uint32_t*)take(sizeof(uint32_t) * ((size_t)kKnnFirstCells + 1));
+    w.list       = (uint32_t*)take(sizeof(uint32_t) * n);
+    w.list2      = (uint32_t*)take(sizeof(uint32_t) * n);
+    w.total      = o;
     return w;
 }
 
@@ -1086,18 +1077,19 @@ static adop_status knn_prepare(const float* position, int32_t num_points, const 
         box.ext[k] = bbox_max[k] - bbox_min[k];
         if (!(box.ext[k] >= 0) || !(box.ext[k] < 1.0e30f)) return fail(ADOP_INVALID_ARG, "bounding box is not finite");
     }
-    const uint32_t max_cells = knn_max_cells(num_points);
-    const float4* pos        = (const float4*)position;
-    // first grid (kept: the search falls back on it for points in sparse parts of the cloud)
+    const float4* pos = (const float4*)position;
+    const int stride  = knn_sample_stride(num_points);
+    const int n0      = (num_points + stride - 1) / stride;
+    const int samples = knn_num_samples(n0);
     launch_knn_first_grid(pos, num_points, box, out->grid0, stream);
-    launch_knn_build(pos, num_points, out->grid0, kKnnFirstCells, out->count0, out->offset0, out->chunk, out->sorted0,
-                     stream);
-    const int samples = knn_num_samples(num_points);
-    if (!launch_knn_sample(sample_rank, out->sorted0, num_points, out->grid0, out->offset0, out->sample, samples, stream))
+    launch_knn_coarse(pos, n0, stride, out->grid0, out->count0, out->start0, out->bricks.rank, out->bricks.chunk_sum,
+                      out->bricks.scratch, nullptr, stream);
+    if (!launch_knn_sample(stride > 1 ? 1 : sample_rank, out->bricks.scratch, n0, out->grid0, out->start0, out->sample,
+                           samples, stream))
         return fail(ADOP_INVALID_ARG, "rank must be 1..8");
-    // second grid
-    launch_knn_refine_grid(out->sample, samples, out->grid0, out->grid, max_cells, stream);
-    launch_knn_build(pos, num_points, out->grid, max_cells, out->count, out->offset, out->chunk, out->sorted, stream);
+    launch_knn_refine_grid(out->sample, samples, sample_rank, stride, out->grid0, out->grid,
+                           (uint32_t)out->bricks.max_bricks, out->counts, stream);
+    launch_knn_bricks(pos, num_points, out->bricks, stream);
     return ADOP_OK;
 }
 
@@ -1113,9 +1105,9 @@ adop_status adop_knn_distance(const float* position, int32_t num_points, int32_t
     adop_status st =
         knn_prepare(position, num_points, bbox_min, bbox_max, rank, workspace, workspace_bytes, true, stream, &w);
     if (st != ADOP_OK) return st;
-    if ((st = fill_async(w.counts, 2 * sizeof(uint32_t), 0, stream)) != ADOP_OK) return st;
-    KnnSearchArg a{w.grid, w.grid0, w.sorted, w.sorted0, w.offset, w.offset0, w.list, w.list2, w.counts};
-    if (!launch_knn_search(rank, num_points, a, out_distance, stream))
+    const KnnSearchArg a{w.view(), w.grid0, w.count0, w.start0, w.bricks.rank, w.bricks.chunk_sum, w.bricks.scratch, w.list,
+                         w.list2, w.counts};
+    if (!launch_knn_search(rank, (const float4*)position, num_points, a, out_distance, stream))
         return fail(ADOP_INVALID_ARG, "rank must be 1..8");
     ADOP_HIP_CHECK(hipGetLastError());
     return ADOP_OK;
@@ -1138,7 +1130,7 @@ adop_status adop_close_points(const float* position, int32_t num_points, const f
     if (!resume && (st = fill_async(state, sizeof(int32_t) * (size_t)num_points, 0, stream)) != ADOP_OK) return st;
     if ((st = fill_async(round_undecided, sizeof(uint32_t) * (size_t)num_rounds, 0, stream)) != ADOP_OK) return st;
     for (int r = 0; r < num_rounds; ++r)
-        launch_close_points(w.sorted, num_points, w.grid, w.offset, radius, state, round_undecided, r, stream);
+        launch_close_points(w.view(), num_points, radius, state, round_undecided, r, stream);
     ADOP_HIP_CHECK(hipGetLastError());
     return ADOP_OK;
 }

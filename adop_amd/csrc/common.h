@@ -129,14 +129,27 @@ struct ParamArg
 };
 
 // Uniform grid of the nearest-neighbour search: cubic cells of edge `cell` from `min`, dim cells per axis.  The grid
-// lives in device memory: the second one of a search is sized on the device from sampled neighbour distances.
+// lives in device memory: it is sized there from sampled neighbour distances.
 struct KnnGrid
 {
     float min[3];
     float ext[3];  // size of the bounding box
     float cell, inv_cell;
     int32_t dim[3];
-    uint32_t cells;  // dim[0] * dim[1] * dim[2]
+    uint32_t cells;  // coarse grid: dim[0] * dim[1] * dim[2]
+    int32_t bricks_x, bricks_y;  // search grid: bricks of kBrickCells cells along x and y
+    uint32_t bricks;             // all of them
+};
+constexpr int kBrickCells      = 128;
+constexpr size_t kKnnMaxBricks = (size_t)1 << 21;
+
+// What a search reads of the search grid (all device memory).
+struct KnnView
+{
+    const KnnGrid* grid;
+    const float4* sorted;        // the points (x, y, z, bits of the id), brick after brick, cell after cell
+    const uint32_t* slot;        // per brick: its row of cell_start, or all ones where it holds no point
+    const uint32_t* cell_start;  // [slots * kBrickCells + 1] first point of every cell of the bricks that hold points
 };
 
 struct ViewChunk

@@ -21,27 +21,42 @@ void launch_fill_u32(uint32_t* p, size_t n, uint32_t v, hipStream_t st);
 void launch_clear(const Levels& lv, int first_level, int grid, float* accum, size_t accum_floats, uint32_t* zero_u32,
                   int zero_n, const ViewPrep& vp, hipStream_t st, Gate gate = {nullptr, 0}, adop_stats* zero_stats = nullptr);
 void launch_knn_first_grid(const float4* position, int n, const KnnGrid& box, KnnGrid* dst, hipStream_t st);
-void launch_knn_refine_grid(const float* sample, int samples, const KnnGrid* first, KnnGrid* g, uint32_t budget,
-                            hipStream_t st);
+int knn_sample_stride(int n);  // the grid of a cloud of n points is sized on every stride-th of them
 int knn_num_samples(int n);
-size_t knn_chunk_words(uint32_t max_cells);  // uint32 words of the scan's scratch array
-void launch_knn_build(const float4* position, int n, const KnnGrid* g, uint32_t max_cells, uint32_t* count,
-                      uint32_t* offset, uint32_t* chunk_sum, float4* sorted, hipStream_t st);
+size_t knn_chunk_words();  // uint32 words of the scan's scratch array
+void launch_knn_refine_grid(const float* sample, int samples, int rank, int stride, const KnnGrid* first, KnnGrid* g,
+                            uint32_t budget, uint32_t* list_counts, hipStream_t st);
+void launch_knn_coarse(const float4* position, int n, int stride, const KnnGrid* g, uint32_t* count, uint32_t* start,
+                       uint32_t* rank, unsigned long long* chunk_sum, float4* sorted, const uint32_t* gate, hipStream_t st);
+struct KnnBricks
+{
+    const KnnGrid* grid;
+    size_t max_bricks;
+    uint32_t *count, *start, *slot;          // [max_bricks]
+    uint32_t *slot_brick, *cell_start;       // [slots], [slots * kBrickCells + 1]
+    uint32_t* num_slots;
+    uint32_t* rank;                          // [n]
+    unsigned long long* chunk_sum;
+    float4 *scratch, *sorted;                // [n]
+};
+void launch_knn_bricks(const float4* position, int n, const KnnBricks& b, hipStream_t st);
 bool launch_knn_sample(int rank, const float4* sorted, int n, const KnnGrid* g, const uint32_t* offset, float* out,
                        int samples, hipStream_t st);
 struct KnnSearchArg
 {
-    const KnnGrid *grid, *grid0;          // second / first grid (device)
-    const float4 *sorted, *sorted0;       // the points in cell order of either grid
-    const uint32_t *offset, *offset0;
-    uint32_t *list, *list2;               // [n] points left over by the first / second stage
-    uint32_t* counts;                     // [2] their numbers, zero at the start
+    KnnView view;
+    const KnnGrid* grid0;  // coarse grid, and the arrays to put the whole cloud into it
+    uint32_t *count0, *start0, *rank;
+    unsigned long long* chunk_sum;
+    float4* sorted0;
+    uint32_t *list, *list2;  // [n] points left over by a stage
+    uint32_t* counts;        // [3] their numbers, zero at the start
 };
-bool launch_knn_search(int rank, int n, const KnnSearchArg& a, float* out, hipStream_t st);
+bool launch_knn_search(int rank, const float4* position, int n, const KnnSearchArg& a, float* out, hipStream_t st);
 void launch_camera_distance(const float4* position, int n, const ViewConst* views, int num_frames, float* out,
                             hipStream_t st);
-void launch_close_points(const float4* sorted, int n, const KnnGrid* g, const uint32_t* offset, const float* radius,
-                         int32_t* state, uint32_t* round_count, int round, hipStream_t st);
+void launch_close_points(const KnnView& view, int n, const float* radius, int32_t* state, uint32_t* round_count, int round,
+                         hipStream_t st);
 size_t bounding_box_floats();  // the box and the partial boxes behind it
 void launch_bounding_box(const float4* position, int n, float* box, hipStream_t st);
 void launch_gather_rows(const float4* src, int rows, const long long* index, int n, float4* dst, hipStream_t st);

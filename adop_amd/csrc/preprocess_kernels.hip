@@ -3,17 +3,16 @@
 // kd-tree k-nearest-neighbour search per point on the host) and the Morton code of every point (the key of
 // ReorderMorton64, SceneData.cpp:101).
 //
-// Nearest neighbours: the points are binned into a uniform grid (count, prefix sum, scatter: the structure of the
-// rasterizer's tile bins), stored cell after cell, and every point then walks the shells of cells around its own
-// until the n-th best distance cannot be beaten from outside the cube searched so far.  The distances are formed as
-// sqrt((dx*dx + dy*dy) + dz*dz) in fp32; the result is the n-th smallest of them over all other points, whatever the
-// search order and whatever the grid, so a brute-force search over the same arithmetic gives the same bits.
+// Nearest neighbours: the points are put into the cells of a uniform grid, stored cell after cell, and every point then
+// walks the cube of cells around its own until the n-th best distance cannot be beaten from outside the cube.  The
+// distances are formed as sqrt((dx*dx + dy*dy) + dz*dz) in fp32; the result is the n-th smallest of them over all other
+// points, whatever the search order and whatever the grid, so a brute-force search over the same arithmetic gives the
+// same bits.
 // The cost is the number of candidates, which the cell size decides, and the right cell size depends on how the cloud
 // fills space (scans are surfaces: a grid sized by volume puts hundreds of points into the few cells that have any).
-// So there are two grids, both sized on the device (no host round trip): a first one sized by volume, on which 2048
-// sample points are searched, and a second one with cells of twice the median distance those found.  All points are
-// searched on the second grid (2 shells at most), what that leaves on the first (4 shells), and the stray points
-// neither settles against all points.
+// So the search grid is sized on the device (no host round trip) from the neighbour distances of 1024 sample points,
+// measured in a part of the cloud (every 16th point) on a coarse grid sized by volume.  The coarse grid over the whole cloud is
+// built only when the search grid leaves points undecided (sparse parts of the cloud), which the device finds out.
 #include "common.h"
 #include "launch.h"
 
@@ -21,6 +20,16 @@
 
 namespace adop
 {
+// The search grid is stored in bricks of 8 x 4 x 4 cells: the points brick after brick and, inside a brick, cell after
+// cell with x fastest.  A cloud of 10 M points asks for 100 M cells and more, nearly all of them empty: the bricks are
+// counted in one dense table (a 128th of the cells) and only the bricks that hold points have a row in the table of the
+// cells' first points.  (A dense table of cells took 650 us to clear and sum up for 10 M points on 1000 patches, and
+// its 10 M atomics on single cells 720 us; the bricks and the sort inside them take 235 us in all.)  A wavefront of consecutive points stays inside a brick or two, and so do
+// the cells it searches.
+constexpr int kBrickX = 3, kBrickY = 2, kBrickZ = 2;  // log2 of the cells per brick
+static_assert(kBrickX + kBrickY + kBrickZ == 7 && (1 << 7) == kBrickCells, "128 cells");
+constexpr uint32_t kNoBrick = 0xFFFFFFFFu;
+
 // Cell of a point; points outside the grid's box (the box leaves the far tails of the cloud out) belong to the nearest
 // boundary cell.
 __device__ __forceinline__ int3 grid_cell(const KnnGrid& g, float x, float y, float z)
@@ -36,80 +45,363 @@ __device__ __forceinline__ uint32_t grid_index(const KnnGrid& g, int cx, int cy,
     return ((uint32_t)cz * (uint32_t)g.dim[1] + (uint32_t)cy) * (uint32_t)g.dim[0] + (uint32_t)cx;
 }
 
-// pass 0: points per cell; pass 1: the points cell after cell, (x, y, z, bits of the point id)
-__global__ __launch_bounds__(kBlock) void knn_bin_kernel(int pass, const float4* __restrict__ position, int n,
-                                                         const KnnGrid* __restrict__ gp, uint32_t* __restrict__ count,
-                                                         const uint32_t* __restrict__ offset, float4* __restrict__ sorted)
+// first brick of the row of bricks that holds the cells (., cy, cz); brick of cell cx: + (cx >> kBrickX)
+__device__ __forceinline__ uint32_t brick_row(const KnnGrid& g, int cy, int cz)
 {
-    const int i = blockIdx.x * kBlock + threadIdx.x;
-    if (i >= n) return;
-    const KnnGrid g = *gp;
-    const float4 p    = nt_load4(position + i);
-    const int3 c      = grid_cell(g, p.x, p.y, p.z);
-    const uint32_t ci = grid_index(g, c.x, c.y, c.z);
-    if (pass == 0)
-        atomicAdd(&count[ci], 1u);
-    else  // the counter runs down to zero: slots are handed out from the end of the cell's range
-        sorted[offset[ci] + atomicSub(&count[ci], 1u) - 1u] = make_float4(p.x, p.y, p.z, __uint_as_float((uint32_t)i));
+    return ((uint32_t)(cz >> kBrickZ) * (uint32_t)g.bricks_y + (uint32_t)(cy >> kBrickY)) * (uint32_t)g.bricks_x;
+}
+__device__ __forceinline__ uint32_t brick_local(int cx, int cy, int cz)
+{
+    return (uint32_t)(cz & 3) << (kBrickX + kBrickY) | (uint32_t)(cy & 3) << kBrickX | (uint32_t)(cx & 7);
+}
+static_assert(kBrickY == 2 && kBrickZ == 2 && kBrickX == 3, "masks of brick_local");
+
+// The points [first, end) of the cells x0..x1 of row (cy, cz) that lie in the brick of x0 (part 0) or in the brick of x1
+// where that is another one (part 1; x1 - x0 < 8 cells, so there is no third).
+__device__ __forceinline__ void brick_range(const KnnView& k, uint32_t slot, int xa, int xb, int cy, int cz,
+                                            uint32_t* first, uint32_t* end)
+{
+    const uint32_t* row = k.cell_start + ((size_t)slot << 7) + brick_local(0, cy, cz);
+    *first              = row[xa & 7];
+    *end                = row[(xb & 7) + 1];
 }
 
-// The search of one point by one thread: the cube of cells around the point's cell grows until the K-th best distance
-// cannot be beaten from outside it; a row of cells along x is one contiguous run of the cell-ordered array, so a cube
-// of (2r+1)^3 cells is (2r+1)^2 runs.  A larger cube is searched from scratch (the first cube, r = 1, settles nearly
-// every point).  Gives up after rmax shells: false, and the caller hands the point to the next, coarser stage.
-template <int K>  // K = n + 1 best squared distances are kept (the point itself is one of them)
-__device__ __forceinline__ bool knn_cubes(const float4 p, const KnnGrid& g, const float4* __restrict__ sorted,
-                                          const uint32_t* __restrict__ offset, int rmax, float* kth)
+// ---- binning ----------------------------------------------------------------------------------------------------
+// Points per bin (BRICKS: bricks of the search grid, else cells of the coarse grid) and the rank of every point in its
+// bin.  Neighbouring lanes mostly hold points of one bin where the cloud is stored in spatial order: every run of equal
+// bins takes its ranks with one returning atomic.  `stride` > 1: every stride-th point only (n of them).
+constexpr int kBinPer = 4;
+
+template <bool BRICKS>
+__global__ __launch_bounds__(kBlock) void knn_count_kernel(const float4* __restrict__ position, int n, int stride,
+                                                           const KnnGrid* __restrict__ gp, uint32_t* __restrict__ count,
+                                                           uint32_t* __restrict__ rank, const uint32_t* __restrict__ gate)
 {
-    const int3 c = grid_cell(g, p.x, p.y, p.z);
-    float best[K];
-    for (int r = 1; r <= rmax; ++r)
+    if (gate && *gate == 0) return;  // (kernel-uniform)
+    const KnnGrid g    = *gp;
+    const int lane     = threadIdx.x & 63;
+    const size_t base  = (size_t)blockIdx.x * (kBlock * kBinPer) + threadIdx.x;
+    float4 p[kBinPer];
+#pragma unroll
+    for (int k = 0; k < kBinPer; ++k)
     {
+        const size_t i = base + k * kBlock;
+        p[k]           = i < (size_t)n ? position[i * (size_t)stride] : make_float4(0, 0, 0, 0);
+    }
+    uint32_t first[kBinPer];
+    int head[kBinPer];
 #pragma unroll
-        for (int k = 0; k < K; ++k) best[k] = 3.0e38f;
-        const int z0 = max(c.z - r, 0), z1 = min(c.z + r, g.dim[2] - 1);
-        const int y0 = max(c.y - r, 0), y1 = min(c.y + r, g.dim[1] - 1);
-        const int x0 = max(c.x - r, 0), x1 = min(c.x + r, g.dim[0] - 1);
-        for (int cz = z0; cz <= z1; ++cz)
-            for (int cy = y0; cy <= y1; ++cy)
-            {
-                const uint32_t row = grid_index(g, 0, cy, cz);
-                const uint32_t e   = offset[row + x1 + 1];
-                for (uint32_t q = offset[row + x0]; q < e; ++q)
-                {
-                    const float4 o = sorted[q];
-                    const float dx = p.x - o.x, dy = p.y - o.y, dz = p.z - o.z;
-                    float d2 = (dx * dx + dy * dy) + dz * dz;
-                    if (d2 < best[K - 1])
-                    {
-#pragma unroll
-                        for (int k = 0; k < K; ++k)  // insertion into the ascending list
-                        {
-                            const float b = best[k];
-                            const bool lt = d2 < b;
-                            best[k]       = lt ? d2 : b;
-                            d2            = lt ? b : d2;
-                        }
-                    }
-                }
-            }
-        // Nothing outside the cube is closer than the nearest face of the cube that has cells behind it (slightly
-        // shrunk: the cell of a point and the faces are computed in fp32).  No such face: the cube is the whole grid.
-        float bound = 3.0e38f;
-        if (c.x - r > 0) bound = fminf(bound, p.x - (g.min[0] + (float)(c.x - r) * g.cell));
-        if (c.y - r > 0) bound = fminf(bound, p.y - (g.min[1] + (float)(c.y - r) * g.cell));
-        if (c.z - r > 0) bound = fminf(bound, p.z - (g.min[2] + (float)(c.z - r) * g.cell));
-        if (c.x + r < g.dim[0] - 1) bound = fminf(bound, (g.min[0] + (float)(c.x + r + 1) * g.cell) - p.x);
-        if (c.y + r < g.dim[1] - 1) bound = fminf(bound, (g.min[1] + (float)(c.y + r + 1) * g.cell) - p.y);
-        if (c.z + r < g.dim[2] - 1) bound = fminf(bound, (g.min[2] + (float)(c.z + r + 1) * g.cell) - p.z);
-        bound = fmaxf(bound, 0.f) * 0.999f;
-        if (bound >= 1.0e38f || best[K - 1] <= bound * bound)
+    for (int k = 0; k < kBinPer; ++k)
+    {
+        const bool valid = base + k * kBlock < (size_t)n;
+        const int3 c     = grid_cell(g, p[k].x, p[k].y, p[k].z);
+        const uint32_t b = !valid ? kNoBrick : (BRICKS ? brick_row(g, c.y, c.z) + (uint32_t)(c.x >> kBrickX) : grid_index(g, c.x, c.y, c.z));
+        const uint32_t prev = (uint32_t)__shfl_up((int)b, 1, 64);
+        const bool starts   = lane == 0 || prev != b;
+        const unsigned long long heads = __ballot(starts);
+        const unsigned long long upto  = (2ull << lane) - 1ull;  // lanes 0..lane (lane 63: all)
+        head[k]  = 63 - __clzll((long long)(heads & upto));
+        first[k] = 0;
+        if (starts && valid)
         {
-            *kth = best[K - 1];
-            return true;
+            const unsigned long long above = heads & ~upto;
+            const int next                 = above ? __ffsll((long long)above) - 1 : 64;
+            first[k]                       = atomicAdd(&count[b], (uint32_t)(next - lane));
         }
     }
-    return false;
+#pragma unroll
+    for (int k = 0; k < kBinPer; ++k)
+    {
+        const uint32_t f = (uint32_t)__shfl((int)first[k], head[k], 64);
+        const size_t i   = base + k * kBlock;
+        if (i < (size_t)n) __builtin_nontemporal_store(f + (uint32_t)(lane - head[k]), rank + i);
+    }
+}
+
+// The points bin after bin, (x, y, z, bits of the point id): no atomics, the rank comes from the counting pass.
+template <bool BRICKS>
+__global__ __launch_bounds__(kBlock) void knn_scatter_kernel(const float4* __restrict__ position, int n, int stride,
+                                                             const KnnGrid* __restrict__ gp,
+                                                             const uint32_t* __restrict__ start,
+                                                             const uint32_t* __restrict__ rank, float4* __restrict__ out,
+                                                             const uint32_t* __restrict__ gate)
+{
+    if (gate && *gate == 0) return;
+    const KnnGrid g   = *gp;
+    const size_t base = (size_t)blockIdx.x * (kBlock * kBinPer) + threadIdx.x;
+    float4 p[kBinPer];
+    uint32_t r[kBinPer];
+#pragma unroll
+    for (int k = 0; k < kBinPer; ++k)
+    {
+        const size_t i = base + k * kBlock;
+        p[k]           = i < (size_t)n ? position[i * (size_t)stride] : make_float4(0, 0, 0, 0);
+        r[k]           = i < (size_t)n ? __builtin_nontemporal_load(rank + i) : 0u;
+    }
+#pragma unroll
+    for (int k = 0; k < kBinPer; ++k)
+    {
+        const size_t i = base + k * kBlock;
+        if (i >= (size_t)n) continue;
+        const int3 c     = grid_cell(g, p[k].x, p[k].y, p[k].z);
+        const uint32_t b = BRICKS ? brick_row(g, c.y, c.z) + (uint32_t)(c.x >> kBrickX) : grid_index(g, c.x, c.y, c.z);
+        out[start[b] + r[k]] = make_float4(p[k].x, p[k].y, p[k].z, __uint_as_float((uint32_t)(i * (size_t)stride)));
+    }
+}
+
+// Zeroes the counters of the grid's bins.
+template <bool BRICKS>
+__global__ __launch_bounds__(kBlock) void knn_clear_kernel(uint32_t* __restrict__ count, const KnnGrid* __restrict__ gp,
+                                                           const uint32_t* __restrict__ gate)
+{
+    if (gate && *gate == 0) return;
+    const uint32_t bins = BRICKS ? gp->bricks : gp->cells;
+    for (size_t i = (size_t)blockIdx.x * kBlock + threadIdx.x; i < bins; i += (size_t)gridDim.x * kBlock)
+        __builtin_nontemporal_store(0u, count + i);
+}
+
+// Exclusive prefix sums over the bins in two launches: sums of chunks of 8192 bins, then the sums inside every chunk on top of
+// those of the chunks before it (at most 1024 chunks, which every workgroup sums up for itself).  BRICKS: the bins that
+// hold points are numbered in the same pass (slots), in the high half of a 64-bit sum.
+constexpr int kScanChunk  = 8192;
+constexpr int kScanChunks = 1024;
+
+__device__ __forceinline__ unsigned long long block_exclusive_scan_1024(unsigned long long sum, unsigned long long* s_wave,
+                                                                        unsigned long long* total)
+{
+    const int tid          = threadIdx.x;
+    unsigned long long inc = sum;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1)
+    {
+        const unsigned long long u = __shfl_up(inc, off, 64);
+        if ((tid & 63) >= off) inc += u;
+    }
+    __syncthreads();  // s_wave of the last call has been read
+    if ((tid & 63) == 63) s_wave[tid >> 6] = inc;
+    __syncthreads();
+    unsigned long long run = inc - sum, all = 0;
+    for (int w = 0; w < 16; ++w)
+    {
+        if (w < (tid >> 6)) run += s_wave[w];
+        all += s_wave[w];
+    }
+    *total = all;
+    return run;
+}
+
+__device__ __forceinline__ void scan_load(const uint32_t* __restrict__ count, size_t t0, uint32_t bins, uint32_t v[8])
+{
+    if (t0 + 8 <= bins)
+    {
+        const uint4 a = ((const uint4*)(count + t0))[0], c = ((const uint4*)(count + t0))[1];
+        v[0] = a.x, v[1] = a.y, v[2] = a.z, v[3] = a.w, v[4] = c.x, v[5] = c.y, v[6] = c.z, v[7] = c.w;
+    }
+    else
+#pragma unroll
+        for (int k = 0; k < 8; ++k) v[k] = t0 + k < bins ? count[t0 + k] : 0u;
+}
+
+template <bool BRICKS>
+__global__ __launch_bounds__(1024) void knn_scan_reduce_kernel(const uint32_t* __restrict__ count,
+                                                               const KnnGrid* __restrict__ gp,
+                                                               unsigned long long* __restrict__ chunk_sum,
+                                                               const uint32_t* __restrict__ gate)
+{
+    __shared__ unsigned long long s_wave[16];
+    if (gate && *gate == 0) return;
+    const uint32_t bins = BRICKS ? gp->bricks : gp->cells;
+    const uint32_t nb   = (bins + kScanChunk - 1) / kScanChunk;
+    for (uint32_t b = blockIdx.x; b < nb; b += gridDim.x)
+    {
+        uint32_t v[8];
+        scan_load(count, (size_t)b * kScanChunk + (size_t)threadIdx.x * 8, bins, v);
+        unsigned long long sum = 0, total;
+#pragma unroll
+        for (int k = 0; k < 8; ++k) sum += (unsigned long long)v[k] | (BRICKS && v[k] ? 1ull << 32 : 0ull);
+        block_exclusive_scan_1024(sum, s_wave, &total);
+        if (threadIdx.x == 0) chunk_sum[b] = total;
+    }
+}
+
+// start[b]: first point of bin b.  BRICKS also: slot[b] (kNoBrick: the brick is empty), slot_brick[slot], the number of
+// slots, and the end of the last cell (cell_start holds one word more than the cells of the bricks).
+// not BRICKS also: start[bins] = number of points.
+template <bool BRICKS>
+__global__ __launch_bounds__(1024) void knn_scan_apply_kernel(const uint32_t* __restrict__ count,
+                                                              const KnnGrid* __restrict__ gp,
+                                                              const unsigned long long* __restrict__ chunk_sum,
+                                                              uint32_t* __restrict__ start, uint32_t* __restrict__ slot,
+                                                              uint32_t* __restrict__ slot_brick,
+                                                              uint32_t* __restrict__ num_slots,
+                                                              uint32_t* __restrict__ cell_start,
+                                                              const uint32_t* __restrict__ gate)
+{
+    __shared__ unsigned long long s_wave[16];
+    if (gate && *gate == 0) return;
+    const uint32_t bins = BRICKS ? gp->bricks : gp->cells;
+    const uint32_t nb   = (bins + kScanChunk - 1) / kScanChunk;
+    const unsigned long long mine = threadIdx.x < nb ? chunk_sum[threadIdx.x] : 0ull;  // nb <= kScanChunks
+    for (uint32_t b = blockIdx.x; b < nb; b += gridDim.x)
+    {
+        const size_t t0 = (size_t)b * kScanChunk + (size_t)threadIdx.x * 8;
+        uint32_t v[8];
+        scan_load(count, t0, bins, v);
+        unsigned long long before, sum = 0, total;
+        block_exclusive_scan_1024(threadIdx.x < b ? mine : 0ull, s_wave, &before);
+#pragma unroll
+        for (int k = 0; k < 8; ++k) sum += (unsigned long long)v[k] | (BRICKS && v[k] ? 1ull << 32 : 0ull);
+        const unsigned long long run = before + block_exclusive_scan_1024(sum, s_wave, &total);
+        uint32_t point = (uint32_t)run, s = (uint32_t)(run >> 32);
+        uint32_t o[8], q[8];
+#pragma unroll
+        for (int k = 0; k < 8; ++k)
+        {
+            o[k] = point;
+            q[k] = v[k] ? s : kNoBrick;
+            if (BRICKS && v[k]) slot_brick[s++] = (uint32_t)(t0 + k);
+            point += v[k];
+        }
+        if (t0 + 8 <= bins)
+        {
+            ((uint4*)(start + t0))[0] = make_uint4(o[0], o[1], o[2], o[3]);
+            ((uint4*)(start + t0))[1] = make_uint4(o[4], o[5], o[6], o[7]);
+            if (BRICKS)
+            {
+                ((uint4*)(slot + t0))[0] = make_uint4(q[0], q[1], q[2], q[3]);
+                ((uint4*)(slot + t0))[1] = make_uint4(q[4], q[5], q[6], q[7]);
+            }
+        }
+        else
+#pragma unroll
+            for (int k = 0; k < 8; ++k)
+                if (t0 + k < bins)
+                {
+                    start[t0 + k] = o[k];
+                    if (BRICKS) slot[t0 + k] = q[k];
+                }
+        if (b == nb - 1 && threadIdx.x == 0)
+        {
+            const unsigned long long all = before + total;
+            if (BRICKS)
+            {
+                *num_slots                                = (uint32_t)(all >> 32);
+                cell_start[(size_t)(all >> 32) << 7] = (uint32_t)all;
+            }
+            else
+                start[bins] = (uint32_t)all;
+        }
+    }
+}
+
+// The points of every brick in the order of its cells, and the first point of every cell: one wavefront per brick that
+// holds points, the 128 counters in LDS.  A brick of a surface holds ~160 points: up to 256 stay in registers between
+// the count and the scatter, a fuller brick is read twice.
+constexpr int kBrickPer = 4;
+
+__global__ __launch_bounds__(kBlock) void knn_brick_sort_kernel(const float4* __restrict__ in,
+                                                                const KnnGrid* __restrict__ gp,
+                                                                const uint32_t* __restrict__ num_slots,
+                                                                const uint32_t* __restrict__ slot_brick,
+                                                                const uint32_t* __restrict__ start,
+                                                                const uint32_t* __restrict__ count,
+                                                                uint32_t* __restrict__ cell_start,
+                                                                float4* __restrict__ out)
+{
+    __shared__ uint32_t s_count[kBlock / 64][kBrickCells];
+    uint32_t* cnt       = s_count[threadIdx.x >> 6];
+    const int lane      = threadIdx.x & 63;
+    const KnnGrid g     = *gp;
+    const uint32_t all  = *num_slots;
+    for (uint32_t s = blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6); s < all; s += gridDim.x * (kBlock / 64))  // wavefront-uniform
+    {
+        const uint32_t b = slot_brick[s], first = start[b], num = count[b];
+        wave_lds_sync();
+        cnt[lane]      = 0;
+        cnt[lane + 64] = 0;
+        wave_lds_sync();
+        float4 p[kBrickPer];
+        uint32_t cell[kBrickPer], rank[kBrickPer];
+        for (uint32_t q0 = 0; q0 < num; q0 += 64 * kBrickPer)
+        {
+#pragma unroll
+            for (int k = 0; k < kBrickPer; ++k)
+            {
+                const uint32_t q = q0 + k * 64 + lane;
+                p[k]             = q < num ? in[first + q] : make_float4(0, 0, 0, 0);
+            }
+#pragma unroll
+            for (int k = 0; k < kBrickPer; ++k)
+            {
+                const int3 c = grid_cell(g, p[k].x, p[k].y, p[k].z);
+                cell[k]      = brick_local(c.x, c.y, c.z);
+                rank[k]      = q0 + k * 64 + lane < num ? atomicAdd(&cnt[cell[k]], 1u) : 0u;
+            }
+        }
+        wave_lds_sync();
+        const uint32_t c0 = cnt[2 * lane], c1 = cnt[2 * lane + 1];
+        uint32_t inc = c0 + c1;
+#pragma unroll
+        for (int off = 1; off < 64; off <<= 1)
+        {
+            const uint32_t u = (uint32_t)__shfl_up((int)inc, off, 64);
+            if (lane >= off) inc += u;
+        }
+        const uint32_t at = first + inc - c0 - c1;
+        ((uint2*)(cell_start + ((size_t)s << 7)))[lane] = make_uint2(at, at + c0);
+        wave_lds_sync();
+        cnt[2 * lane]     = at;
+        cnt[2 * lane + 1] = at + c0;
+        wave_lds_sync();
+        if (num <= 64 * kBrickPer)
+        {
+#pragma unroll
+            for (int k = 0; k < kBrickPer; ++k)
+                if (k * 64 + (uint32_t)lane < num) out[cnt[cell[k]] + rank[k]] = p[k];
+        }
+        else
+            for (uint32_t q = lane; q < num; q += 64)
+            {
+                const float4 o = in[first + q];
+                const int3 c   = grid_cell(g, o.x, o.y, o.z);
+                out[atomicAdd(&cnt[brick_local(c.x, c.y, c.z)], 1u)] = o;
+            }
+    }
+}
+
+// ---- search -----------------------------------------------------------------------------------------------------
+// A candidate into the ascending list of the K smallest: every place takes the middle one of its left neighbour, the
+// candidate and itself.
+template <int K>
+__device__ __forceinline__ void keep_smallest(float* best, float d2)
+{
+#pragma unroll
+    for (int k = K - 1; k > 0; --k) best[k] = __builtin_amdgcn_fmed3f(best[k - 1], d2, best[k]);
+    best[0] = fminf(best[0], d2);
+}
+
+__device__ __forceinline__ float distance2(const float4 p, const float4 o)
+{
+    const float dx = p.x - o.x, dy = p.y - o.y, dz = p.z - o.z;
+    return (dx * dx + dy * dy) + dz * dz;
+}
+
+// Nothing outside the cube of r shells around cell c is closer than the nearest face of the cube that has cells behind
+// it (slightly shrunk: the cell of a point and the faces are computed in fp32).  3e38: the cube is the whole grid.
+__device__ __forceinline__ float cube_bound(const KnnGrid& g, const float4 p, int3 c, int r)
+{
+    float bound = 3.0e38f;
+    if (c.x - r > 0) bound = fminf(bound, p.x - (g.min[0] + (float)(c.x - r) * g.cell));
+    if (c.y - r > 0) bound = fminf(bound, p.y - (g.min[1] + (float)(c.y - r) * g.cell));
+    if (c.z - r > 0) bound = fminf(bound, p.z - (g.min[2] + (float)(c.z - r) * g.cell));
+    if (c.x + r < g.dim[0] - 1) bound = fminf(bound, (g.min[0] + (float)(c.x + r + 1) * g.cell) - p.x);
+    if (c.y + r < g.dim[1] - 1) bound = fminf(bound, (g.min[1] + (float)(c.y + r + 1) * g.cell) - p.y);
+    if (c.z + r < g.dim[2] - 1) bound = fminf(bound, (g.min[2] + (float)(c.z + r + 1) * g.cell) - p.z);
+    return fmaxf(bound, 0.f) * 0.999f;
+}
+__device__ __forceinline__ bool cube_settles(float kth, float bound)
+{
+    return bound >= 1.0e38f || kth <= bound * bound;
 }
 
 // Appends `value` of the lanes with `push` to a list (one atomic per wavefront).  Called by all lanes of a wavefront.
@@ -125,38 +417,132 @@ __device__ __forceinline__ void wave_push(bool push, uint32_t value, uint32_t* _
     if (push) list[base + (uint32_t)__popcll(m & ((1ull << lane) - 1ull))] = value;
 }
 
-// Stage 1: every point, one thread each in cell order of the second grid (the lanes of a wavefront search nearly the
-// same cells), at most 2 shells; what is left (points in sparse parts of the cloud) goes to list.
-template <int K>
-__global__ __launch_bounds__(kBlock) void knn_search_kernel(const float4* __restrict__ sorted, int n,
-                                                            const KnnGrid* __restrict__ gp,
-                                                            const uint32_t* __restrict__ offset, float* __restrict__ out,
+// Stage 1: every point, one thread each in the order of the search grid, the cube of 3 x 3 x 3 cells around its own: 9
+// rows of cells, each one run of consecutive points, or two where the row crosses into the next brick.  The runs are
+// looked up first, all of them at once (two dependent round trips), and kept in LDS; the candidates then come in ONE
+// loop over all runs, so that a wavefront takes as many rounds as its fullest cube has candidates and not, row after
+// row, as the fullest row.  Points whose n-th neighbour may lie outside the cube go to list.
+constexpr int kMaxRuns = 18;
+
+template <int K>  // K = n + 1 best squared distances are kept (the point itself is one of them)
+__global__ __launch_bounds__(kBlock) void knn_search_kernel(KnnView kv, int n, float* __restrict__ out,
                                                             uint32_t* __restrict__ list, uint32_t* list_count)
 {
-    const int t = blockIdx.x * kBlock + threadIdx.x;
-    bool left   = false;
-    if (t < n)
+    __shared__ uint2 s_run[kMaxRuns][kBlock];
+    const int t     = blockIdx.x * kBlock + threadIdx.x;
+    const KnnGrid g = *kv.grid;
+    const float4 p  = kv.sorted[t < n ? t : n - 1];
+    const int3 c    = grid_cell(g, p.x, p.y, p.z);
+    const int x0 = max(c.x - 1, 0), x1 = min(c.x + 1, g.dim[0] - 1);
+    const bool two = (x0 >> kBrickX) != (x1 >> kBrickX);
+    int runs       = 0;
+    for (int part = 0; part < 2; ++part)
     {
-        const KnnGrid g = *gp;
-        const float4 p  = sorted[t];
-        float kth;
-        if (knn_cubes<K>(p, g, sorted, offset, 2, &kth))
-            out[__float_as_uint(p.w)] = sqrtf(kth);
-        else
-            left = true;
+        if (part == 1 && !__ballot(two)) break;
+        const int xa = part == 0 ? x0 : (x1 >> kBrickX) << kBrickX;
+        const int xb = part == 0 && two ? (x0 | 7) : x1;
+        uint32_t slot[9], first[9], end[9];
+#pragma unroll
+        for (int q = 0; q < 9; ++q)
+        {
+            const int cy = c.y + q % 3 - 1, cz = c.z + q / 3 - 1;
+            const bool ok = (unsigned)cy < (unsigned)g.dim[1] && (unsigned)cz < (unsigned)g.dim[2] && (part == 0 || two);
+            slot[q]       = ok ? kv.slot[brick_row(g, cy, cz) + (uint32_t)(xa >> kBrickX)] : kNoBrick;
+        }
+#pragma unroll
+        for (int q = 0; q < 9; ++q)
+        {
+            first[q] = end[q] = 0;
+            if (slot[q] != kNoBrick) brick_range(kv, slot[q], xa, xb, c.y + q % 3 - 1, c.z + q / 3 - 1, &first[q], &end[q]);
+        }
+#pragma unroll
+        for (int q = 0; q < 9; ++q)
+            if (end[q] > first[q]) s_run[runs++][threadIdx.x] = make_uint2(first[q], end[q]);
     }
-    wave_push(left, (uint32_t)t, list, list_count);
+    float best[K];
+#pragma unroll
+    for (int k = 0; k < K; ++k) best[k] = 3.0e38f;
+    uint32_t q = 0, e = 0;
+    int next = 0;
+    for (;;)
+    {
+        if (q >= e)
+        {
+            if (next == runs) break;
+            const uint2 r = s_run[next++][threadIdx.x];
+            q             = r.x;
+            e             = r.y;
+        }
+        const float4 o0 = kv.sorted[q], o1 = kv.sorted[min(q + 1, e - 1)];
+        const float d0 = distance2(p, o0), d1 = distance2(p, o1);
+        keep_smallest<K>(best, d0);
+        keep_smallest<K>(best, q + 1 < e ? d1 : 3.0e38f);
+        q += 2;
+    }
+    const bool settled = cube_settles(best[K - 1], cube_bound(g, p, c, 1));
+    if (t < n && settled) out[__float_as_uint(p.w)] = sqrtf(best[K - 1]);
+    wave_push(t < n && !settled, (uint32_t)t, list, list_count);
 }
 
-// Stage 2: the points stage 1 left, on the first (coarser) grid, at most 4 shells; the rest goes to list2.
+// Stage 2: the points stage 1 left, cubes of 2 and 3 shells of the same grid; the rest goes to list2.  A larger cube is
+// searched from scratch.
 template <int K>
-__global__ __launch_bounds__(kBlock) void knn_list_kernel(const float4* __restrict__ points,
-                                                          const uint32_t* __restrict__ list,
-                                                          const uint32_t* __restrict__ list_count,
-                                                          const float4* __restrict__ sorted0,
-                                                          const KnnGrid* __restrict__ gp0,
-                                                          const uint32_t* __restrict__ offset0, float* __restrict__ out,
-                                                          uint32_t* __restrict__ list2, uint32_t* list2_count)
+__global__ __launch_bounds__(kBlock) void knn_shells_kernel(KnnView kv, const uint32_t* __restrict__ list,
+                                                            const uint32_t* __restrict__ list_count,
+                                                            float* __restrict__ out, uint32_t* __restrict__ list2,
+                                                            uint32_t* list2_count)
+{
+    const uint32_t count = *list_count;
+    const KnnGrid g      = *kv.grid;
+    const uint32_t lane  = threadIdx.x & 63;
+    for (uint32_t e0 = blockIdx.x * kBlock + (threadIdx.x & ~63u); e0 < count; e0 += gridDim.x * kBlock)  // wavefront-uniform
+    {
+        const uint32_t e = e0 + lane;
+        bool left        = false;
+        uint32_t t       = 0;
+        if (e < count)
+        {
+            t              = list[e];
+            const float4 p = kv.sorted[t];
+            const int3 c   = grid_cell(g, p.x, p.y, p.z);
+            left           = true;
+            for (int r = 2; r <= 3 && left; ++r)
+            {
+                float best[K];
+#pragma unroll
+                for (int k = 0; k < K; ++k) best[k] = 3.0e38f;
+                const int x0 = max(c.x - r, 0), x1 = min(c.x + r, g.dim[0] - 1);
+                for (int cz = max(c.z - r, 0); cz <= min(c.z + r, g.dim[2] - 1); ++cz)
+                    for (int cy = max(c.y - r, 0); cy <= min(c.y + r, g.dim[1] - 1); ++cy)
+                        for (int part = x0 >> kBrickX; part <= x1 >> kBrickX; ++part)
+                        {
+                            const uint32_t slot = kv.slot[brick_row(g, cy, cz) + (uint32_t)part];
+                            if (slot == kNoBrick) continue;
+                            uint32_t q, end;
+                            brick_range(kv, slot, max(x0, part << kBrickX), min(x1, part << kBrickX | 7), cy, cz, &q, &end);
+                            for (; q < end; ++q) keep_smallest<K>(best, distance2(p, kv.sorted[q]));
+                        }
+                if (cube_settles(best[K - 1], cube_bound(g, p, c, r)))
+                {
+                    out[__float_as_uint(p.w)] = sqrtf(best[K - 1]);
+                    left                      = false;
+                }
+            }
+        }
+        wave_push(left, t, list2, list2_count);
+    }
+}
+
+// Stage 3: what is left (points in sparse parts of the cloud), on the coarse grid over all points, at most 4 shells; the
+// rest goes to list3.
+template <int K>
+__global__ __launch_bounds__(kBlock) void knn_coarse_kernel(const float4* __restrict__ points,
+                                                            const uint32_t* __restrict__ list,
+                                                            const uint32_t* __restrict__ list_count,
+                                                            const float4* __restrict__ sorted0,
+                                                            const KnnGrid* __restrict__ gp0,
+                                                            const uint32_t* __restrict__ start0, float* __restrict__ out,
+                                                            uint32_t* __restrict__ list3, uint32_t* list3_count)
 {
     const uint32_t count = *list_count;
     const KnnGrid g      = *gp0;
@@ -170,13 +556,28 @@ __global__ __launch_bounds__(kBlock) void knn_list_kernel(const float4* __restri
         {
             t              = list[e];
             const float4 p = points[t];
-            float kth;
-            if (knn_cubes<K>(p, g, sorted0, offset0, 4, &kth))
-                out[__float_as_uint(p.w)] = sqrtf(kth);
-            else
-                left = true;
+            const int3 c   = grid_cell(g, p.x, p.y, p.z);
+            left           = true;
+            for (int r = 1; r <= 4 && left; ++r)
+            {
+                float best[K];
+#pragma unroll
+                for (int k = 0; k < K; ++k) best[k] = 3.0e38f;
+                const int x0 = max(c.x - r, 0), x1 = min(c.x + r, g.dim[0] - 1);
+                for (int cz = max(c.z - r, 0); cz <= min(c.z + r, g.dim[2] - 1); ++cz)
+                    for (int cy = max(c.y - r, 0); cy <= min(c.y + r, g.dim[1] - 1); ++cy)
+                    {
+                        const uint32_t row = grid_index(g, 0, cy, cz), end = start0[row + x1 + 1];
+                        for (uint32_t q = start0[row + x0]; q < end; ++q) keep_smallest<K>(best, distance2(p, sorted0[q]));
+                    }
+                if (cube_settles(best[K - 1], cube_bound(g, p, c, r)))
+                {
+                    out[__float_as_uint(p.w)] = sqrtf(best[K - 1]);
+                    left                      = false;
+                }
+            }
         }
-        wave_push(left, t, list2, list2_count);
+        wave_push(left, t, list3, list3_count);
     }
 }
 
@@ -204,7 +605,7 @@ __device__ __forceinline__ float wave_kth(float* best)
     return kth;
 }
 
-// Stage 3: stray points far from everything (no cube of a few shells of either grid settles them): one wavefront
+// Stage 4: stray points far from everything (no cube of a few shells of either grid settles them): one wavefront
 // per point goes through all points.
 template <int K>
 __global__ __launch_bounds__(kBlock) void knn_brute_kernel(const float4* __restrict__ points, int n,
@@ -220,32 +621,17 @@ __global__ __launch_bounds__(kBlock) void knn_brute_kernel(const float4* __restr
         float best[K];
 #pragma unroll
         for (int k = 0; k < K; ++k) best[k] = 3.0e38f;
-        for (int q = lane; q < n; q += 64)
-        {
-            const float4 o = points[q];
-            const float dx = p.x - o.x, dy = p.y - o.y, dz = p.z - o.z;
-            float d2 = (dx * dx + dy * dy) + dz * dz;
-            if (d2 < best[K - 1])
-            {
-#pragma unroll
-                for (int k = 0; k < K; ++k)
-                {
-                    const float b = best[k];
-                    const bool lt = d2 < b;
-                    best[k]       = lt ? d2 : b;
-                    d2            = lt ? b : d2;
-                }
-            }
-        }
+#pragma unroll 4
+        for (int q = lane; q < n; q += 64) keep_smallest<K>(best, distance2(p, points[q]));
         const float kth = wave_kth<K>(best);
         if (lane == 0) out[__float_as_uint(p.w)] = sqrtf(kth);
     }
 }
 
-// The search of stage 1 for `samples` points evenly spaced in cell order, one wavefront per point (on the first grid a
-// point has thousands of candidates: the lanes share them, every lane keeps the K best of its share).  out[s] =
-// distance of sample s, 3e38 for a sample that 4 shells do not settle (a stray point: it shall not size the grid).
-// All branches on r, the bound and the result are uniform over the wavefront.
+// The neighbour distance of `samples` points evenly spaced in the order of the coarse grid, one wavefront per point (the
+// lanes share the candidates, every lane keeps the K best of its share).  out[s] = distance of sample s, 3e38 for a sample
+// that 4 shells do not settle (a stray point: it shall not size the grid).  All branches on r, the bound and the
+// result are uniform over the wavefront.
 template <int K>
 __global__ __launch_bounds__(kBlock) void knn_sample_kernel(const float4* __restrict__ sorted, int n,
                                                             const KnnGrid* __restrict__ gp,
@@ -265,42 +651,15 @@ __global__ __launch_bounds__(kBlock) void knn_sample_kernel(const float4* __rest
         float best[K];
 #pragma unroll
         for (int k = 0; k < K; ++k) best[k] = 3.0e38f;
-        const int z0 = max(c.z - r, 0), z1 = min(c.z + r, g.dim[2] - 1);
-        const int y0 = max(c.y - r, 0), y1 = min(c.y + r, g.dim[1] - 1);
         const int x0 = max(c.x - r, 0), x1 = min(c.x + r, g.dim[0] - 1);
-        for (int cz = z0; cz <= z1; ++cz)
-            for (int cy = y0; cy <= y1; ++cy)
+        for (int cz = max(c.z - r, 0); cz <= min(c.z + r, g.dim[2] - 1); ++cz)
+            for (int cy = max(c.y - r, 0); cy <= min(c.y + r, g.dim[1] - 1); ++cy)
             {
-                const uint32_t row = grid_index(g, 0, cy, cz);
-                const uint32_t e   = offset[row + x1 + 1];
-                for (uint32_t q = offset[row + x0] + lane; q < e; q += 64)
-                {
-                    const float4 o = sorted[q];
-                    const float dx = p.x - o.x, dy = p.y - o.y, dz = p.z - o.z;
-                    float d2 = (dx * dx + dy * dy) + dz * dz;
-                    if (d2 < best[K - 1])
-                    {
-#pragma unroll
-                        for (int k = 0; k < K; ++k)
-                        {
-                            const float b = best[k];
-                            const bool lt = d2 < b;
-                            best[k]       = lt ? d2 : b;
-                            d2            = lt ? b : d2;
-                        }
-                    }
-                }
+                const uint32_t row = grid_index(g, 0, cy, cz), e = offset[row + x1 + 1];
+                for (uint32_t q = offset[row + x0] + lane; q < e; q += 64) keep_smallest<K>(best, distance2(p, sorted[q]));
             }
         const float kth = wave_kth<K>(best);
-        float bound = 3.0e38f;
-        if (c.x - r > 0) bound = fminf(bound, p.x - (g.min[0] + (float)(c.x - r) * g.cell));
-        if (c.y - r > 0) bound = fminf(bound, p.y - (g.min[1] + (float)(c.y - r) * g.cell));
-        if (c.z - r > 0) bound = fminf(bound, p.z - (g.min[2] + (float)(c.z - r) * g.cell));
-        if (c.x + r < g.dim[0] - 1) bound = fminf(bound, (g.min[0] + (float)(c.x + r + 1) * g.cell) - p.x);
-        if (c.y + r < g.dim[1] - 1) bound = fminf(bound, (g.min[1] + (float)(c.y + r + 1) * g.cell) - p.y);
-        if (c.z + r < g.dim[2] - 1) bound = fminf(bound, (g.min[2] + (float)(c.z + r + 1) * g.cell) - p.z);
-        bound = fmaxf(bound, 0.f) * 0.999f;
-        if (bound >= 1.0e38f || kth <= bound * bound)
+        if (cube_settles(kth, cube_bound(g, p, c, r)))
         {
             result = sqrtf(kth);
             break;
@@ -309,77 +668,72 @@ __global__ __launch_bounds__(kBlock) void knn_sample_kernel(const float4* __rest
     if (lane == 0) out[slot] = result;
 }
 
-constexpr int kKnnSamples   = 2048;
+// ---- sizing the grids -------------------------------------------------------------------------------------------
+constexpr int kKnnSamples   = 1024;
 constexpr int kKnnMaxDim    = 2048;
 constexpr int kKnnCoarseDim = 160;
+static_assert(kKnnCoarseDim * kKnnCoarseDim * kKnnCoarseDim <= kScanChunk * kScanChunks, "chunks of the coarse grid");
+static_assert(kKnnMaxBricks <= (size_t)kScanChunk * kScanChunks, "chunks of the search grid");
 
-// ascending bitonic sort of kKnnSamples floats in LDS by a workgroup of 1024 threads
-__device__ __forceinline__ void sort_samples(float* s)
+// A = 1 or 3 arrays of kKnnSamples floats in LDS, each sorted ascending by a workgroup of 1024 threads (bitonic; the
+// arrays share the barriers)
+template <int A>
+__device__ __forceinline__ void sort_samples(float (*s)[kKnnSamples])
 {
     for (int k = 2; k <= kKnnSamples; k <<= 1)
         for (int j = k >> 1; j > 0; j >>= 1)
         {
-            for (int i = threadIdx.x; i < kKnnSamples; i += 1024)
+            for (int w = threadIdx.x; w < A * (kKnnSamples / 2); w += 1024)
             {
-                const int o = i ^ j;
-                if (o > i)
+                float* a    = s[w / (kKnnSamples / 2)];
+                const int h = w & (kKnnSamples / 2 - 1);
+                const int i = ((h & ~(j - 1)) << 1) | (h & (j - 1)), o = i | j;
+                const float u = a[i], v = a[o];
+                if ((u > v) == ((i & k) == 0))
                 {
-                    const float a = s[i], b = s[o];
-                    const bool up = (i & k) == 0;
-                    if ((a > b) == up)
-                    {
-                        s[i] = b;
-                        s[o] = a;
-                    }
+                    a[i] = v;
+                    a[o] = u;
                 }
             }
             __syncthreads();
         }
 }
 
-// First grid.  Its box is not the bounding box of the cloud (one far outlier would stretch that until all other points
-// share a cell) but, per axis, the 1st to 99th percentile of 2048 points taken at equal steps through the array,
+// Coarse grid.  Its box is not the bounding box of the cloud (one far outlier would stretch that until all other points
+// share a cell) but, per axis, the 1st to 99th percentile of 1024 points taken at equal steps through the array,
 // widened by 5 % of that range on either side and cut to the caller's box; the points outside it go to the boundary
 // cells, which keeps the search exact (a cube of cells then stands for a region open to the outside).  Cells for ~8
 // points each if the cloud filled the box, at most kKnnCoarseDim per axis.  One workgroup.
 __global__ __launch_bounds__(1024) void knn_first_grid_kernel(const float4* __restrict__ position, int n, KnnGrid box,
                                                               KnnGrid* __restrict__ dst)
 {
-    __shared__ float s[kKnnSamples];
+    __shared__ float s[3][kKnnSamples];
     const int samples = n < kKnnSamples ? n : kKnnSamples;
-    float lo[3], hi[3];
-#pragma unroll
-    for (int axis = 0; axis < 3; ++axis)
     {
-        for (int i = threadIdx.x; i < kKnnSamples; i += 1024)
-        {
-            float v = 3.0e38f;
-            if (i < samples)
-            {
-                const float4 p = position[(size_t)((long long)i * n / samples)];
-                v              = axis == 0 ? p.x : (axis == 1 ? p.y : p.z);
-            }
-            s[i] = v;
-        }
-        __syncthreads();
-        sort_samples(s);
-        const float a = s[samples / 100], b = s[samples - 1 - samples / 100];
-        const float box_hi = box.min[axis] + box.ext[axis];
-        lo[axis] = fmaxf(a - 0.05f * (b - a), box.min[axis]);
-        hi[axis] = fminf(b + 0.05f * (b - a), box_hi);
-        if (!(hi[axis] >= lo[axis]))  // not a number among the samples
-        {
-            lo[axis] = box.min[axis];
-            hi[axis] = box_hi;
-        }
-        __syncthreads();
+        static_assert(kKnnSamples == 1024, "one sample per thread");
+        const int i = threadIdx.x;
+        float4 p    = make_float4(3.0e38f, 3.0e38f, 3.0e38f, 0.f);
+        if (i < samples) p = position[(size_t)((long long)i * n / samples)];
+        s[0][i] = p.x;
+        s[1][i] = p.y;
+        s[2][i] = p.z;
     }
+    __syncthreads();
+    sort_samples<3>(s);
     if (threadIdx.x != 0) return;
     KnnGrid g;
     for (int k = 0; k < 3; ++k)
     {
-        g.min[k] = lo[k];
-        g.ext[k] = hi[k] - lo[k];
+        const float a = s[k][samples / 100], b = s[k][samples - 1 - samples / 100];
+        const float box_hi = box.min[k] + box.ext[k];
+        float lo = fmaxf(a - 0.05f * (b - a), box.min[k]), hi = fminf(b + 0.05f * (b - a), box_hi);
+        if (!(hi >= lo))  // not a number among the samples
+        {
+            lo = box.min[k];
+            hi = box_hi;
+        }
+        g.min[k] = lo;
+        g.ext[k] = hi - lo;
     }
     const float longest = fmaxf(g.ext[0], fmaxf(g.ext[1], g.ext[2]));
     float volume        = 1.f;  // thin axes count as a millionth of the longest one
@@ -396,155 +750,54 @@ __global__ __launch_bounds__(1024) void knn_first_grid_kernel(const float4* __re
         g.dim[k] = d < 1 ? 1 : (d > kKnnCoarseDim ? kKnnCoarseDim : d);
         g.cells *= (uint32_t)g.dim[k];
     }
-    *dst = g;
+    g.bricks_x = g.bricks_y = 0;
+    g.bricks                = 0;
+    *dst                    = g;
 }
 
-// Second grid: cells of twice the median sampled neighbour distance (a cube of 3 cells then settles every point whose
-// own distance is below twice the median, with ~60 candidates on a surface, ~260 in a volume), never coarser than the
-// first grid, at most kKnnMaxDim cells per axis and `budget` cells in all, over the same box.  One workgroup.
-__global__ __launch_bounds__(1024) void knn_refine_grid_kernel(const float* __restrict__ sample, int samples,
+// Search grid: cells of `factor` times the median sampled neighbour distance, never coarser than the coarse grid, at
+// most kKnnMaxDim cells per axis and `budget` bricks in all, over the same box.  One workgroup.  Also clears the list
+// counters of the search.
+__global__ __launch_bounds__(1024) void knn_refine_grid_kernel(const float* __restrict__ sample, int samples, float factor,
                                                                const KnnGrid* __restrict__ first,
-                                                               KnnGrid* __restrict__ gp, uint32_t budget)
+                                                               KnnGrid* __restrict__ gp, uint32_t budget,
+                                                               uint32_t* __restrict__ list_counts)
 {
-    __shared__ float s[kKnnSamples];
-    for (int i = threadIdx.x; i < kKnnSamples; i += 1024) s[i] = i < samples ? sample[i] : 3.0e38f;
+    __shared__ float s[1][kKnnSamples];
+    s[0][threadIdx.x] = (int)threadIdx.x < samples ? sample[threadIdx.x] : 3.0e38f;
+    if (threadIdx.x < 3) list_counts[threadIdx.x] = 0;
     __syncthreads();
-    sort_samples(s);
+    sort_samples<1>(s);
     if (threadIdx.x != 0) return;
-    KnnGrid g          = *first;
-    const float median = s[samples / 2];
+    KnnGrid g           = *first;
+    const float median  = s[0][samples / 2];
     const float longest = fmaxf(g.ext[0], fmaxf(g.ext[1], g.ext[2]));
-    float cell = 2.0f * median;
+    float cell = factor * median;
     if (!(cell < g.cell)) cell = g.cell;  // also NaN / the 3e38 of a cloud with fewer points than neighbours asked for
     if (!(cell > longest / (float)(kKnnMaxDim - 1))) cell = longest / (float)(kKnnMaxDim - 1);
     if (!(cell > 0.f)) cell = g.cell;
     for (;;)
     {
-        unsigned long long cells = 1;
+        uint32_t b[3];
         for (int k = 0; k < 3; ++k)
         {
             int d    = (int)(g.ext[k] / cell) + 1;
             g.dim[k] = d < 1 ? 1 : (d > kKnnMaxDim ? kKnnMaxDim : d);
-            cells *= (unsigned long long)g.dim[k];
+            b[k]     = k == 0 ? ((uint32_t)g.dim[k] + 7) >> kBrickX : ((uint32_t)g.dim[k] + 3) >> kBrickY;
         }
-        if (cells <= budget)
+        const unsigned long long bricks = (unsigned long long)b[0] * b[1] * b[2];
+        if (bricks <= budget)
         {
-            g.cells = (uint32_t)cells;
+            g.bricks_x = (int)b[0];
+            g.bricks_y = (int)b[1];
+            g.bricks   = (uint32_t)bricks;
             break;
         }
-        cell *= 1.26f;
+        cell *= 1.1f;
     }
     g.cell     = cell;
     g.inv_cell = 1.0f / cell;
     *gp        = g;
-}
-
-// Zeroes the cell counters of the grid.
-__global__ __launch_bounds__(kBlock) void knn_clear_kernel(uint32_t* __restrict__ count, const KnnGrid* __restrict__ gp)
-{
-    const uint32_t cells = gp->cells;
-    for (size_t i = (size_t)blockIdx.x * kBlock + threadIdx.x; i < cells; i += (size_t)gridDim.x * kBlock)
-        __builtin_nontemporal_store(0u, count + i);
-}
-
-// Exclusive prefix sum over the cell counters (offset[0..cells]) in three launches: sums of chunks of 8192 cells,
-// their prefix sum (one workgroup: at most 16384 chunks), the prefix sum inside every chunk.
-constexpr int kScanChunk = 8192;
-
-__device__ __forceinline__ uint32_t block_exclusive_scan_1024(uint32_t sum, uint32_t* s_wave, uint32_t* total)
-{
-    const int tid = threadIdx.x;
-    uint32_t inc  = sum;
-#pragma unroll
-    for (int off = 1; off < 64; off <<= 1)
-    {
-        const uint32_t u = __shfl_up(inc, off, 64);
-        if ((tid & 63) >= off) inc += u;
-    }
-    __syncthreads();  // s_wave of the last call has been read
-    if ((tid & 63) == 63) s_wave[tid >> 6] = inc;
-    __syncthreads();
-    uint32_t run = inc - sum, all = 0;
-    for (int w = 0; w < 16; ++w)
-    {
-        if (w < (tid >> 6)) run += s_wave[w];
-        all += s_wave[w];
-    }
-    *total = all;
-    return run;
-}
-
-__global__ __launch_bounds__(1024) void knn_scan_reduce_kernel(const uint32_t* __restrict__ count,
-                                                               const KnnGrid* __restrict__ gp,
-                                                               uint32_t* __restrict__ chunk_sum)
-{
-    __shared__ uint32_t s_wave[16];
-    const uint32_t cells = gp->cells;
-    const uint32_t nb    = (cells + kScanChunk - 1) / kScanChunk;
-    for (uint32_t b = blockIdx.x; b < nb; b += gridDim.x)
-    {
-        const size_t t0 = (size_t)b * kScanChunk + (size_t)threadIdx.x * 8;
-        uint32_t sum    = 0;
-        if (t0 + 8 <= cells)
-        {
-            const uint4 a = ((const uint4*)(count + t0))[0], c = ((const uint4*)(count + t0))[1];
-            sum = a.x + a.y + a.z + a.w + c.x + c.y + c.z + c.w;
-        }
-        else
-            for (int k = 0; k < 8; ++k) sum += t0 + k < cells ? count[t0 + k] : 0u;
-        uint32_t total;
-        block_exclusive_scan_1024(sum, s_wave, &total);
-        if (threadIdx.x == 0) chunk_sum[b] = total;
-    }
-}
-
-__global__ __launch_bounds__(1024) void knn_scan_chunks_kernel(const uint32_t* __restrict__ chunk_sum,
-                                                               const KnnGrid* __restrict__ gp,
-                                                               uint32_t* __restrict__ chunk_offset)
-{
-    __shared__ uint32_t s_wave[16];
-    const uint32_t nb = (gp->cells + kScanChunk - 1) / kScanChunk;
-    uint32_t carry    = 0;
-    for (uint32_t c0 = 0; c0 < nb; c0 += 1024)
-    {
-        const uint32_t i = c0 + threadIdx.x;
-        const uint32_t v = i < nb ? chunk_sum[i] : 0u;
-        uint32_t total;
-        const uint32_t run = block_exclusive_scan_1024(v, s_wave, &total);
-        if (i < nb) chunk_offset[i] = carry + run;
-        carry += total;
-    }
-    if (threadIdx.x == 0) chunk_offset[nb] = carry;
-}
-
-__global__ __launch_bounds__(1024) void knn_scan_apply_kernel(const uint32_t* __restrict__ count,
-                                                              const KnnGrid* __restrict__ gp,
-                                                              const uint32_t* __restrict__ chunk_offset,
-                                                              uint32_t* __restrict__ offset)
-{
-    __shared__ uint32_t s_wave[16];
-    const uint32_t cells = gp->cells;
-    const uint32_t nb    = (cells + kScanChunk - 1) / kScanChunk;
-    for (uint32_t b = blockIdx.x; b < nb; b += gridDim.x)
-    {
-        const size_t t0 = (size_t)b * kScanChunk + (size_t)threadIdx.x * 8;
-        uint32_t v[8];
-#pragma unroll
-        for (int k = 0; k < 8; ++k) v[k] = t0 + k < cells ? count[t0 + k] : 0u;
-        uint32_t sum = 0;
-#pragma unroll
-        for (int k = 0; k < 8; ++k) sum += v[k];
-        uint32_t total;
-        uint32_t run = chunk_offset[b] + block_exclusive_scan_1024(sum, s_wave, &total);
-#pragma unroll
-        for (int k = 0; k < 8; ++k)
-            if (t0 + k < cells)
-            {
-                offset[t0 + k] = run;
-                run += v[k];
-            }
-    }
-    if (blockIdx.x == 0 && threadIdx.x == 0) offset[cells] = chunk_offset[nb];
 }
 
 // SceneData::PointDistanceToCamera (SceneData.cpp:645-669): distance from every point to the nearest camera that sees
@@ -582,56 +835,55 @@ __global__ __launch_bounds__(kBlock) void camera_distance_kernel(const float4* _
 // undecided to kept / erased, so reading a neighbour's state of this round instead of the last one is as good.
 // One thread per point in cell order; count[round] receives the points still undecided after this round, and a round
 // that finds count[round - 1] == 0 has nothing to do.
+// The cells a ball can reach are those of the corners of its bounding cube: the cell of a coordinate never decreases
+// with it, in fp32 as in real numbers, and a point counts only if every |difference of coordinates| is below the radius up to
+// the rounding of four operations, which the widened reach covers (1e-4 of the radius; 1e-20 where its square
+// underflows).  The radii of the filter are a hundredth of a cell: one row of one or two cells in place of the 27 around the
+// point (3 M points in random order: 730 -> 177 us, most of it the states and radii, which are gathered by id).
 constexpr int kStateUndecided = 0, kStateKept = 1, kStateErased = 2;
 
-__global__ __launch_bounds__(kBlock) void close_points_kernel(const float4* __restrict__ sorted, int n,
-                                                              const KnnGrid* __restrict__ gp,
-                                                              const uint32_t* __restrict__ offset,
-                                                              const float* __restrict__ radius, int32_t* state,
-                                                              uint32_t* round_count, int round)
+__global__ __launch_bounds__(kBlock) void close_points_kernel(KnnView kv, int n, const float* __restrict__ radius,
+                                                              int32_t* state, uint32_t* round_count, int round)
 {
     if (round > 0 && *(volatile uint32_t*)(round_count + round - 1) == 0) return;
     const int t = blockIdx.x * kBlock + threadIdx.x;
     bool pending = false;
     if (t < n)
     {
-        const KnnGrid g  = *gp;
-        const float4 p   = sorted[t];
+        const KnnGrid g  = *kv.grid;
+        const float4 p   = kv.sorted[t];
         const uint32_t i = __float_as_uint(p.w);
         if (__atomic_load_n(&state[i], __ATOMIC_RELAXED) == kStateUndecided)
         {
             const float rad = radius[i];
             const float r2  = rad * rad;
-            const int3 c    = grid_cell(g, p.x, p.y, p.z);
-            // cells the ball can reach (the cell of a point is computed in fp32: one cell of slack)
-            const float reach = fminf(fmaxf(rad, 0.f) * g.inv_cell, 1.0e6f);
-            const int rc      = (int)reach + 1;
-            const int z0 = max(c.z - rc, 0), z1 = min(c.z + rc, g.dim[2] - 1);
-            const int y0 = max(c.y - rc, 0), y1 = min(c.y + rc, g.dim[1] - 1);
-            const int x0 = max(c.x - rc, 0), x1 = min(c.x + rc, g.dim[0] - 1);
+            const float reach = fabsf(rad) * 1.0001f + 1.0e-20f;
+            const int3 lo   = grid_cell(g, p.x - reach, p.y - reach, p.z - reach);
+            const int3 hi   = grid_cell(g, p.x + reach, p.y + reach, p.z + reach);
             int result = kStateKept;
-            for (int cz = z0; cz <= z1 && result != kStateErased; ++cz)
-                for (int cy = y0; cy <= y1 && result != kStateErased; ++cy)
-                {
-                    const uint32_t row = grid_index(g, 0, cy, cz);
-                    const uint32_t e   = offset[row + x1 + 1];
-                    for (uint32_t q = offset[row + x0]; q < e; ++q)
+            for (int cz = lo.z; cz <= hi.z && result != kStateErased; ++cz)
+                for (int cy = lo.y; cy <= hi.y && result != kStateErased; ++cy)
+                    for (int part = lo.x >> kBrickX; part <= hi.x >> kBrickX && result != kStateErased; ++part)
                     {
-                        const float4 o   = sorted[q];
-                        const uint32_t j = __float_as_uint(o.w);
-                        if (j >= i) continue;
-                        const float dx = p.x - o.x, dy = p.y - o.y, dz = p.z - o.z;
-                        const float d2 = (dx * dx + dy * dy) + dz * dz;
-                        if (!(d2 < r2)) continue;
-                        const int sj = __atomic_load_n(&state[j], __ATOMIC_RELAXED);
-                        if (sj == kStateKept)
+                        const uint32_t slot = kv.slot[brick_row(g, cy, cz) + (uint32_t)part];
+                        if (slot == kNoBrick) continue;
+                        uint32_t q, e;
+                        brick_range(kv, slot, max(lo.x, part << kBrickX), min(hi.x, part << kBrickX | 7), cy, cz, &q, &e);
+                        for (; q < e; ++q)
                         {
-                            result = kStateErased;
-                            break;
+                            const float4 o   = kv.sorted[q];
+                            const uint32_t j = __float_as_uint(o.w);
+                            if (j >= i) continue;
+                            if (!(distance2(p, o) < r2)) continue;
+                            const int sj = __atomic_load_n(&state[j], __ATOMIC_RELAXED);
+                            if (sj == kStateKept)
+                            {
+                                result = kStateErased;
+                                break;
+                            }
+                            if (sj == kStateUndecided) result = kStateUndecided;
                         }
-                        if (sj == kStateUndecided) result = kStateUndecided;
                     }
-                }
             if (result != kStateUndecided) __atomic_store_n(&state[i], result, __ATOMIC_RELAXED);
             pending = result == kStateUndecided;
         }
@@ -669,42 +921,64 @@ __global__ __launch_bounds__(kBlock) void morton_kernel(const float4* __restrict
 // ------------------------------------------------------------------------------------------------
 // launchers
 // ------------------------------------------------------------------------------------------------
+int knn_sample_stride(int n) { return n >= (1 << 17) ? 16 : 1; }
+int knn_num_samples(int n) { return n < kKnnSamples ? n : kKnnSamples; }
+size_t knn_chunk_words() { return 2 * (size_t)kScanChunks; }
+
 void launch_knn_first_grid(const float4* position, int n, const KnnGrid& box, KnnGrid* dst, hipStream_t st)
 {
     hipLaunchKernelGGL(knn_first_grid_kernel, dim3(1), dim3(1024), 0, st, position, n, box, dst);
 }
 
-void launch_knn_refine_grid(const float* sample, int samples, const KnnGrid* first, KnnGrid* g, uint32_t budget,
-                            hipStream_t st)
+// The cells of the search grid as a multiple of the median distance d_R to the R-th neighbour: with 2 the cube of 3 x 3 x 3
+// cells settles every point whose own distance is below twice the median, with ~60 candidates on a surface and ~260 in
+// a volume.  Where the samples are taken in every s-th point, their nearest neighbour there stands in for the s-th in
+// the cloud, and d_R = d_s (R / s)^(1 / D) for a cloud of dimension D: 2.5 is within 14 % for surfaces and volumes alike.
+void launch_knn_refine_grid(const float* sample, int samples, int rank, int stride, const KnnGrid* first, KnnGrid* g,
+                            uint32_t budget, uint32_t* list_counts, hipStream_t st)
 {
-    hipLaunchKernelGGL(knn_refine_grid_kernel, dim3(1), dim3(1024), 0, st, sample, samples, first, g, budget);
+    const float factor = 2.0f * (stride > 1 ? powf((float)rank / (float)stride, 0.4f) : 1.0f);
+    hipLaunchKernelGGL(knn_refine_grid_kernel, dim3(1), dim3(1024), 0, st, sample, samples, factor, first, g, budget,
+                       list_counts);
 }
 
-int knn_num_samples(int n) { return n < kKnnSamples ? n : kKnnSamples; }
+static int bin_blocks(int n) { return (int)(((size_t)n + kBlock * kBinPer - 1) / (kBlock * kBinPer)); }
 
-// count, prefix sum and scatter of the points into the cells of *g (device)
-void launch_knn_build(const float4* position, int n, const KnnGrid* g, uint32_t max_cells, uint32_t* count,
-                      uint32_t* offset, uint32_t* chunk_sum, float4* sorted, hipStream_t st)
+// every stride-th point (n of them) in the cell order of the coarse grid
+void launch_knn_coarse(const float4* position, int n, int stride, const KnnGrid* g, uint32_t* count, uint32_t* start,
+                       uint32_t* rank, unsigned long long* chunk_sum, float4* sorted, const uint32_t* gate, hipStream_t st)
 {
-    const int chunks = (int)((max_cells + kScanChunk - 1) / kScanChunk);
-    const int blocks = chunks < 1024 ? chunks : 1024;
-    const int clear  = (int)((max_cells / 4 + kBlock - 1) / kBlock);
-    hipLaunchKernelGGL(knn_clear_kernel, dim3(clear < 4096 ? (clear ? clear : 1) : 4096), dim3(kBlock), 0, st, count, g);
-    hipLaunchKernelGGL(knn_bin_kernel, dim3((n + kBlock - 1) / kBlock), dim3(kBlock), 0, st, 0, position, n, g, count,
-                       offset, sorted);
-    // chunk sums and their offsets share one array: [chunks] sums, [chunks + 1] offsets
-    hipLaunchKernelGGL(knn_scan_reduce_kernel, dim3(blocks), dim3(1024), 0, st, count, g, chunk_sum);
-    hipLaunchKernelGGL(knn_scan_chunks_kernel, dim3(1), dim3(1024), 0, st, chunk_sum, g, chunk_sum + chunks);
-    hipLaunchKernelGGL(knn_scan_apply_kernel, dim3(blocks), dim3(1024), 0, st, count, g, chunk_sum + chunks, offset);
-    hipLaunchKernelGGL(knn_bin_kernel, dim3((n + kBlock - 1) / kBlock), dim3(kBlock), 0, st, 1, position, n, g, count,
-                       offset, sorted);
+    hipLaunchKernelGGL(knn_clear_kernel<false>, dim3(1024), dim3(kBlock), 0, st, count, g, gate);
+    hipLaunchKernelGGL(knn_count_kernel<false>, dim3(bin_blocks(n)), dim3(kBlock), 0, st, position, n, stride, g, count, rank, gate);
+    hipLaunchKernelGGL(knn_scan_reduce_kernel<false>, dim3(512), dim3(1024), 0, st, count, g, chunk_sum, gate);
+    hipLaunchKernelGGL(knn_scan_apply_kernel<false>, dim3(512), dim3(1024), 0, st, count, g, chunk_sum, start, nullptr, nullptr,
+                       nullptr, nullptr, gate);
+    hipLaunchKernelGGL(knn_scatter_kernel<false>, dim3(bin_blocks(n)), dim3(kBlock), 0, st, position, n, stride, g, start, rank,
+                       sorted, gate);
 }
 
-size_t knn_chunk_words(uint32_t max_cells)
+// the points in the order of the search grid's bricks and cells
+void launch_knn_bricks(const float4* position, int n, const KnnBricks& b, hipStream_t st)
 {
-    const size_t chunks = (max_cells + kScanChunk - 1) / kScanChunk;
-    return 2 * chunks + 1;
+    const int chunks = (int)((b.max_bricks + kScanChunk - 1) / kScanChunk);
+    hipLaunchKernelGGL(knn_clear_kernel<true>, dim3(1024), dim3(kBlock), 0, st, b.count, b.grid, nullptr);
+    hipLaunchKernelGGL(knn_count_kernel<true>, dim3(bin_blocks(n)), dim3(kBlock), 0, st, position, n, 1, b.grid, b.count, b.rank,
+                       nullptr);
+    hipLaunchKernelGGL(knn_scan_reduce_kernel<true>, dim3(chunks), dim3(1024), 0, st, b.count, b.grid, b.chunk_sum, nullptr);
+    hipLaunchKernelGGL(knn_scan_apply_kernel<true>, dim3(chunks), dim3(1024), 0, st, b.count, b.grid, b.chunk_sum, b.start, b.slot,
+                       b.slot_brick, b.num_slots, b.cell_start, nullptr);
+    hipLaunchKernelGGL(knn_scatter_kernel<true>, dim3(bin_blocks(n)), dim3(kBlock), 0, st, position, n, 1, b.grid, b.start, b.rank,
+                       b.scratch, nullptr);
+    // (as many wavefronts as there can be bricks with points, at most 2 per wave slot of the GPU)
+    const size_t slots = (size_t)n < b.max_bricks ? (size_t)n : b.max_bricks;
+    const size_t want  = (slots + kBlock / 64 - 1) / (kBlock / 64);
+    hipLaunchKernelGGL(knn_brick_sort_kernel, dim3((int)(want < 4096 ? want : 4096)), dim3(kBlock), 0, st, b.scratch, b.grid,
+                       b.num_slots, b.slot_brick, b.start, b.count, b.cell_start, b.sorted);
 }
+
+#define ADOP_KNN_RANKS                                                                                 \
+    ADOP_KNN_CASE(1) ADOP_KNN_CASE(2) ADOP_KNN_CASE(3) ADOP_KNN_CASE(4) ADOP_KNN_CASE(5) ADOP_KNN_CASE(6) \
+    ADOP_KNN_CASE(7) ADOP_KNN_CASE(8)
 
 bool launch_knn_sample(int rank, const float4* sorted, int n, const KnnGrid* g, const uint32_t* offset, float* out,
                        int samples, hipStream_t st)
@@ -714,33 +988,35 @@ bool launch_knn_sample(int rank, const float4* sorted, int n, const KnnGrid* g, 
     case R: hipLaunchKernelGGL(knn_sample_kernel<R + 1>, grid, block, 0, st, sorted, n, g, offset, out, samples); return true;
     switch (rank)
     {
-        ADOP_KNN_CASE(1) ADOP_KNN_CASE(2) ADOP_KNN_CASE(3) ADOP_KNN_CASE(4)
-        ADOP_KNN_CASE(5) ADOP_KNN_CASE(6) ADOP_KNN_CASE(7) ADOP_KNN_CASE(8)
+        ADOP_KNN_RANKS
     }
 #undef ADOP_KNN_CASE
     return false;
 }
 
-// The three stages of the search: second grid (all points), first grid (what that left), all points (strays).
-bool launch_knn_search(int rank, int n, const KnnSearchArg& a, float* out, hipStream_t st)
+// The four stages of the search: the cube of 27 cells (all points), 2 and 3 shells, the coarse grid over all points
+// (built only if something is left), all points (strays).
+bool launch_knn_search(int rank, const float4* position, int n, const KnnSearchArg& a, float* out, hipStream_t st)
 {
-    const dim3 block(kBlock), grid((n + kBlock - 1) / kBlock), grid2(512), grid3(1024);
-#define ADOP_KNN_CASE(R)                                                                                              \
-    case R:                                                                                                           \
-        hipLaunchKernelGGL(knn_search_kernel<R + 1>, grid, block, 0, st, a.sorted, n, a.grid, a.offset, out, a.list,   \
-                           a.counts);                                                                                 \
-        hipLaunchKernelGGL(knn_list_kernel<R + 1>, grid2, block, 0, st, a.sorted, a.list, a.counts, a.sorted0, a.grid0, \
-                           a.offset0, out, a.list2, a.counts + 1);                                                    \
-        hipLaunchKernelGGL(knn_brute_kernel<R + 1>, grid3, block, 0, st, a.sorted, n, a.list2, a.counts + 1, out);     \
+    const dim3 block(kBlock), grid((n + kBlock - 1) / kBlock), grid2(1024), grid3(1024);
+#define ADOP_KNN_CASE(R)                                                                                                \
+    case R:                                                                                                             \
+        hipLaunchKernelGGL(knn_search_kernel<R + 1>, grid, block, 0, st, a.view, n, out, a.list, a.counts);              \
+        hipLaunchKernelGGL(knn_shells_kernel<R + 1>, grid2, block, 0, st, a.view, a.list, a.counts, out, a.list2,        \
+                           a.counts + 1);                                                                               \
+        launch_knn_coarse(position, n, 1, a.grid0, a.count0, a.start0, a.rank, a.chunk_sum, a.sorted0, a.counts + 1, st); \
+        hipLaunchKernelGGL(knn_coarse_kernel<R + 1>, grid2, block, 0, st, a.view.sorted, a.list2, a.counts + 1,          \
+                           a.sorted0, a.grid0, a.start0, out, a.list, a.counts + 2);                                    \
+        hipLaunchKernelGGL(knn_brute_kernel<R + 1>, grid3, block, 0, st, a.view.sorted, n, a.list, a.counts + 2, out);   \
         return true;
     switch (rank)
     {
-        ADOP_KNN_CASE(1) ADOP_KNN_CASE(2) ADOP_KNN_CASE(3) ADOP_KNN_CASE(4)
-        ADOP_KNN_CASE(5) ADOP_KNN_CASE(6) ADOP_KNN_CASE(7) ADOP_KNN_CASE(8)
+        ADOP_KNN_RANKS
     }
 #undef ADOP_KNN_CASE
     return false;
 }
+#undef ADOP_KNN_RANKS
 
 void launch_camera_distance(const float4* position, int n, const ViewConst* views, int num_frames, float* out,
                             hipStream_t st)
@@ -749,11 +1025,11 @@ void launch_camera_distance(const float4* position, int n, const ViewConst* view
                        num_frames, out);
 }
 
-void launch_close_points(const float4* sorted, int n, const KnnGrid* g, const uint32_t* offset, const float* radius,
-                         int32_t* state, uint32_t* round_count, int round, hipStream_t st)
+void launch_close_points(const KnnView& view, int n, const float* radius, int32_t* state, uint32_t* round_count, int round,
+                         hipStream_t st)
 {
-    hipLaunchKernelGGL(close_points_kernel, dim3((n + kBlock - 1) / kBlock), dim3(kBlock), 0, st, sorted, n, g, offset,
-                       radius, state, round_count, round);
+    hipLaunchKernelGGL(close_points_kernel, dim3((n + kBlock - 1) / kBlock), dim3(kBlock), 0, st, view, n, radius, state,
+                       round_count, round);
 }
 
 void launch_morton(const float4* position, int n, const float* mn, const float* scale, unsigned long long* code,

@@ -34,11 +34,16 @@ def _bbox(position):
     return (C.c_float * 3)(*host[:3]), (C.c_float * 3)(*host[3:])
 
 
-def _knn_distance(position, rank, box):
+def _knn_workspace(position):
+    lib = _capi.load_library()
+    return torch.empty(int(lib.adop_knn_workspace_size(int(position.shape[0]))), dtype=torch.uint8, device=position.device)
+
+
+def _knn_distance(position, rank, box, ws=None):
     n = int(position.shape[0])
     lib = _capi.load_library()
     out = torch.empty(n, dtype=torch.float32, device=position.device)
-    ws = torch.empty(int(lib.adop_knn_workspace_size(n)), dtype=torch.uint8, device=position.device)
+    ws = _knn_workspace(position) if ws is None else ws
     rc = lib.adop_knn_distance(_ptr(position), n, int(rank), *box, _ptr(out), _ptr(ws), int(ws.numel()), _stream_ptr())
     _check(rc, lib)
     return out
@@ -103,38 +108,45 @@ def RemoveLonelyPoints(position, camera_distance, n=5, dis_th=0.02):
     return ~(d / camera_distance > dis_th)
 
 
-def RemoveClosePoints(position, camera_distance, dis_th=0.00005, rounds_per_call=8):
-    """Keep mask of SceneData::RemoveClosePoints (SceneData.cpp:598-642): in index order, a point goes when a point
-    kept before it lies within dis_th / camera_distance of it."""
-    assert position.is_cuda and position.dtype == torch.float32 and position.dim() == 2 and position.shape[1] == 4
-    position = position.contiguous()
-    n = int(position.shape[0])
-    radius = (dis_th / camera_distance).to(torch.float32).contiguous()
+def _decide_close_points(position, radius, box, state, ws, rounds_per_call, resume):
+    """Rounds of the close-point filter until every point is decided.  resume = 1: ``ws`` holds the search grid of these
+    points and ``state`` what is decided already."""
     lib = _capi.load_library()
-    state = torch.empty(n, dtype=torch.int32, device=position.device)
     undecided = torch.empty(rounds_per_call, dtype=torch.int32, device=position.device)
-    ws = torch.empty(int(lib.adop_knn_workspace_size(n)), dtype=torch.uint8, device=position.device)
-    mn, mx = _bbox(position)
-    resume = 0
     while True:
-        rc = lib.adop_close_points(C.c_void_p(position.data_ptr()), n, C.c_void_p(radius.data_ptr()), mn, mx,
-                                   C.c_void_p(state.data_ptr()), C.c_void_p(undecided.data_ptr()), rounds_per_call,
-                                   resume, C.c_void_p(ws.data_ptr()), int(ws.numel()), _stream_ptr())
+        rc = lib.adop_close_points(_ptr(position), int(position.shape[0]), _ptr(radius), *box, _ptr(state), _ptr(undecided),
+                                   rounds_per_call, resume, _ptr(ws), int(ws.numel()), _stream_ptr())
         _check(rc, lib)
         if int(undecided[-1].item()) == 0:
             return state == 1
         resume = 1
 
 
+def RemoveClosePoints(position, camera_distance, dis_th=0.00005, rounds_per_call=8):
+    """Keep mask of SceneData::RemoveClosePoints (SceneData.cpp:598-642): in index order, a point goes when a point
+    kept before it lies within dis_th / camera_distance of it."""
+    position = _checked_position(position)
+    radius = (dis_th / camera_distance).to(torch.float32).contiguous()
+    state = torch.empty(int(position.shape[0]), dtype=torch.int32, device=position.device)
+    return _decide_close_points(position, radius, _bbox(position), state, _knn_workspace(position), rounds_per_call, 0)
+
+
 def FilterPointCloud(position, poses_se3, intrinsics, frames, lonely=(5, 0.02), close=0.00005):
     """The two filters of a new scene in the reference's order (SceneData.cpp:98-99): RemoveLonelyPoints(5, 0.02), then
-    RemoveClosePoints(0.00005) on what is left.  Returns the ids of the surviving points, ascending."""
-    ids = torch.arange(int(position.shape[0]), device=position.device)
+    RemoveClosePoints(0.00005) on what is left.  Returns the ids of the surviving points, ascending.
+
+    One search grid serves both: a point the first filter takes is erased before the second one starts, and neither
+    the distances nor the order of the others change by its staying in the grid."""
     cam = PointDistanceToCamera(position, poses_se3, intrinsics, frames)  # per point: erasing others does not change it
-    keep = RemoveLonelyPoints(position, cam, *lonely)
-    position, cam, ids = position[keep].contiguous(), cam[keep], ids[keep]
-    keep = RemoveClosePoints(position, cam, close)
-    return ids[keep]
+    position = _checked_position(position)
+    box, ws = _bbox(position), _knn_workspace(position)
+    n, dis_th = lonely
+    state = (_knn_distance(position, n, box, ws) / cam > dis_th).to(torch.int32) * 2  # 2: erased
+    radius = (close / cam).to(torch.float32)
+    ids = _decide_close_points(position, radius, box, state, ws, 8, 1).nonzero().squeeze(1)
+    if ids.numel() == 0:  # (the first point the lonely filter leaves stays, so it has left none)
+        raise RuntimeError("FilterPointCloud: no point is left")
+    return ids
 
 
 def ReorderMorton64(position):

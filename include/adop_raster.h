@@ -336,7 +336,9 @@ adop_status adop_point_distance_to_camera_static(const adop_scene* scene, const 
  * point j < i with state[j] = 1 (kept) lies closer than radius[i] (d2 < radius^2 in fp32), else 1; the result equals
  * the sweep in index order.  The points are decided in rounds (a point waits for its earlier neighbours):
  * round_undecided [num_rounds] (device) receives the number of points still 0 (undecided) after every round; when
- * the last entry is not 0 call again with resume = 1 and the workspace untouched.  state [N] int32 (device),
+ * the last entry is not 0 call again with resume = 1 and the workspace untouched.  resume = 1 also starts from the
+ * workspace that adop_knn_distance left for the same points, with the states preset by the caller (0 undecided, 2 erased
+ * beforehand: such a point is as if it were not there).  state [N] int32 (device),
  * radius [N] f32, workspace: adop_knn_workspace_size(num_points) bytes. */
 adop_status adop_close_points(const float* position, int32_t num_points, const float* radius, const float* bbox_min,
                               const float* bbox_max, int32_t* state, uint32_t* round_undecided, int32_t num_rounds,

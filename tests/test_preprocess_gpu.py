@@ -293,3 +293,44 @@ def test_bounding_box_and_gather(n):
     p[n - 1, 1] = float("nan")
     with pytest.raises(RuntimeError, match="not finite"):
         pp.MortonCodes(p)
+
+
+@pytest.mark.parametrize("kind", ["surface", "volume", "clusters", "one_brick", "tails", "line"])
+def test_knn_distance_of_large_clouds(kind):
+    """From 2^17 points on the search grid is sized on every 16th point; the clouds here fill its bricks in ways that take every
+    branch: bricks of more than 256 points (clusters, one_brick), points that only the coarse grid reaches (tails),
+    rows across brick borders.  Distances of a sample bit for bit against the distances to all points."""
+    import torch
+    from adop_amd import preprocess
+
+    n = (1 << 17) + 77
+    g = np.random.default_rng(3)
+    xyz = {"surface": lambda: g.random((n, 3)) * [4.0, 3.0, 0.0] + [0, 0, 1.0],
+           "volume": lambda: g.random((n, 3)) - 0.5,
+           "clusters": lambda: g.standard_normal((n, 3)) * 1e-3 * 10.0 ** g.integers(0, 3, (n, 1)) + g.integers(0, 9, (n, 3)),
+           "one_brick": lambda: np.concatenate([g.random((n - 40, 3)), g.random((40, 3)) * 1e-4 + 0.5]) * [1.0, 1e-3, 1e-3],
+           "tails": lambda: g.standard_cauchy((n, 3)),
+           "line": lambda: np.outer(g.random(n), [3.0, 0.0, 0.0])}[kind]().astype(np.float32)
+    p = np.zeros((n, 4), np.float32)
+    p[:, :3] = xyz
+    announce(f"knn distance, {kind}, N={n}")
+    dev = torch.from_numpy(p).cuda()
+    sample = np.concatenate([g.integers(0, n, 400), [0, n - 1], np.argsort(np.abs(xyz).max(1))[-40:]])
+    q = dev[torch.from_numpy(sample).cuda(), :3]
+    for rank in (1, 4, 8):
+        got = preprocess.KNearestNeighbourDistance(dev, rank)
+        d = [q[:, k, None] - dev[None, :, k] for k in range(3)]
+        want = ((d[0] * d[0] + d[1] * d[1]) + d[2] * d[2]).kthvalue(rank + 1, dim=1).values.sqrt()
+        assert torch.equal(got[torch.from_numpy(sample).cuda()].view(torch.int32), want.view(torch.int32)), (kind, rank)
+
+
+def test_filter_refuses_a_cloud_it_empties():
+    import torch
+    from adop_amd import preprocess, scenes
+
+    p, views, poses, K, fr = _orbit_scene(500, 2, 8)
+    announce("FilterPointCloud that leaves nothing")
+    with pytest.raises(RuntimeError):
+        preprocess.FilterPointCloud(torch.from_numpy(p).cuda(), torch.from_numpy(views).cuda(), torch.from_numpy(K).cuda(),
+                                    [scenes.make_view(w, h, image_index=f, camera_index=c) for w, h, f, c in fr],
+                                    lonely=(5, 0.0))
