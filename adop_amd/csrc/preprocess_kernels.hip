@@ -423,6 +423,8 @@ __device__ __forceinline__ void wave_push(bool push, uint32_t value, uint32_t* _
 // loop over all runs, so that a wavefront takes as many rounds as its fullest cube has candidates and not, row after
 // row, as the fullest row.  Points whose n-th neighbour may lie outside the cube go to list.
 constexpr int kMaxRuns = 18;
+constexpr int kUnroll  = 6;  // candidates of a run per round, their loads in flight together (10 M points on patches, whole
+                             // call: 1: 1720 us, 2: 1490, 4: 1300, 6: 1264, 8: 1279)
 
 template <int K>  // K = n + 1 best squared distances are kept (the point itself is one of them)
 __global__ __launch_bounds__(kBlock) void knn_search_kernel(KnnView kv, int n, float* __restrict__ out,
@@ -473,117 +475,22 @@ __global__ __launch_bounds__(kBlock) void knn_search_kernel(KnnView kv, int n, f
             q             = r.x;
             e             = r.y;
         }
-        const float4 o0 = kv.sorted[q], o1 = kv.sorted[min(q + 1, e - 1)];
-        const float d0 = distance2(p, o0), d1 = distance2(p, o1);
-        keep_smallest<K>(best, d0);
-        keep_smallest<K>(best, q + 1 < e ? d1 : 3.0e38f);
-        q += 2;
+        float4 o[kUnroll];
+#pragma unroll
+        for (int u = 0; u < kUnroll; ++u) o[u] = kv.sorted[min(q + u, e - 1)];
+#pragma unroll
+        for (int u = 0; u < kUnroll; ++u) keep_smallest<K>(best, q + u < e ? distance2(p, o[u]) : 3.0e38f);
+        q += kUnroll;
     }
     const bool settled = cube_settles(best[K - 1], cube_bound(g, p, c, 1));
     if (t < n && settled) out[__float_as_uint(p.w)] = sqrtf(best[K - 1]);
     wave_push(t < n && !settled, (uint32_t)t, list, list_count);
 }
 
-// Stage 2: the points stage 1 left, cubes of 2 and 3 shells of the same grid; the rest goes to list2.  A larger cube is
-// searched from scratch.
+// K-th smallest of the union of the lanes' ascending lists (destroys them): K rounds of taking the smallest head.  all != null
+// receives the K smallest.
 template <int K>
-__global__ __launch_bounds__(kBlock) void knn_shells_kernel(KnnView kv, const uint32_t* __restrict__ list,
-                                                            const uint32_t* __restrict__ list_count,
-                                                            float* __restrict__ out, uint32_t* __restrict__ list2,
-                                                            uint32_t* list2_count)
-{
-    const uint32_t count = *list_count;
-    const KnnGrid g      = *kv.grid;
-    const uint32_t lane  = threadIdx.x & 63;
-    for (uint32_t e0 = blockIdx.x * kBlock + (threadIdx.x & ~63u); e0 < count; e0 += gridDim.x * kBlock)  // wavefront-uniform
-    {
-        const uint32_t e = e0 + lane;
-        bool left        = false;
-        uint32_t t       = 0;
-        if (e < count)
-        {
-            t              = list[e];
-            const float4 p = kv.sorted[t];
-            const int3 c   = grid_cell(g, p.x, p.y, p.z);
-            left           = true;
-            for (int r = 2; r <= 3 && left; ++r)
-            {
-                float best[K];
-#pragma unroll
-                for (int k = 0; k < K; ++k) best[k] = 3.0e38f;
-                const int x0 = max(c.x - r, 0), x1 = min(c.x + r, g.dim[0] - 1);
-                for (int cz = max(c.z - r, 0); cz <= min(c.z + r, g.dim[2] - 1); ++cz)
-                    for (int cy = max(c.y - r, 0); cy <= min(c.y + r, g.dim[1] - 1); ++cy)
-                        for (int part = x0 >> kBrickX; part <= x1 >> kBrickX; ++part)
-                        {
-                            const uint32_t slot = kv.slot[brick_row(g, cy, cz) + (uint32_t)part];
-                            if (slot == kNoBrick) continue;
-                            uint32_t q, end;
-                            brick_range(kv, slot, max(x0, part << kBrickX), min(x1, part << kBrickX | 7), cy, cz, &q, &end);
-                            for (; q < end; ++q) keep_smallest<K>(best, distance2(p, kv.sorted[q]));
-                        }
-                if (cube_settles(best[K - 1], cube_bound(g, p, c, r)))
-                {
-                    out[__float_as_uint(p.w)] = sqrtf(best[K - 1]);
-                    left                      = false;
-                }
-            }
-        }
-        wave_push(left, t, list2, list2_count);
-    }
-}
-
-// Stage 3: what is left (points in sparse parts of the cloud), on the coarse grid over all points, at most 4 shells; the
-// rest goes to list3.
-template <int K>
-__global__ __launch_bounds__(kBlock) void knn_coarse_kernel(const float4* __restrict__ points,
-                                                            const uint32_t* __restrict__ list,
-                                                            const uint32_t* __restrict__ list_count,
-                                                            const float4* __restrict__ sorted0,
-                                                            const KnnGrid* __restrict__ gp0,
-                                                            const uint32_t* __restrict__ start0, float* __restrict__ out,
-                                                            uint32_t* __restrict__ list3, uint32_t* list3_count)
-{
-    const uint32_t count = *list_count;
-    const KnnGrid g      = *gp0;
-    const uint32_t lane  = threadIdx.x & 63;
-    for (uint32_t e0 = blockIdx.x * kBlock + (threadIdx.x & ~63u); e0 < count; e0 += gridDim.x * kBlock)  // wavefront-uniform
-    {
-        const uint32_t e = e0 + lane;
-        bool left        = false;
-        uint32_t t       = 0;
-        if (e < count)
-        {
-            t              = list[e];
-            const float4 p = points[t];
-            const int3 c   = grid_cell(g, p.x, p.y, p.z);
-            left           = true;
-            for (int r = 1; r <= 4 && left; ++r)
-            {
-                float best[K];
-#pragma unroll
-                for (int k = 0; k < K; ++k) best[k] = 3.0e38f;
-                const int x0 = max(c.x - r, 0), x1 = min(c.x + r, g.dim[0] - 1);
-                for (int cz = max(c.z - r, 0); cz <= min(c.z + r, g.dim[2] - 1); ++cz)
-                    for (int cy = max(c.y - r, 0); cy <= min(c.y + r, g.dim[1] - 1); ++cy)
-                    {
-                        const uint32_t row = grid_index(g, 0, cy, cz), end = start0[row + x1 + 1];
-                        for (uint32_t q = start0[row + x0]; q < end; ++q) keep_smallest<K>(best, distance2(p, sorted0[q]));
-                    }
-                if (cube_settles(best[K - 1], cube_bound(g, p, c, r)))
-                {
-                    out[__float_as_uint(p.w)] = sqrtf(best[K - 1]);
-                    left                      = false;
-                }
-            }
-        }
-        wave_push(left, t, list3, list3_count);
-    }
-}
-
-// K-th smallest of the union of the lanes' ascending lists (destroys them): K rounds of taking the smallest head.
-template <int K>
-__device__ __forceinline__ float wave_kth(float* best)
+__device__ __forceinline__ float wave_kth(float* best, float* all = nullptr)
 {
     const int lane = threadIdx.x & 63;
     float kth      = 3.0e38f;
@@ -594,6 +501,7 @@ __device__ __forceinline__ float wave_kth(float* best)
 #pragma unroll
         for (int off = 32; off > 0; off >>= 1) m = fminf(m, __shfl_xor(m, off, 64));
         kth = m;
+        if (all && lane == 0) all[k] = m;
         const unsigned long long holders = __ballot(best[0] == m);
         if (lane == __ffsll((long long)holders) - 1)
         {
@@ -605,26 +513,140 @@ __device__ __forceinline__ float wave_kth(float* best)
     return kth;
 }
 
-// Stage 4: stray points far from everything (no cube of a few shells of either grid settles them): one wavefront
-// per point goes through all points.
+// Stage 2: the points stage 1 left, cubes of 2 and 3 shells of the same grid, one wavefront per point: the lanes share the
+// rows of the cube (a thread per point waits for 25 to 49 rows one after the other, and few points are left: 250 us for a
+// list that a wavefront per point works off in 15).  A larger cube is searched from scratch; the rest goes to list2.
 template <int K>
-__global__ __launch_bounds__(kBlock) void knn_brute_kernel(const float4* __restrict__ points, int n,
-                                                           const uint32_t* __restrict__ list,
-                                                           const uint32_t* __restrict__ list_count,
-                                                           float* __restrict__ out)
+__global__ __launch_bounds__(kBlock) void knn_shells_kernel(KnnView kv, const uint32_t* __restrict__ list,
+                                                            const uint32_t* __restrict__ list_count,
+                                                            float* __restrict__ out, uint32_t* __restrict__ list2,
+                                                            uint32_t* list2_count)
 {
     const uint32_t count = *list_count;
+    const KnnGrid g      = *kv.grid;
     const int lane       = threadIdx.x & 63;
     for (uint32_t e = blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6); e < count; e += gridDim.x * (kBlock / 64))
+    {
+        const uint32_t t = list[e];
+        const float4 p   = kv.sorted[t];
+        const int3 c     = grid_cell(g, p.x, p.y, p.z);
+        bool left        = true;
+        for (int r = 2; r <= 3 && left; ++r)  // (uniform over the wavefront)
+        {
+            float best[K];
+#pragma unroll
+            for (int k = 0; k < K; ++k) best[k] = 3.0e38f;
+            const int x0 = max(c.x - r, 0), x1 = min(c.x + r, g.dim[0] - 1);
+            const int rows = 2 * r + 1;
+            for (int q = lane; q < 2 * rows * rows; q += 64)  // (a row lies in two bricks at most)
+            {
+                const int row = q >> 1, part = (x0 >> kBrickX) + (q & 1);
+                const int cy = c.y - r + row % rows, cz = c.z - r + row / rows;
+                if ((unsigned)cy >= (unsigned)g.dim[1] || (unsigned)cz >= (unsigned)g.dim[2] || part > x1 >> kBrickX) continue;
+                const uint32_t slot = kv.slot[brick_row(g, cy, cz) + (uint32_t)part];
+                if (slot == kNoBrick) continue;
+                uint32_t i, end;
+                brick_range(kv, slot, max(x0, part << kBrickX), min(x1, part << kBrickX | 7), cy, cz, &i, &end);
+                for (; i < end; ++i) keep_smallest<K>(best, distance2(p, kv.sorted[i]));
+            }
+            const float kth = wave_kth<K>(best);
+            if (cube_settles(kth, cube_bound(g, p, c, r)))
+            {
+                if (lane == 0) out[__float_as_uint(p.w)] = sqrtf(kth);
+                left = false;
+            }
+        }
+        if (left && lane == 0) list2[atomicAdd(list2_count, 1u)] = t;
+    }
+}
+
+// The K-th smallest squared distance of point p on the coarse grid: cubes of 1 to 4 shells, by one wavefront (every lane takes
+// its share of the candidates of a row and keeps the K best of them).  False: 4 shells do not settle it.  Uniform over the
+// wavefront.
+template <int K>
+__device__ __forceinline__ bool coarse_cubes(const float4 p, const KnnGrid& g, const float4* __restrict__ sorted,
+                                             const uint32_t* __restrict__ start, float* kth)
+{
+    const int lane = threadIdx.x & 63;
+    const int3 c   = grid_cell(g, p.x, p.y, p.z);
+    for (int r = 1; r <= 4; ++r)
+    {
+        float best[K];
+#pragma unroll
+        for (int k = 0; k < K; ++k) best[k] = 3.0e38f;
+        const int x0 = max(c.x - r, 0), x1 = min(c.x + r, g.dim[0] - 1);
+        for (int cz = max(c.z - r, 0); cz <= min(c.z + r, g.dim[2] - 1); ++cz)
+            for (int cy = max(c.y - r, 0); cy <= min(c.y + r, g.dim[1] - 1); ++cy)
+            {
+                const uint32_t row = grid_index(g, 0, cy, cz), e = start[row + x1 + 1];
+                for (uint32_t q = start[row + x0] + lane; q < e; q += 64) keep_smallest<K>(best, distance2(p, sorted[q]));
+            }
+        *kth = wave_kth<K>(best);
+        if (cube_settles(*kth, cube_bound(g, p, c, r))) return true;
+    }
+    return false;
+}
+
+// Stage 3: what is left (points in sparse parts of the cloud), on the coarse grid over all points, at most 4 shells, one
+// wavefront per point; the rest goes to list3.
+template <int K>
+__global__ __launch_bounds__(kBlock) void knn_coarse_kernel(const float4* __restrict__ points,
+                                                            const uint32_t* __restrict__ list,
+                                                            const uint32_t* __restrict__ list_count,
+                                                            const float4* __restrict__ sorted0,
+                                                            const KnnGrid* __restrict__ gp0,
+                                                            const uint32_t* __restrict__ start0, float* __restrict__ out,
+                                                            uint32_t* __restrict__ list3, uint32_t* list3_count)
+{
+    const uint32_t count = *list_count;
+    const KnnGrid g      = *gp0;
+    const int lane       = threadIdx.x & 63;
+    for (uint32_t e = blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6); e < count; e += gridDim.x * (kBlock / 64))
+    {
+        const uint32_t t = list[e];
+        const float4 p   = points[t];
+        float kth;
+        if (coarse_cubes<K>(p, g, sorted0, start0, &kth))
+        {
+            if (lane == 0) out[__float_as_uint(p.w)] = sqrtf(kth);
+        }
+        else if (lane == 0)
+            list3[atomicAdd(list3_count, 1u)] = t;
+    }
+}
+
+// Stage 4: stray points far from everything (no cube of a few shells of either grid settles them): one workgroup per point
+// goes through all points (a wavefront per point, 1 M points of a Gaussian cloud: 1.5 ms; a workgroup of 16: 0.25 ms - there
+// are fewer strays than the GPU has wavefronts).
+constexpr int kBruteBlock = 1024;
+
+template <int K>
+__global__ __launch_bounds__(kBruteBlock) void knn_brute_kernel(const float4* __restrict__ points, int n,
+                                                                const uint32_t* __restrict__ list,
+                                                                const uint32_t* __restrict__ list_count,
+                                                                float* __restrict__ out)
+{
+    __shared__ float s_best[kBruteBlock / 64][K];
+    const uint32_t count = *list_count;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    for (uint32_t e = blockIdx.x; e < count; e += gridDim.x)
     {
         const float4 p = points[list[e]];
         float best[K];
 #pragma unroll
         for (int k = 0; k < K; ++k) best[k] = 3.0e38f;
 #pragma unroll 4
-        for (int q = lane; q < n; q += 64) keep_smallest<K>(best, distance2(p, points[q]));
-        const float kth = wave_kth<K>(best);
-        if (lane == 0) out[__float_as_uint(p.w)] = sqrtf(kth);
+        for (int q = threadIdx.x; q < n; q += kBruteBlock) keep_smallest<K>(best, distance2(p, points[q]));
+        wave_kth<K>(best, s_best[wave]);
+        __syncthreads();
+        if (wave == 0)  // the wavefronts' lists, one per lane
+        {
+#pragma unroll
+            for (int k = 0; k < K; ++k) best[k] = lane < kBruteBlock / 64 ? s_best[lane][k] : 3.0e38f;
+            const float kth = wave_kth<K>(best);
+            if (lane == 0) out[__float_as_uint(p.w)] = sqrtf(kth);
+        }
+        __syncthreads();  // s_best has been read
     }
 }
 
@@ -642,30 +664,9 @@ __global__ __launch_bounds__(kBlock) void knn_sample_kernel(const float4* __rest
     const int lane = threadIdx.x & 63;
     if (slot >= samples) return;
     const int t     = (int)((long long)slot * n / samples);
-    const KnnGrid g = *gp;
-    const float4 p  = sorted[t];
-    const int3 c    = grid_cell(g, p.x, p.y, p.z);
-    float result    = 3.0e38f;
-    for (int r = 1; r <= 4; ++r)
-    {
-        float best[K];
-#pragma unroll
-        for (int k = 0; k < K; ++k) best[k] = 3.0e38f;
-        const int x0 = max(c.x - r, 0), x1 = min(c.x + r, g.dim[0] - 1);
-        for (int cz = max(c.z - r, 0); cz <= min(c.z + r, g.dim[2] - 1); ++cz)
-            for (int cy = max(c.y - r, 0); cy <= min(c.y + r, g.dim[1] - 1); ++cy)
-            {
-                const uint32_t row = grid_index(g, 0, cy, cz), e = offset[row + x1 + 1];
-                for (uint32_t q = offset[row + x0] + lane; q < e; q += 64) keep_smallest<K>(best, distance2(p, sorted[q]));
-            }
-        const float kth = wave_kth<K>(best);
-        if (cube_settles(kth, cube_bound(g, p, c, r)))
-        {
-            result = sqrtf(kth);
-            break;
-        }
-    }
-    if (lane == 0) out[slot] = result;
+    float kth;
+    const bool settled = coarse_cubes<K>(sorted[t], *gp, sorted, offset, &kth);
+    if (lane == 0) out[slot] = settled ? sqrtf(kth) : 3.0e38f;
 }
 
 // ---- sizing the grids -------------------------------------------------------------------------------------------
@@ -930,14 +931,16 @@ void launch_knn_first_grid(const float4* position, int n, const KnnGrid& box, Kn
     hipLaunchKernelGGL(knn_first_grid_kernel, dim3(1), dim3(1024), 0, st, position, n, box, dst);
 }
 
-// The cells of the search grid as a multiple of the median distance d_R to the R-th neighbour: with 2 the cube of 3 x 3 x 3
-// cells settles every point whose own distance is below twice the median, with ~60 candidates on a surface and ~260 in
-// a volume.  Where the samples are taken in every s-th point, their nearest neighbour there stands in for the s-th in
-// the cloud, and d_R = d_s (R / s)^(1 / D) for a cloud of dimension D: 2.5 is within 14 % for surfaces and volumes alike.
+// The cells of the search grid as a multiple of the median distance d_R to the R-th neighbour.  Smaller cells mean fewer
+// candidates (their number goes with the square of the cell on a surface, with the cube in a volume) and more points that the
+// cube of 27 cells does not settle.  1.5 measured best over surfaces and volumes (search of 10 M points on 1000 patches,
+// 3 M in a volume, whole call: 2.0: 1365, 786 us; 1.5: 1264, 574; 1.2: 1283, 1015).  Where the samples are taken in every
+// s-th point, their nearest neighbour there stands in for the s-th in the cloud, and d_R = d_s (R / s)^(1 / D) for a
+// cloud of dimension D: 2.5 is within 14 % for surfaces and volumes alike.
 void launch_knn_refine_grid(const float* sample, int samples, int rank, int stride, const KnnGrid* first, KnnGrid* g,
                             uint32_t budget, uint32_t* list_counts, hipStream_t st)
 {
-    const float factor = 2.0f * (stride > 1 ? powf((float)rank / (float)stride, 0.4f) : 1.0f);
+    const float factor = 1.5f * (stride > 1 ? powf((float)rank / (float)stride, 0.4f) : 1.0f);
     hipLaunchKernelGGL(knn_refine_grid_kernel, dim3(1), dim3(1024), 0, st, sample, samples, factor, first, g, budget,
                        list_counts);
 }
@@ -998,7 +1001,7 @@ bool launch_knn_sample(int rank, const float4* sorted, int n, const KnnGrid* g, 
 // (built only if something is left), all points (strays).
 bool launch_knn_search(int rank, const float4* position, int n, const KnnSearchArg& a, float* out, hipStream_t st)
 {
-    const dim3 block(kBlock), grid((n + kBlock - 1) / kBlock), grid2(1024), grid3(1024);
+    const dim3 block(kBlock), grid((n + kBlock - 1) / kBlock), grid2(2048), grid3(512);
 #define ADOP_KNN_CASE(R)                                                                                                \
     case R:                                                                                                             \
         hipLaunchKernelGGL(knn_search_kernel<R + 1>, grid, block, 0, st, a.view, n, out, a.list, a.counts);              \
@@ -1007,7 +1010,7 @@ bool launch_knn_search(int rank, const float4* position, int n, const KnnSearchA
         launch_knn_coarse(position, n, 1, a.grid0, a.count0, a.start0, a.rank, a.chunk_sum, a.sorted0, a.counts + 1, st); \
         hipLaunchKernelGGL(knn_coarse_kernel<R + 1>, grid2, block, 0, st, a.view.sorted, a.list2, a.counts + 1,          \
                            a.sorted0, a.grid0, a.start0, out, a.list, a.counts + 2);                                    \
-        hipLaunchKernelGGL(knn_brute_kernel<R + 1>, grid3, block, 0, st, a.view.sorted, n, a.list, a.counts + 2, out);   \
+        hipLaunchKernelGGL(knn_brute_kernel<R + 1>, grid3, dim3(kBruteBlock), 0, st, a.view.sorted, n, a.list, a.counts + 2, out);   \
         return true;
     switch (rank)
     {
