@@ -1019,7 +1019,6 @@ static KnnWorkspace knn_layout(void* workspace, int32_t num_points)
 {
     const size_t bricks = knn_max_bricks(num_points);
     const size_t n      = (size_t)(num_points > 0 ? num_points : 0);
-    const size_t slots  = bricks < n ? bricks : n;
     size_t o            = 0;
     auto take           = [&](size_t bytes) {
         const size_t at = o;
@@ -1040,14 +1039,14 @@ static KnnWorkspace knn_layout(void* workspace, int32_t num_points)
     b.count      = (uint32_t*)take(sizeof(uint32_t) * bricks);
     b.start      = (uint32_t*)take(sizeof(uint32_t) * bricks);
     b.slot       = (uint32_t*)take(sizeof(uint32_t) * bricks);
-    b.slot_brick = (uint32_t*)take(sizeof(uint32_t) * slots);
-    b.cell_start = (uint32_t*)take(sizeof(uint32_t) * (slots * kBrickCells + 1));
-    b.rank       = (uint32_t*)take(sizeof(uint32_t) * n);
+    b.slot_brick = (uint32_t*)take(sizeof(uint32_t) * bricks);
+    b.cell_start = (uint32_t*)take(sizeof(uint32_t) * (bricks * kBrickCells + 1));
     b.scratch    = (float4*)take(sizeof(float4) * n);  // (also the points in the order of the coarse grid)
     b.sorted     = (float4*)take(sizeof(float4) * n);
     w.count0     = (uint32_t*)take(sizeof(uint32_t) * (size_t)kKnnFirstCells);
     w.start0     = (uint32_t*)take(sizeof(uint32_t) * ((size_t)kKnnFirstCells + 1));
     w.list       = (uint32_t*)take(sizeof(uint32_t) * n);
+    b.rank       = w.list;  // (a grid is built before the first list is written, and the coarse one when it has been read)
     w.list2      = (uint32_t*)take(sizeof(uint32_t) * n);
     w.total      = o;
     return w;
@@ -1185,6 +1184,25 @@ adop_status adop_point_distance_to_camera(const adop_scene* scene, const adop_vi
     if (!workspace || workspace_bytes < adop_frames_workspace_size(num_frames))
         return fail(ADOP_WORKSPACE_TOO_SMALL, "workspace too small");
     return camera_distance_run(scene, frames, num_frames, out_distance, (ViewConst*)workspace, (hipStream_t)hip_stream);
+}
+
+adop_status adop_point_distance_to_camera_grid(const adop_scene* scene, const adop_view* frames, int32_t num_frames,
+                                               float* out_distance, void* workspace, size_t workspace_bytes,
+                                               const void* knn_workspace, size_t knn_workspace_bytes, void* hip_stream)
+{
+    adop_status st = camera_distance_check(scene, frames, num_frames, out_distance);
+    if (st != ADOP_OK) return st;
+    if (scene->num_points < 1) return fail(ADOP_INVALID_ARG, "empty cloud");
+    if (!workspace || workspace_bytes < adop_frames_workspace_size(num_frames) || !knn_workspace ||
+        knn_workspace_bytes < adop_knn_workspace_size(scene->num_points))
+        return fail(ADOP_WORKSPACE_TOO_SMALL, "workspace too small");
+    hipStream_t stream = (hipStream_t)hip_stream;
+    if ((st = upload_views(scene, frames, num_frames, (ViewConst*)workspace, stream)) != ADOP_OK) return st;
+    const KnnWorkspace w = knn_layout((void*)knn_workspace, scene->num_points);
+    launch_camera_distance_sorted(w.bricks.sorted, scene->num_points, (const ViewConst*)workspace, num_frames, out_distance,
+                                  stream);
+    ADOP_HIP_CHECK(hipGetLastError());
+    return ADOP_OK;
 }
 
 int32_t adop_static_max_frames(void)

@@ -233,6 +233,25 @@ __device__ __forceinline__ T wave_sum(T v)
     return v;
 }
 
+// Smallest value of the wavefront's lanes, in every lane (six DPP steps, no LDS).  NaNs are left out.
+template <int CTRL, int ROWS>
+__device__ __forceinline__ float dpp_or_own(float v)
+{
+    const int i = (int)__float_as_uint(v);
+    return __uint_as_float((uint32_t)__builtin_amdgcn_update_dpp(i, i, CTRL, ROWS, 0xF, false));
+}
+__device__ __forceinline__ float wave_min(float v)
+{
+    v = fminf(v, dpp_or_own<0x111, 0xF>(v));  // row_shr:1, 2, 4, 8: the last lane of a row of 16 holds its minimum
+    v = fminf(v, dpp_or_own<0x112, 0xF>(v));
+    v = fminf(v, dpp_or_own<0x114, 0xF>(v));
+    v = fminf(v, dpp_or_own<0x118, 0xF>(v));
+    v = fminf(v, dpp_or_own<0x142, 0xA>(v));  // row_bcast:15, then row_bcast:31: lane 63 holds that of all rows
+    v = fminf(v, dpp_or_own<0x143, 0xC>(v));
+    return __uint_as_float((uint32_t)__builtin_amdgcn_readlane((int)__float_as_uint(v), 63));
+}
+__device__ __forceinline__ float wave_max(float v) { return -wave_min(-v); }
+
 // counter += number of lanes with pred (one atomic per wavefront; counter passes only)
 __device__ __forceinline__ void stat_add(uint64_t* dst, bool pred)
 {

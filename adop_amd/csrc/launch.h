@@ -55,6 +55,8 @@ struct KnnSearchArg
 bool launch_knn_search(int rank, const float4* position, int n, const KnnSearchArg& a, float* out, hipStream_t st);
 void launch_camera_distance(const float4* position, int n, const ViewConst* views, int num_frames, float* out,
                             hipStream_t st);
+void launch_camera_distance_sorted(const float4* sorted, int n, const ViewConst* views, int num_frames, float* out,
+                                   hipStream_t st);
 void launch_close_points(const KnnView& view, int n, const float* radius, int32_t* state, uint32_t* round_count, int round,
                          hipStream_t st);
 size_t bounding_box_floats();  // the box and the partial boxes behind it

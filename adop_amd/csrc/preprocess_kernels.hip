@@ -801,6 +801,20 @@ __global__ __launch_bounds__(1024) void knn_refine_grid_kernel(const float* __re
     *gp        = g;
 }
 
+// One frame of it: the squared distance of the point, if the frame sees it and it is smaller.
+__device__ __forceinline__ void nearest_camera(const ViewConst& vc, V3 pos, float* best)
+{
+    const V3 r = quat_rotate(vc.qx, vc.qy, vc.qz, vc.qw, pos);
+    const V3 v = {r.x + vc.tx, r.y + vc.ty, r.z + vc.tz};
+    const float d = (v.x * v.x + v.y * v.y) + v.z * v.z;
+    if (!(v.z > 0.f) || !(d < *best)) return;
+    const V2 np   = {v.x / v.z, v.y / v.z};
+    const V2 dp   = distort<false>(np, vc.d, 3.0e38f, nullptr, nullptr);
+    const V2 ip   = k_apply(vc.k, dp);
+    const bool in = ip.x >= 0.f && ip.y >= 0.f && ip.x < (float)vc.w && ip.y < (float)vc.h;
+    if (in) *best = d;
+}
+
 // SceneData::PointDistanceToCamera (SceneData.cpp:645-669): distance from every point to the nearest camera that sees
 // it (in front of the camera, projected inside the image with the frame's pinhole + distortion model), 10258.4 (the
 // root of the reference's start value 105235545) where no frame does.  The distance is taken in camera space
@@ -814,20 +828,53 @@ __global__ __launch_bounds__(kBlock) void camera_distance_kernel(const float4* _
     const float4 P = nt_load4(position + i);
     const V3 pos   = {P.x, P.y, P.z};
     float best     = 105235545.f;
-    for (int f = 0; f < num_frames; ++f)
-    {
-        const ViewConst& vc = views[f];
-        const V3 r          = quat_rotate(vc.qx, vc.qy, vc.qz, vc.qw, pos);
-        const V3 v          = {r.x + vc.tx, r.y + vc.ty, r.z + vc.tz};
-        if (!(v.z > 0.f)) continue;
-        const V2 np   = {v.x / v.z, v.y / v.z};
-        const V2 dp   = distort<false>(np, vc.d, 3.0e38f, nullptr, nullptr);
-        const V2 ip   = k_apply(vc.k, dp);
-        const bool in = ip.x >= 0.f && ip.y >= 0.f && ip.x < (float)vc.w && ip.y < (float)vc.h;
-        const float d = (v.x * v.x + v.y * v.y) + v.z * v.z;
-        if (in && d < best) best = d;
-    }
+    for (int f = 0; f < num_frames; ++f) nearest_camera(views[f], pos, &best);
     out[i] = sqrtf(best);
+}
+
+// The same for points in the order of the search grid: a wavefront's points lie close together, so most frames are ruled out for
+// all of them at once.  Per 64 frames, every lane takes one: a bound below the distance of its camera to any point of
+// the wavefront's bounding sphere, or none if the whole sphere lies behind the camera.  The frames then come nearest first,
+// until the next bound is above what every lane has found.  The minimum over the frames
+// that see a point does not depend on their order, and the bound leaves 1e-5 of the coordinates for rounding.
+// 3 M points of a sphere on a plane, 100 frames: 708 -> 307 us (the corners of the plane
+// are in few images, and a point no frame sees takes all of them).
+__global__ __launch_bounds__(kBlock) void camera_distance_sorted_kernel(const float4* __restrict__ sorted, int n,
+                                                                        const ViewConst* __restrict__ views, int num_frames,
+                                                                        float* __restrict__ out)
+{
+    const int t    = blockIdx.x * kBlock + threadIdx.x;
+    const int lane = threadIdx.x & 63;
+    const float4 P = sorted[t < n ? t : n - 1];
+    const V3 pos   = {P.x, P.y, P.z};
+    const float lo[3] = {wave_min(P.x), wave_min(P.y), wave_min(P.z)}, hi[3] = {wave_max(P.x), wave_max(P.y), wave_max(P.z)};
+    const V3 c     = {0.5f * (lo[0] + hi[0]), 0.5f * (lo[1] + hi[1]), 0.5f * (lo[2] + hi[2])};
+    const V3 half  = {hi[0] - lo[0], hi[1] - lo[1], hi[2] - lo[2]};
+    const float radius = 0.5f * sqrtf(dot3(half, half));
+    float best     = 105235545.f;
+    for (int f0 = 0; f0 < num_frames; f0 += 64)
+    {
+        const float never = __builtin_inff();
+        float bound       = never;
+        if (f0 + lane < num_frames)
+        {
+            const ViewConst& vc = views[f0 + lane];
+            const V3 r = quat_rotate(vc.qx, vc.qy, vc.qz, vc.qw, c);
+            const V3 v = {r.x + vc.tx, r.y + vc.ty, r.z + vc.tz};
+            const float slack = radius * 1.0001f + 1.0e-5f * (fabsf(c.x) + fabsf(c.y) + fabsf(c.z) + radius + fabsf(vc.tx) + fabsf(vc.ty) + fabsf(vc.tz));
+            const float reach = sqrtf(dot3(v, v)) - slack;
+            if (!(v.z + slack <= 0.f)) bound = reach > 0.f ? reach * reach * 0.9999f : 0.f;
+        }
+        for (;;)
+        {
+            const float next = wave_min(bound);
+            if (next == never || next >= wave_max(best)) break;  // (wavefront-uniform)
+            const int f = __ffsll((long long)__ballot(bound == next)) - 1;
+            nearest_camera(views[f0 + f], pos, &best);
+            if (lane == f) bound = never;
+        }
+    }
+    if (t < n) out[__float_as_uint(P.w)] = sqrtf(best);
 }
 
 // SceneData::RemoveClosePoints (SceneData.cpp:598-642) walks the points in order and erases point i when a point it
@@ -1025,6 +1072,13 @@ void launch_camera_distance(const float4* position, int n, const ViewConst* view
                             hipStream_t st)
 {
     hipLaunchKernelGGL(camera_distance_kernel, dim3((n + kBlock - 1) / kBlock), dim3(kBlock), 0, st, position, n, views,
+                       num_frames, out);
+}
+
+void launch_camera_distance_sorted(const float4* sorted, int n, const ViewConst* views, int num_frames, float* out,
+                                   hipStream_t st)
+{
+    hipLaunchKernelGGL(camera_distance_sorted_kernel, dim3((n + kBlock - 1) / kBlock), dim3(kBlock), 0, st, sorted, n, views,
                        num_frames, out);
 }
 

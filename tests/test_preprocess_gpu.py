@@ -334,3 +334,28 @@ def test_filter_refuses_a_cloud_it_empties():
         preprocess.FilterPointCloud(torch.from_numpy(p).cuda(), torch.from_numpy(views).cuda(), torch.from_numpy(K).cuda(),
                                     [scenes.make_view(w, h, image_index=f, camera_index=c) for w, h, f, c in fr],
                                     lonely=(5, 0.0))
+
+
+@pytest.mark.parametrize("n,frames", [(6, 1), (257, 64), (5000, 65), (40001, 150)])
+def test_camera_distance_in_grid_order_equals_the_plain_one(n, frames):
+    """The distances taken in the order of the search grid, with most frames ruled out per wavefront, are those of all frames
+    for every point, bit for bit: cameras around, far from and inside the cloud, strays, more and fewer than 64 frames."""
+    import torch
+    from adop_amd import preprocess as pp, scenes
+
+    announce(f"camera distance in grid order, N={n}, {frames} frames")
+    g = np.random.default_rng(n)
+    p = np.zeros((n, 4), np.float32)
+    p[:, :3] = g.standard_normal((n, 3)) * [1.0, 1.0, 0.1]
+    p[g.choice(n, n // 100, replace=False), :3] *= 300.0
+    poses = torch.from_numpy(np.stack([scenes.look_at_view(g.standard_normal(3) * g.choice([0.2, 2.0, 50.0]), g.standard_normal(3) * 0.3)
+                                       for _ in range(frames)])).cuda()
+    K = torch.from_numpy(np.stack([scenes.pinhole_row(300, 300, 160, 120, dist=[-0.06, 0.02, -0.003, 0, 0, 0, 4e-4, -3e-4]),
+                                   scenes.pinhole_row(200, 210, 150, 110)])).cuda()
+    fr = [scenes.make_view(320, 240, image_index=f, camera_index=f % 2) for f in range(frames)]
+    dev = torch.from_numpy(p).cuda()
+    want = pp.PointDistanceToCamera(dev, poses, K, fr)
+    ws = pp._knn_workspace(dev)
+    pp._knn_distance(dev, 4, pp._bbox(dev), ws)
+    got = pp._camera_distance(dev, poses, K, fr, ws)
+    assert torch.equal(got.view(torch.int32), want.view(torch.int32))
