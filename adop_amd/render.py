@@ -81,24 +81,15 @@ class NeuralScene:
                    environment_map=None if hs.env_texture is None else torch.from_numpy(hs.env_texture))
 
     def struct(self):
-        s = _capi.Scene()
-        pc = self.point_cloud_cuda
-        s.position = _ptr(pc.t_position)
-        s.normal = _ptr(pc.t_normal)
-        s.index = _ptr(pc.t_index)
-        s.num_points = pc.Size()
-        s.texture = _ptr(self.texture)
-        s.texture_dtype = _capi.TEXTURE_F16 if self.texture.dtype == torch.float16 else _capi.TEXTURE_F32
-        s.num_channels = int(self.texture.shape[0])
-        s.num_texels = int(self.texture.shape[1])
-        s.background_color = _ptr(self.background_color)
-        s.poses_se3 = _ptr(self.poses_se3)
-        s.num_poses = int(self.poses_se3.shape[0])
-        s.intrinsics = _ptr(self.intrinsics)
-        s.num_cameras = int(self.intrinsics.shape[0])
-        s.intrinsics_cols = int(self.intrinsics.shape[1])
-        s.index_is_identity = 1 if (pc.index_is_identity() and s.num_texels == s.num_points) else 0
-        return s
+        pc, tex = self.point_cloud_cuda, self.texture
+        n, texels = pc.Size(), tex.shape[1]
+        # (positional: one call instead of fifteen attribute assignments)
+        return _capi.Scene(pc.t_position.data_ptr(), None if pc.t_normal is None else pc.t_normal.data_ptr(),
+                           pc.t_index.data_ptr(), n, tex.data_ptr(),
+                           _capi.TEXTURE_F16 if tex.dtype == torch.float16 else _capi.TEXTURE_F32, tex.shape[0], texels,
+                           self.background_color.data_ptr(), self.poses_se3.data_ptr(), self.poses_se3.shape[0],
+                           self.intrinsics.data_ptr(), self.intrinsics.shape[0], self.intrinsics.shape[1],
+                           1 if (pc.index_is_identity() and texels == n) else 0)
 
 
 @dataclass
@@ -151,7 +142,8 @@ class PointRendererCache:
         self.output_forward = []
         self.output_forward_background_mask = []
         self.workspace = None
-        self.stats = None
+        self._workspace_key = None
+        self._stats = None
         self.info = None
         self.num_batches = 0
 
@@ -185,11 +177,26 @@ class PointRendererCache:
             w //= 2
             h //= 2
             scale *= 0.5
-        s = scene.struct()
-        nbytes = self.lib.adop_workspace_size_for(C.byref(s), B, info.num_layers, fd.w, fd.h, int(info.workspace_flags))
-        self.workspace = torch.empty(max(int(nbytes), 256), dtype=torch.uint8, device=dev)
-        self.stats = torch.zeros(C.sizeof(_capi.Stats) // 8, dtype=torch.int64, device=dev)
+        # The workspace is scratch memory: nothing in it outlives the passes queued on its stream, so it stays while
+        # they take the same amount of it on the same stream.  (A pass that is captured takes its own: the graph keeps it.)
+        stream = _raw_stream()
+        key = (new_size, dev, stream, scene.poses_se3.shape[0], tuple(scene.intrinsics.shape))
+        capturing = torch.cuda.is_current_stream_capturing()
+        if capturing or key != self._workspace_key:
+            s = scene.struct()
+            nbytes = self.lib.adop_workspace_size_for(C.byref(s), B, info.num_layers, fd.w, fd.h, int(info.workspace_flags))
+            self.workspace = None  # (given back before the next one is taken)
+            self.workspace = torch.empty(max(int(nbytes), 256), dtype=torch.uint8, device=dev)
+            self._workspace_key = None if capturing else key
+        self._stats = None
         self.cache_size = new_size
+
+    @property
+    def stats(self):
+        """Counters of the passes since the buffers were allocated (made when first asked for)."""
+        if self._stats is None:
+            self._stats = torch.zeros(C.sizeof(_capi.Stats) // 8, dtype=torch.int64, device=self.workspace.device)
+        return self._stats
 
     def InitializeData(self, forward):
         info = self.info
@@ -225,32 +232,31 @@ class PointRendererCache:
     def forward_struct(self):
         fb = _capi.ForwardBuffers()
         fb.num_layers = len(self.layers_cuda)
+        masks = self.output_forward_background_mask
         for l, L in enumerate(self.layers_cuda):
-            S = fb.layers[l]
-            S.w, S.h = L.size
-            S.depth_index = _ptr(L.depth_index_tensor)
-            S.depth = _ptr(L.depth)
-            S.weight = _ptr(L.weight)
-            S.out = _ptr(self.output_forward[l])
-            S.mask = _ptr(self.output_forward_background_mask[l]) if self.output_forward_background_mask else None
+            w, h = L.size
+            fb.layers[l] = _capi.Layer(w, h, L.depth_index_tensor.data_ptr(), L.depth.data_ptr(), L.weight.data_ptr(),
+                                       self.output_forward[l].data_ptr(), masks[l].data_ptr() if masks else None)
         fb.dropout_points = _ptr(self.dropout_points)
         fb.point_cache = _ptr(self.point_cache)
         fb.pixel_cache = _ptr(self.pixel_cache)
         return fb
 
     def views_array(self):
-        arr = (_capi.View * self.num_batches)()
-        for i, v in enumerate(self.info.images):
-            arr[i] = v
-        return arr
+        return (_capi.View * self.num_batches)(*self.info.images)
 
     def read_stats(self):
         host = self.stats.cpu().numpy().tobytes()
         return _capi.Stats.from_buffer_copy(host)
 
 
+def _raw_stream():
+    """hipStream_t of the current stream of the current device."""
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
+
+
 def _stream_ptr():
-    return C.c_void_p(torch.cuda.current_stream().cuda_stream)
+    return C.c_void_p(_raw_stream())
 
 
 def BlendPointCloudForward(ctx, info, build=True):
@@ -272,6 +278,10 @@ def BlendPointCloudForward(ctx, info, build=True):
             weight_sum += float(L.weight.sum().item())
         print(f"# Rasterized Points = {int(weight_sum)}", flush=True)
     if ctx is not None:
+        # depth / weight / packed depth now belong to the graph (the kernels write them through raw pointers, autograd
+        # would not notice a later forward overwriting them): the next forward allocates fresh ones
+        cache.cache_size = None
+    if ctx is not None and any(getattr(ctx, "needs_input_grad", (True,))):
         save = []
         for L in cache.layers_cuda:
             save += [L.depth, L.weight]
@@ -282,9 +292,6 @@ def BlendPointCloudForward(ctx, info, build=True):
         ctx.pixel_cache = cache.pixel_cache
         ctx.depth_index = [L.depth_index_tensor for L in cache.layers_cuda]
         ctx.masks = list(cache.output_forward_background_mask)
-        # depth / weight / packed depth now belong to the graph (the kernels write them through raw pointers, autograd
-        # would not notice a later forward overwriting them): the next forward allocates fresh ones
-        cache.cache_size = None
     return list(cache.output_forward), list(cache.output_forward_background_mask)
 
 
@@ -304,13 +311,10 @@ def BlendPointCloudBackward(ctx, info, image_gradients, needs=(True, True, True)
     fb = _capi.ForwardBuffers()
     fb.num_layers = L
     for l in range(L):
-        S = fb.layers[l]
-        S.w, S.h = int(saved[2 * l].shape[3]), int(saved[2 * l].shape[2])
-        S.depth = _ptr(saved[2 * l])
-        S.weight = _ptr(saved[2 * l + 1])
-        S.out = _ptr(saved[2 * L + l])
-        S.depth_index = _ptr(ctx.depth_index[l])
-        S.mask = _ptr(ctx.masks[l]) if ctx.masks else None
+        depth = saved[2 * l]
+        fb.layers[l] = _capi.Layer(depth.shape[3], depth.shape[2], ctx.depth_index[l].data_ptr(), depth.data_ptr(),
+                                   saved[2 * l + 1].data_ptr(), saved[2 * L + l].data_ptr(),
+                                   ctx.masks[l].data_ptr() if ctx.masks else None)
     fb.dropout_points = _ptr(ctx.dropout_points)
     fb.point_cache = _ptr(getattr(ctx, "point_cache", None))
     fb.pixel_cache = _ptr(getattr(ctx, "pixel_cache", None))
