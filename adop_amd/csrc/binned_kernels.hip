@@ -33,30 +33,36 @@ __device__ __forceinline__ void entry_tiles(const Levels& lv, const ParamArg& rp
                                             V2 ip, float radius_pixels, bool* in_out, bool* any_in, uint32_t* nlev,
                                             uint32_t* ptile, uint32_t* xtile)
 {
-    int px[ADOP_MAX_LAYERS], py[ADOP_MAX_LAYERS];
-    bool in[ADOP_MAX_LAYERS];
+    int px[2] = {0, 0}, py[2] = {0, 0};
+    bool in[2] = {false, false};
     bool alive = ok;
+    bool rest  = false;  // a point that only a level from 2 on can still put into the image
     *any_in    = false;
     *nlev      = 0;
 #pragma unroll
     for (int l = 0; l < ADOP_MAX_LAYERS; ++l)
     {
-        px[l] = py[l] = 0;
-        in[l]         = false;
+        bool in_l = false;
         if (l < lv.num)
         {
             if (rp.drop_by_radius && radius_pixels < rp.drop_threshold) alive = false;  // break, :261-264
             if (alive) *nlev = l + 1;
-            const LevelArg& L = lv.l[l];
-            px[l]             = f2i_rn(ip.x);
-            py[l]             = f2i_rn(ip.y);
-            in[l] = alive && (unsigned)px[l] < (unsigned)L.w && (unsigned)py[l] < (unsigned)L.h;
-            *any_in |= in[l];
+            // (levels are not nested, but nearly all points of the image are in it at level 0: the pixels of the levels from
+            // 2 on are computed only where a lane of the wavefront needs them, or all of them are counted)
+            if (l == 2) rest = in_out != nullptr || __ballot(alive && !*any_in) != 0;
+            if (l < 2 || rest)
+            {
+                const LevelArg& L = lv.l[l];
+                const int x = f2i_rn(ip.x), y = f2i_rn(ip.y);
+                in_l = alive && (unsigned)x < (unsigned)L.w && (unsigned)y < (unsigned)L.h;
+                *any_in |= in_l;
+                if (l < 2) px[l] = x, py[l] = y, in[l] = in_l;
+            }
             radius_pixels *= 0.5f;
             ip.x *= 0.5f;
             ip.y *= 0.5f;
         }
-        if (in_out) in_out[l] = in[l];
+        if (in_out) in_out[l] = in_l;
     }
     const int tiles_per_view = bin.tiles_x * bin.tiles_y;
     int cx = px[0] < 0 ? 0 : (px[0] >= lv.l[0].w ? lv.l[0].w - 1 : px[0]);
@@ -170,7 +176,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(PPT > 2 
             bool in[ADOP_MAX_LAYERS];
             bool any_in;
             uint32_t nlev, ptile, xtile;
-            entry_tiles(lv, rp, bin, b, ok, ip, radius_pixels, in, &any_in, &nlev, &ptile, &xtile);
+            entry_tiles(lv, rp, bin, b, ok, ip, radius_pixels, STATS ? in : nullptr, &any_in, &nlev, &ptile, &xtile);
             if (valid)
             {
                 uint32_t word = 0;

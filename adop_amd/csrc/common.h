@@ -388,6 +388,11 @@ __device__ __forceinline__ ViewConst make_view_const(const adop_view& v, const d
     c.npoly        = cols - 5;
     c.no_distortion = v.camera_model_type == ADOP_CAMERA_PINHOLE_DISTORTION;
     for (int i = 0; i < 8; ++i) c.no_distortion = c.no_distortion && c.d[i] == 0.f;
+    const V3 back = quat_rotate(-c.qx, -c.qy, -c.qz, c.qw, V3{c.tx, c.ty, c.tz});
+    c.cx   = -back.x;
+    c.cy   = -back.y;
+    c.cz   = -back.z;
+    c.csum = (fabsf(back.x) + fabsf(back.y)) + fabsf(back.z) + 1.0e-31f;  // (above what underflow leaves uncertain)
     return c;
 }
 

@@ -329,8 +329,8 @@ adop_status adop_point_distance_to_camera_grid(const adop_scene* scene, const ad
 
 /* adop_point_distance_to_camera without a workspace, for callers that cannot allocate device memory (code under HIP
  * graph capture, tight serving loops, harnesses that forbid hipMalloc).  No counterpart in the reference.  The
- * per-frame constants live in an array inside the library (132 bytes per frame, adop_static_max_frames() = 1024
- * frames = 132 KiB per GPU, held until the process ends); more frames are rejected with ADOP_INVALID_ARG.  The call
+ * per-frame constants live in an array inside the library (148 bytes per frame, adop_static_max_frames() = 1024
+ * frames = 148 KiB per GPU, held until the process ends); more frames are rejected with ADOP_INVALID_ARG.  The call
  * allocates and frees nothing; the first call on a device looks the array's address up (make that call outside a
  * stream capture).  All calls on one GPU share the array: calls that overlap on one GPU (different streams or
  * threads) race; calls on one stream are ordered and safe.  Results equal adop_point_distance_to_camera's. */

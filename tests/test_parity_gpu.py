@@ -784,6 +784,40 @@ def test_every_tuning_variant_gives_the_same_results(oracle_mod, variant, forwar
             _fwd_bwd(scene, oracle_mod, collect_stats=False, poison=True)
 
 
+@pytest.mark.parametrize("model", ["pinhole", "ocam"])
+@pytest.mark.parametrize("scale", [1.0, 1e-9, 1e6])
+def test_back_face_test_at_grazing_angles(oracle_mod, model, scale):
+    """Normals nearly perpendicular to the line of sight: the kernels take the sign of the back-face test in world
+    coordinates where it is beyond doubt and evaluate the reference's form elsewhere.  Whatever the size of the scene, the
+    points culled are the checker's: packed depth and weights bit for bit."""
+    from adop_amd import scenes
+
+    announce(f"back faces at grazing angles, {model}, scene scaled by {scale}")
+    if model == "pinhole":
+        hs = scenes.config1(n=20_000, w=160, h=120)
+    else:
+        hs = scenes.config5(n=20_000, w=200, h=150, batch=1, patches=20, env_hw=(16, 32))
+    hs.params.check_normal = 1
+    g = np.random.default_rng(17)
+    xyz = g.uniform(-1.0, 1.0, (20_000, 3))
+    camera = np.array([0.3, 0.5, -3.0])
+    line = xyz - camera
+    line /= np.linalg.norm(line, axis=1, keepdims=True)
+    nrm = np.cross(line, g.standard_normal(line.shape))
+    nrm /= np.linalg.norm(nrm, axis=1, keepdims=True)
+    nrm += line * 10.0 ** g.uniform(-8, -1, (len(nrm), 1)) * g.choice([-1.0, 1.0], (len(nrm), 1))
+    nrm /= np.linalg.norm(nrm, axis=1, keepdims=True)
+    hs.position = hs.position[:20_000].copy()
+    hs.position[:, :3] = (xyz * scale).astype(np.float32)
+    hs.normal = scenes.pack_normals(nrm.astype(np.float32))
+    hs.poses_se3 = np.stack([scenes.look_at_view(camera)] * len(hs.poses_se3))
+    hs.poses_se3[:, 4:7] *= scale
+    ref = oracle_mod.forward(hs)
+    _, info, ctx, images, masks = run_hip_forward(hs)
+    check_forward(hs, ref, ctx, images, masks, info)
+    assert 0.2 < ref.stats.visible[0] / 20_000 < 0.8  # about half of them face the camera
+
+
 def test_zz_report_end_to_end_misses():
     """Prints what the end-to-end element-wise check of every case above found (the asserts are in _fwd_bwd)."""
     for case, rec in end_to_end_misses.items():
