@@ -164,7 +164,7 @@ __device__ __forceinline__ void load_channels(const float* __restrict__ src, flo
 //
 // backward_ghost_kernel — one thread per queue item, all lanes busy: the four-neighbour gather from the
 // pixel-major [I|G] array, the approximate image-space gradient (:491-611) and ProjectPoint*Backward.
-template <int CT, bool HALF, bool MULTI>
+template <int CT, bool HALF, bool MULTI, bool STATS>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(CT != 0 ? 8 : 4, 8))) void backward_tex_kernel(CloudArg pc, const ViewConst* __restrict__ views,
                                                                Levels lv, ParamArg rp, const float* __restrict__ ig,
                                                                const float2* __restrict__ dw,
@@ -181,7 +181,6 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(CT != 0 
     __shared__ unsigned long long s_culled[kBlock / 64];
     __shared__ unsigned long long s_block_culled;
     static_assert(kBlock / 64 == 4, "four runs per workgroup");
-    const bool STATS    = stats != nullptr;  // counter pass (uniform branch)
     const float accept  = rp.depth_accept + 1;
     const int C         = CT ? CT : lv.C;
     const int lane      = threadIdx.x & 63;
@@ -1239,14 +1238,22 @@ static void launch_bwd_tex_t(const CloudArg& pc, const ViewConst* views, const L
                              const QueueArg& q, adop_stats* stats, hipStream_t st)
 {
     int grid = (pc.n + kBlock - 1) / kBlock;
+#define ADOP_TEX(MULTI, STATS)                                                                                             \
+    hipLaunchKernelGGL((backward_tex_kernel<CT, HALF, MULTI, STATS>), dim3(grid), dim3(kBlock), 0, st, pc, views, lv, rp, ig, dw, \
+                       g->grad_texture, g->grad_points, g->grad_points_count, identity_index, q.counts, q.items, q.cap,     \
+                       MULTI ? q.concurrent : 0, stats)
     if (lv.B > 1)
-        hipLaunchKernelGGL((backward_tex_kernel<CT, HALF, true>), dim3(grid), dim3(kBlock), 0, st, pc, views, lv, rp, ig,
-                           dw, g->grad_texture, g->grad_points, g->grad_points_count, identity_index, q.counts, q.items,
-                           q.cap, q.concurrent, stats);
+    {
+        if (stats)
+            ADOP_TEX(true, true);
+        else
+            ADOP_TEX(true, false);
+    }
+    else if (stats)
+        ADOP_TEX(false, true);
     else
-        hipLaunchKernelGGL((backward_tex_kernel<CT, HALF, false>), dim3(grid), dim3(kBlock), 0, st, pc, views, lv, rp, ig,
-                           dw, g->grad_texture, g->grad_points, g->grad_points_count, identity_index, q.counts, q.items,
-                           q.cap, 0, stats);
+        ADOP_TEX(false, false);
+#undef ADOP_TEX
 }
 
 template <int CT, bool HALF>

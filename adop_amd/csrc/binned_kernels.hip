@@ -83,11 +83,16 @@ __device__ __forceinline__ uint32_t shard_of(uint32_t point, int shard_shift)
 
 // First pass over the points: projection (kept in the point cache) and the number of entries per tile.  A thread
 // handles PPT points whose loads are all issued before anything waits.
-template <int PPT>
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(PPT > 2 ? 5 : 8, PPT > 2 ? 5 : 8))) void bin_count_kernel(CloudArg pc, const ViewConst* __restrict__ views, Levels lv,
+// Scalar registers decide the number of its instructions: what does not fit them is parked in lanes of vector registers, one
+// v_writelane / v_readlane per value, and they count against the vector issue this kernel is bound by.  Hence the counter
+// pass as a variant of its own, the projections of all points before the first of them is binned (the view's constants are
+// done with then) and up to 96 scalar registers, which 8 wavefronts per SIMD allow (the compiler stops at 80 when it is asked for 8
+// wavefronts): 1462 vector and 1132 scalar instructions, 197 of them parking, become 1215, 773 and 44.  16 crops of
+// 10 M points: 356 -> 305 us; one view of 12 M: 85 -> 80 us.
+template <int PPT, bool STATS>
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(PPT > 2 ? 5 : 7, PPT > 2 ? 5 : 8), amdgpu_num_sgpr(96))) void bin_count_kernel(CloudArg pc, const ViewConst* __restrict__ views, Levels lv,
                                                            ParamArg rp, BinArg bin, adop_stats* stats)
 {
-    const bool STATS = stats != nullptr;  // counter pass (uniform branch)
     const int lane   = threadIdx.x & 63;
     const int base   = blockIdx.x * (kBlock * PPT) + threadIdx.x;
 
@@ -119,6 +124,21 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(PPT > 2 
         const ViewConst& vc = views[b];
         const bool same_frame = b > 0 && vc.image_index == views[b - 1].image_index &&
                                 vc.camera_index == views[b - 1].camera_index && vc.model == views[b - 1].model;  // uniform
+        if (!same_frame)
+        {
+#pragma unroll
+            for (int k = 0; k < PPT; ++k)
+            {
+                V3 pos = {P[k].x, P[k].y, P[k].z};
+                V3 nrm = unpack_normal10(nenc[k]);
+                V3 view_p;
+                frame_p[k] = {0.f, 0.f};
+                frame_z[k] = 0.f;
+                if (base + k * kBlock < pc.n)
+                    project_frame(vc, pc.intrinsics, pos, nrm, rp.check_normal != 0, rp.dist_cutoff, &frame_p[k], &frame_z[k],
+                                  &view_p);
+            }
+        }
 #pragma unroll
         for (int k = 0; k < PPT; ++k)
         {
@@ -126,17 +146,6 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(PPT > 2 
             const bool valid = i < pc.n;
             V2 ip            = {0.f, 0.f};
             float radius_pixels = 0.f;
-            if (!same_frame)
-            {
-                V3 pos = {P[k].x, P[k].y, P[k].z};
-                V3 nrm = unpack_normal10(nenc[k]);
-                V3 view_p;
-                frame_p[k] = {0.f, 0.f};
-                frame_z[k] = 0.f;
-                if (valid)
-                    project_frame(vc, pc.intrinsics, pos, nrm, rp.check_normal != 0, rp.dist_cutoff, &frame_p[k], &frame_z[k],
-                                  &view_p);
-            }
             const float z = frame_z[k];
             const bool ok = z != 0;
             if (ok) ip = k_apply(vc.crop, frame_p[k]);
@@ -513,15 +522,26 @@ void launch_bin(int pass, const CloudArg& pc, const ViewConst* views, const Leve
         // (one point per thread while the grid is small: twice the workgroups in flight; config 2 0.038 -> 0.033 ms,
         // 10 M points 0.079 against 0.082 ms the other way round)
         const int cppt = tn.count_ppt ? tn.count_ppt : (pc.n <= (1 << 22) ? 1 : 2);
+#define ADOP_BIN_COUNT(PPT)                                                                                              \
+    if (stats)                                                                                                            \
+        hipLaunchKernelGGL((bin_count_kernel<PPT, true>), dim3((pc.n + kBlock * PPT - 1) / (kBlock * PPT)), dim3(kBlock), 0, \
+                           st, pc, views, lv, rp, bin, stats);                                                            \
+    else                                                                                                                  \
+        hipLaunchKernelGGL((bin_count_kernel<PPT, false>), dim3((pc.n + kBlock * PPT - 1) / (kBlock * PPT)), dim3(kBlock), 0, \
+                           st, pc, views, lv, rp, bin, stats);
         if (cppt == 2)
-            hipLaunchKernelGGL((bin_count_kernel<2>), dim3((pc.n + kBlock * 2 - 1) / (kBlock * 2)), dim3(kBlock), 0, st,
-                               pc, views, lv, rp, bin, stats);
+        {
+            ADOP_BIN_COUNT(2)
+        }
         else if (cppt == 4)
-            hipLaunchKernelGGL((bin_count_kernel<4>), dim3((pc.n + kBlock * 4 - 1) / (kBlock * 4)), dim3(kBlock), 0, st,
-                               pc, views, lv, rp, bin, stats);
+        {
+            ADOP_BIN_COUNT(4)
+        }
         else
-            hipLaunchKernelGGL((bin_count_kernel<1>), dim3((pc.n + kBlock - 1) / kBlock), dim3(kBlock), 0, st, pc, views,
-                               lv, rp, bin, stats);
+        {
+            ADOP_BIN_COUNT(1)
+        }
+#undef ADOP_BIN_COUNT
         return;
     }
     const int T = bin.tiles_x * bin.tiles_y * lv.B;

@@ -72,7 +72,7 @@ __global__ __launch_bounds__(kBlock) void clear_kernel(Levels lv, int first_leve
 // pixel, one lane per distinct pixel takes the minimum of its group from LDS and issues the 64-bit atomicMin:
 // clouds stored in Morton-ordered blocks collide heavily at the coarse levels, and a device-scope atomic costs one
 // memory transaction whatever it carries.
-template <int PPT>
+template <int PPT, bool STATS>
 __global__ __launch_bounds__(kBlock) void prepass_kernel(CloudArg pc, const ViewConst* __restrict__ views, Levels lv,
                                                          ParamArg rp, int group_from, adop_stats* stats, Gate gate)
 {
@@ -80,7 +80,6 @@ __global__ __launch_bounds__(kBlock) void prepass_kernel(CloudArg pc, const View
     if (gate_closed(gate)) return;
     __shared__ unsigned long long s_gmask[kBlock];
     __shared__ uint32_t s_gkey[kBlock];
-    const bool STATS = stats != nullptr;  // counter pass (uniform branch)
     const int lane   = threadIdx.x & 63;
     const int wbase  = threadIdx.x & ~63;
     unsigned long long* pk_w    = s_pk + wbase;
@@ -280,7 +279,7 @@ __global__ __launch_bounds__(kBlock) void prepass_kernel(CloudArg pc, const View
 // accum: S floats per workspace pixel (C sums + weight, padded to a power of two).
 // Per level every wavefront groups its accepted lanes by pixel; LG = max(S,8) consecutive lanes then sum the
 // staged descriptors of one group (lane j = channel j, lane C = the count) and add them with ONE cache-line atomic.
-template <int CT, bool HALF>
+template <int CT, bool HALF, bool STATS>
 __global__ __launch_bounds__(kBlock) void blend_kernel(CloudArg pc, const ViewConst* __restrict__ views, Levels lv,
                                                        ParamArg rp, float* __restrict__ accum, int S,
                                                        adop_stats* stats, int group_from, Gate gate)
@@ -290,7 +289,6 @@ __global__ __launch_bounds__(kBlock) void blend_kernel(CloudArg pc, const ViewCo
     __shared__ uint32_t s_gkey[kBlock];
     extern __shared__ float s_stage[];  // kBlock * C descriptors of the block's points
     if (gate_closed(gate)) return;
-    const bool STATS = stats != nullptr;  // counter pass (uniform branch)
     const int C      = CT ? CT : lv.C;
     const int lane   = threadIdx.x & 63;
     const int wbase  = threadIdx.x & ~63;
@@ -612,15 +610,25 @@ void launch_prepass(const CloudArg& pc, const ViewConst* views, const Levels& lv
     if (pc.n < 1) return;
     const int group_from = tn.prepass_group_from;
     const int ppt        = prepass_ppt(pc.n, tn.prepass_ppt);
+    const dim3 grid((pc.n + kBlock * ppt - 1) / (kBlock * ppt));
+#define ADOP_PREPASS(PPT)                                                                                               \
+    if (stats)                                                                                                           \
+        hipLaunchKernelGGL((prepass_kernel<PPT, true>), grid, dim3(kBlock), 0, st, pc, views, lv, rp, group_from, stats, gate); \
+    else                                                                                                                 \
+        hipLaunchKernelGGL((prepass_kernel<PPT, false>), grid, dim3(kBlock), 0, st, pc, views, lv, rp, group_from, stats, gate);
     if (ppt == 4)
-        hipLaunchKernelGGL((prepass_kernel<4>), dim3((pc.n + kBlock * 4 - 1) / (kBlock * 4)), dim3(kBlock), 0, st, pc,
-                           views, lv, rp, group_from, stats, gate);
+    {
+        ADOP_PREPASS(4)
+    }
     else if (ppt == 2)
-        hipLaunchKernelGGL((prepass_kernel<2>), dim3((pc.n + kBlock * 2 - 1) / (kBlock * 2)), dim3(kBlock), 0, st, pc,
-                           views, lv, rp, group_from, stats, gate);
+    {
+        ADOP_PREPASS(2)
+    }
     else
-        hipLaunchKernelGGL((prepass_kernel<1>), dim3((pc.n + kBlock - 1) / kBlock), dim3(kBlock), 0, st, pc, views, lv,
-                           rp, group_from, stats, gate);
+    {
+        ADOP_PREPASS(1)
+    }
+#undef ADOP_PREPASS
 }
 
 template <int CT, bool HALF>
@@ -634,8 +642,12 @@ static void launch_blend_t(const CloudArg& pc, const ViewConst* views, const Lev
                                   : kBlock;
     const int grid  = pc.list_ids ? (pc.n + pc.list_span - 1) / pc.list_span : (pc.n + kBlock - 1) / kBlock;
     size_t lds      = sizeof(float) * (size_t)block * (size_t)lv.C;
-    hipLaunchKernelGGL((blend_kernel<CT, HALF>), dim3(grid), dim3(block), lds, st, pc, views, lv, rp,
-                       accum, S, stats, group_from, gate);
+    if (stats)
+        hipLaunchKernelGGL((blend_kernel<CT, HALF, true>), dim3(grid), dim3(block), lds, st, pc, views, lv, rp, accum, S, stats,
+                           group_from, gate);
+    else
+        hipLaunchKernelGGL((blend_kernel<CT, HALF, false>), dim3(grid), dim3(block), lds, st, pc, views, lv, rp, accum, S, stats,
+                           group_from, gate);
 }
 
 void launch_blend(const CloudArg& pc, const ViewConst* views, const Levels& lv, const ParamArg& rp, bool half,

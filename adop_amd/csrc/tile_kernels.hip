@@ -269,9 +269,11 @@ __device__ __forceinline__ void add_staged(float* acc, const float* s_stage, int
     }
 }
 
-// K entries per thread and batch (BATCH = K * kBlock, a power of two).
-template <int CT, bool HALF, int K>
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu((CT != 0 && K == 1) ? 8 : 4, 8))) void tile_blend_kernel(CloudArg pc, Levels lv, ParamArg rp, BinArg bin,
+// K entries per thread and batch (BATCH = K * kBlock, a power of two).  LT as a constant and the counter pass as a variant: the
+// tile's windows took 111 scalar registers more than there are (see bin_count_kernel), now 13; 1071 -> 768 vector
+// instructions for 4 channels (a frame of 12 M points 73 -> 71 us: the kernel waits for its gathers of descriptors).
+template <int CT, bool HALF, int K, int LT, bool STATS>
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu((CT != 0 && K == 1) ? 7 : 4, 8), amdgpu_num_sgpr(96))) void tile_blend_kernel(CloudArg pc, Levels lv, ParamArg rp, BinArg bin,
                                                             float* __restrict__ accum, int S,
                                                             const float* __restrict__ background, int write_mask,
                                                             float mask_value, int identity_index, adop_stats* stats, int num_tiles)
@@ -282,7 +284,6 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu((CT != 0
     constexpr int TY    = 1 << kTileShiftY;
     extern __shared__ __align__(16) unsigned char smem[];
     if (bin.overflow && *bin.overflow) return;  // the bins of this workspace were too small for the call
-    const bool STATS = stats != nullptr;
     const int C      = CT ? CT : lv.C;
     const int tid    = threadIdx.x;
 
@@ -302,7 +303,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu((CT != 0
     const int tx             = tr - ty * bin.tiles_x;
     const uint32_t start     = mine.y;
     const uint32_t end       = mine.z;
-    const int lt             = bin.lt;
+    constexpr int lt         = LT;  // (= bin.lt: the extents of the tile's windows are constants, as in tile_depth_kernel)
     const TileLayout T       = tile_layout(lv, tx, ty, lt, lv.num);
     const int npix           = T.base[ADOP_MAX_LAYERS];
     const int first_coarse   = lt > 1 ? TX * TY + TX * TY / 4 : TX * TY;  // local pixel index of the first coarse pixel
@@ -705,7 +706,7 @@ static size_t tile_blend_lds(const Levels& lv, const BinArg& bin, int S)
     return stage + rest > flush ? stage + rest : flush;
 }
 
-template <int CT, bool HALF, int K>
+template <int CT, bool HALF, int K, int LT, bool STATS>
 static hipError_t launch_tile_blend_k(const CloudArg& pc, const Levels& lv, const ParamArg& rp, const BinArg& bin,
                                       int num_tiles, float* accum, int S, const float* background, int write_mask,
                                       float mask_value, int identity_index, adop_stats* stats, hipStream_t st)
@@ -715,29 +716,29 @@ static hipError_t launch_tile_blend_k(const CloudArg& pc, const Levels& lv, cons
     static size_t allowed = 0;  // largest dynamic LDS size this instantiation has been enabled for
     if (lds > 65536 && lds > allowed)
     {
-        hipError_t e = hipFuncSetAttribute((const void*)tile_blend_kernel<CT, HALF, K>,
+        hipError_t e = hipFuncSetAttribute((const void*)tile_blend_kernel<CT, HALF, K, LT, STATS>,
                                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
         if (e != hipSuccess) return e;
         allowed = lds;
     }
-    hipLaunchKernelGGL((tile_blend_kernel<CT, HALF, K>), dim3(num_tiles + bin.max_rows), dim3(kBlock), lds, st, pc, lv, rp, bin,
+    hipLaunchKernelGGL((tile_blend_kernel<CT, HALF, K, LT, STATS>), dim3(num_tiles + bin.max_rows), dim3(kBlock), lds, st, pc, lv, rp, bin,
                        accum, S, background, write_mask, mask_value, identity_index, stats, num_tiles);
     return hipSuccess;
 }
 
-template <int CT, bool HALF>
+template <int CT, bool HALF, int LT>
 static hipError_t launch_tile_blend_t(const CloudArg& pc, const Levels& lv, const ParamArg& rp, const BinArg& bin,
                                       int num_tiles, float* accum, int S, const float* background, int write_mask,
                                       float mask_value, int identity_index, adop_stats* stats, int k, hipStream_t st)
 {
-    if (k == 1)
-        return launch_tile_blend_k<CT, HALF, 1>(pc, lv, rp, bin, num_tiles, accum, S, background, write_mask, mask_value,
-                                                identity_index, stats, st);
-    if (k == 4)
-        return launch_tile_blend_k<CT, HALF, 4>(pc, lv, rp, bin, num_tiles, accum, S, background, write_mask, mask_value,
-                                                identity_index, stats, st);
-    return launch_tile_blend_k<CT, HALF, 2>(pc, lv, rp, bin, num_tiles, accum, S, background, write_mask, mask_value,
-                                            identity_index, stats, st);
+#define ADOP_TILE_K(K, STATS)                                                                                            \
+    launch_tile_blend_k<CT, HALF, K, LT, STATS>(pc, lv, rp, bin, num_tiles, accum, S, background, write_mask, mask_value, \
+                                                identity_index, stats, st)
+    if (stats) return ADOP_TILE_K(1, true);  // (a counter pass: one variant)
+    if (k == 1) return ADOP_TILE_K(1, false);
+    if (k == 4) return ADOP_TILE_K(4, false);
+    return ADOP_TILE_K(2, false);
+#undef ADOP_TILE_K
 }
 
 hipError_t launch_tile_blend(const CloudArg& pc, const Levels& lv, const ParamArg& rp, const BinArg& bin, int num_tiles,
@@ -745,8 +746,11 @@ hipError_t launch_tile_blend(const CloudArg& pc, const Levels& lv, const ParamAr
                              float mask_value, int identity_index, adop_stats* stats, const adop_tuning& tn,
                              hipStream_t st)
 {
-#define ADOP_TILE(CT, H) \
-    launch_tile_blend_t<CT, H>(pc, lv, rp, bin, num_tiles, accum, S, background, write_mask, mask_value, identity_index, stats, tn.tile_k, st)
+#define ADOP_TILE(CT, H)                                                                                                 \
+    (bin.lt == 1 ? launch_tile_blend_t<CT, H, 1>(pc, lv, rp, bin, num_tiles, accum, S, background, write_mask, mask_value, \
+                                                 identity_index, stats, tn.tile_k, st)                                   \
+                 : launch_tile_blend_t<CT, H, 2>(pc, lv, rp, bin, num_tiles, accum, S, background, write_mask, mask_value, \
+                                                 identity_index, stats, tn.tile_k, st))
     if (lv.C == 8) return half ? ADOP_TILE(8, true) : ADOP_TILE(8, false);
     if (lv.C == 4) return half ? ADOP_TILE(4, true) : ADOP_TILE(4, false);
     return half ? ADOP_TILE(0, true) : ADOP_TILE(0, false);
