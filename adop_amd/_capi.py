@@ -177,6 +177,11 @@ ENTRY_POINTS = {
         C.c_int,
         [C.c_void_p, C.c_int32, C.POINTER(C.c_float), C.POINTER(C.c_float), C.c_void_p, C.c_void_p],
     ),
+    "adop_morton_keys": (
+        C.c_int,
+        [C.c_void_p, C.c_int32, C.POINTER(C.c_float), C.POINTER(C.c_float), C.c_void_p, C.c_void_p, C.c_void_p],
+    ),
+    "adop_morton_ties": (C.c_int, [C.c_void_p, C.c_void_p, C.c_void_p, C.c_int32, C.c_void_p, C.c_void_p]),
     "adop_frames_workspace_size": (C.c_size_t, [C.c_int32]),
     "adop_point_distance_to_camera": (
         C.c_int,

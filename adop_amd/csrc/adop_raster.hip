@@ -1227,10 +1227,9 @@ adop_status adop_point_distance_to_camera_static(const adop_scene* scene, const 
     return camera_distance_run(scene, frames, num_frames, out_distance, (ViewConst*)dviews, (hipStream_t)hip_stream);
 }
 
-adop_status adop_morton_codes(const float* position, int32_t num_points, const float* bbox_min, const float* bbox_max,
-                              uint64_t* out_codes, void* hip_stream)
+static adop_status morton_run(const float* position, int32_t num_points, const float* bbox_min, const float* bbox_max,
+                              uint64_t* out_codes, int32_t* out_keys, hipStream_t stream)
 {
-    if (!position || !bbox_min || !bbox_max || !out_codes || num_points < 0) return fail(ADOP_INVALID_ARG, "null argument");
     if (num_points == 0) return ADOP_OK;
     float scale[3];
     for (int k = 0; k < 3; ++k)
@@ -1239,8 +1238,34 @@ adop_status adop_morton_codes(const float* position, int32_t num_points, const f
         if (!(ext >= 0) || !(ext < 1.0e30f)) return fail(ADOP_INVALID_ARG, "bounding box is not finite");
         scale[k] = ext > 0 ? 2097151.f / ext : 0.f;
     }
-    launch_morton((const float4*)position, num_points, bbox_min, scale, (unsigned long long*)out_codes,
-                  (hipStream_t)hip_stream);
+    launch_morton((const float4*)position, num_points, bbox_min, scale, (unsigned long long*)out_codes, out_keys, stream);
+    ADOP_HIP_CHECK(hipGetLastError());
+    return ADOP_OK;
+}
+
+adop_status adop_morton_codes(const float* position, int32_t num_points, const float* bbox_min, const float* bbox_max,
+                              uint64_t* out_codes, void* hip_stream)
+{
+    if (!position || !bbox_min || !bbox_max || !out_codes || num_points < 0) return fail(ADOP_INVALID_ARG, "null argument");
+    return morton_run(position, num_points, bbox_min, bbox_max, out_codes, nullptr, (hipStream_t)hip_stream);
+}
+
+adop_status adop_morton_keys(const float* position, int32_t num_points, const float* bbox_min, const float* bbox_max,
+                             uint64_t* out_codes, int32_t* out_keys, void* hip_stream)
+{
+    if (!position || !bbox_min || !bbox_max || !out_codes || !out_keys || num_points < 0)
+        return fail(ADOP_INVALID_ARG, "null argument");
+    return morton_run(position, num_points, bbox_min, bbox_max, out_codes, out_keys, (hipStream_t)hip_stream);
+}
+
+adop_status adop_morton_ties(const int32_t* sorted_keys, int64_t* order, const uint64_t* codes, int32_t num_points,
+                             int32_t* too_long, void* hip_stream)
+{
+    if (!sorted_keys || !order || !codes || !too_long || num_points < 0) return fail(ADOP_INVALID_ARG, "null argument");
+    adop_status st = fill_async(too_long, sizeof(int32_t), 0, (hipStream_t)hip_stream);
+    if (st != ADOP_OK || num_points == 0) return st;
+    launch_morton_ties(sorted_keys, (long long*)order, (const unsigned long long*)codes, num_points, too_long,
+                       (hipStream_t)hip_stream);
     ADOP_HIP_CHECK(hipGetLastError());
     return ADOP_OK;
 }

@@ -67,8 +67,10 @@ void launch_shuffle_gather(const float4* position, const int32_t* normal, const 
 void launch_radius_blocks(const float4* position, const int32_t* normal, const int32_t* id, const float* distance,
                           const double* uniform, int n, float4* out_position, int32_t* out_normal, float4* out_data,
                           long long* out_order, hipStream_t st);
-void launch_morton(const float4* position, int n, const float* mn, const float* scale, unsigned long long* code,
+void launch_morton(const float4* position, int n, const float* mn, const float* scale, unsigned long long* code, int32_t* key,
                    hipStream_t st);
+void launch_morton_ties(const int32_t* sorted_key, long long* order, const unsigned long long* code, int n, int32_t* too_long,
+                        hipStream_t st);
 // The launchers take the tuning switches of the call as an argument (one snapshot per call: adop_forward / adop_backward).
 // points per workgroup of prepass_kernel on a cloud of n points (the unit of its candidate lists)
 int prepass_points_per_block(int n, int tuned_ppt);

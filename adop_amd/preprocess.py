@@ -56,6 +56,27 @@ def _morton_codes(position, box):
     return codes
 
 
+# Below this many points the sort of whole codes takes no longer than the shorter one and the look at its flag.
+_KEY_SORT_FROM = 1 << 20
+
+
+def _morton_order(position, box, key_sort_from=_KEY_SORT_FROM):
+    """Stable order of the points along the Morton curve, as a function that returns it (the host waits in it for the flag
+    of adop_morton_ties: what it can do beforehand, it does before)."""
+    n = int(position.shape[0])
+    if n < key_sort_from:
+        order = torch.sort(_morton_codes(position, box), stable=True).indices
+        return lambda: order
+    lib = _capi.load_library()
+    codes = torch.empty(n, dtype=torch.int64, device=position.device)
+    keys = torch.empty(n, dtype=torch.int32, device=position.device)
+    _check(lib.adop_morton_keys(_ptr(position), n, *box, _ptr(codes), _ptr(keys), _stream_ptr()), lib)
+    keys, order = torch.sort(keys, stable=True)
+    too_long = torch.empty(1, dtype=torch.int32, device=position.device)
+    _check(lib.adop_morton_ties(_ptr(keys), _ptr(order), _ptr(codes), n, _ptr(too_long), _stream_ptr()), lib)
+    return lambda: torch.sort(codes, stable=True).indices if int(too_long.item()) else order
+
+
 def _gather_points(position, index):
     """position[index] for rows of 4 floats (torch's own gather takes ten times as long, and its rows come back wrong
     from 2^26 on)."""
@@ -225,8 +246,9 @@ def PreprocessPointCloud(position, normal=None, rank=4, block_size=256, seed=0):
     shape = None if normal is None else normal.shape
     normal = None if normal is None else normal.contiguous()
     box = _bbox(position)
-    order = torch.sort(_morton_codes(position, box), stable=True).indices
+    order = _morton_order(position, box)
     blocks = torch.randperm(n // block_size, generator=gen, device="cpu").to(position.device)
+    order = order()
     shuffled, ids = torch.empty_like(position), torch.empty(n, dtype=torch.int32, device=position.device)
     shuffled_normal = None if normal is None else torch.empty_like(normal)
     _check(lib.adop_shuffle_points(_ptr(position), _ptr(normal), _ptr(order), _ptr(blocks), n, block_size, _ptr(shuffled),

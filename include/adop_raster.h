@@ -355,6 +355,15 @@ adop_status adop_close_points(const float* position, int32_t num_points, const f
 adop_status adop_morton_codes(const float* position, int32_t num_points, const float* bbox_min, const float* bbox_max,
                               uint64_t* out_codes, void* hip_stream);
 
+/* The same order from a sort of 32 bits.  adop_morton_keys: the codes, and their upper 32 bits as a signed number of the same
+ * order; after a stable sort of the keys (sorted_keys, and in `order` the point of every key; all N >= 0) adop_morton_ties puts the
+ * points of equal keys in the order of their whole codes.  *too_long (device) = 1: more than 32 points share a key, and they
+ * are left as they were; the caller sorts by whole codes then (a cloud with far outliers leaves the others few keys). */
+adop_status adop_morton_keys(const float* position, int32_t num_points, const float* bbox_min, const float* bbox_max,
+                             uint64_t* out_codes, int32_t* out_keys, void* hip_stream);
+adop_status adop_morton_ties(const int32_t* sorted_keys, int64_t* order, const uint64_t* codes, int32_t num_points,
+                             int32_t* too_long, void* hip_stream);
+
 /* The passes of SceneData's initial processing (SceneData.cpp:101-104) that move the cloud.
  * adop_bounding_box: box [adop_bounding_box_size() bytes, device] starts with min x, y, z, max x, y, z (not a number on an
  * axis where a coordinate is not), scratch behind them.

@@ -359,3 +359,29 @@ def test_camera_distance_in_grid_order_equals_the_plain_one(n, frames):
     pp._knn_distance(dev, 4, pp._bbox(dev), ws)
     got = pp._camera_distance(dev, poses, K, fr, ws)
     assert torch.equal(got.view(torch.int32), want.view(torch.int32))
+
+
+@pytest.mark.parametrize("kind", ["volume", "surface", "duplicates", "outlier", "coincident"])
+@pytest.mark.parametrize("n", [1, 2, 33, 70_001])
+def test_morton_order_from_short_keys(kind, n):
+    """The order by the upper 32 bits with the ties put right equals the stable order by whole codes: runs of equal keys
+    shorter and longer than the kernel sorts (an outlier leaves all others one key), equal codes in their old order."""
+    import torch
+    from adop_amd import preprocess as pp
+
+    announce(f"Morton order from short keys, {kind}, N={n}")
+    g = np.random.default_rng(n)
+    p = np.zeros((n, 4), np.float32)
+    p[:, :3] = g.random((n, 3))
+    if kind == "surface":
+        p[:, 2] = 0.5
+    if kind == "duplicates":  # every point 1 to 32 times
+        p = np.repeat(p, g.integers(1, 33, n), axis=0)[g.permutation(n)][:n]
+    if kind == "outlier":
+        p[n // 2, :3] = 1e5
+    if kind == "coincident":
+        p[:, :3] = 0.25
+    dev = torch.from_numpy(np.ascontiguousarray(p)).cuda()
+    box = pp._bbox(dev)
+    want = torch.sort(pp._morton_codes(dev, box), stable=True).indices
+    assert torch.equal(pp._morton_order(dev, box, key_sort_from=1)(), want)
