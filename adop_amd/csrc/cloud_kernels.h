@@ -1,7 +1,8 @@
-// cloud_kernels.hip — moving whole clouds: bounding box, permutations of the points, radii and order of the 256-point
+// cloud_kernels.h — (part of preprocess_kernels.hip) moving whole clouds: bounding box, permutations of the points, radii and order of the 256-point
 // blocks (gfx950).  The counterpart of the loops of SceneData.cpp:101-104 and :441-484, 671-684 that touch every point
 // once; what they compute per point is next to nothing, so these kernels are bound by memory: random 64-byte lines where
 // they gather, the bandwidth of a copy where they do not.
+#pragma once
 #include "common.h"
 #include "launch.h"
 

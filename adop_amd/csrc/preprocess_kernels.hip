@@ -13,6 +13,7 @@
 // So the search grid is sized on the device (no host round trip) from the neighbour distances of 1024 sample points,
 // measured in a part of the cloud (every 16th point) on a coarse grid sized by volume.  The coarse grid over the whole cloud is
 // built only when the search grid leaves points undecided (sparse parts of the cloud), which the device finds out.
+#include "cloud_kernels.h"
 #include "common.h"
 #include "launch.h"
 
