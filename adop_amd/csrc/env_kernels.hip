@@ -34,15 +34,31 @@ __device__ __forceinline__ V2 undistort_simple(V2 p, const float* D)
     return {x, y};
 }
 
-// BuildSphericalUV + SphericalCoordinates for pixel (gx,gy) of a level whose crop is scaled by `sc`.
-__device__ __forceinline__ V2 spherical_uv(const ViewConst& vc, const float* __restrict__ intrinsics, float sc, int gx,
-                                           int gy)
+// What BuildSphericalUV needs of a view and level: the same for all pixels of a workgroup, which computes it once.
+struct EnvView
 {
-    float cr[5] = {vc.crop[0] * sc, vc.crop[1] * sc, vc.crop[2] * sc, vc.crop[3] * sc, vc.crop[4] * sc};
-    V3 t    = {vc.tx, vc.ty, vc.tz};
-    V3 rt   = quat_rotate(-vc.qx, -vc.qy, -vc.qz, vc.qw, t);
-    V3 tinv = {-rt.x, -rt.y, -rt.z};
-    V2 ip   = {(float)gx, (float)gy};
+    ViewConst vc;
+    V3 tinv;      // camera centre
+    float cr[5];  // crop transform of the level
+};
+
+__device__ __forceinline__ void set_env_view(EnvView* v, const ViewConst& vc, int level)
+{
+    float sc = 1;
+    for (int k = 0; k < level; ++k) sc /= 2;
+    const V3 rt = quat_rotate(-vc.qx, -vc.qy, -vc.qz, vc.qw, V3{vc.tx, vc.ty, vc.tz});
+    v->vc       = vc;
+    v->tinv     = {-rt.x, -rt.y, -rt.z};
+    for (int k = 0; k < 5; ++k) v->cr[k] = vc.crop[k] * sc;
+}
+
+// BuildSphericalUV + SphericalCoordinates for pixel (gx,gy) of the level.
+__device__ __forceinline__ V2 spherical_uv(const EnvView& v, const float* __restrict__ intrinsics, int gx, int gy)
+{
+    const ViewConst& vc = v.vc;
+    const float* cr     = v.cr;
+    const V3 tinv       = v.tinv;
+    V2 ip               = {(float)gx, (float)gy};
     V3 inp;
     if (vc.model == 0)
     {
@@ -97,24 +113,25 @@ __device__ __forceinline__ Bilinear bilinear_setup(V2 uv, int ew, int eh)
 }
 
 
-// Both kernels work on tiles of 16 x 16 pixels of one level of one view: workgroup -> (view, level, tile).
-constexpr int kEnvTile = 16;
+// Both kernels work on tiles of one level of one view: workgroup -> (view, level, tile).
+constexpr int kEnvTile = 16;                          // gradient: tiles of 16 x 16 pixels, one per thread
+constexpr int kEnvWide = 64, kEnvRows = 16;           // sampling: tiles of 64 x 16 pixels, four per thread
+constexpr int kEnvPer  = kEnvWide * kEnvRows / kBlock;
 struct EnvTiles
 {
     int prefix[ADOP_MAX_LAYERS + 1];  // tiles of the levels before l (one view)
     int tiles_x[ADOP_MAX_LAYERS];
 };
 
-struct EnvPixel
+struct EnvTileOf
 {
-    int b, l, gx, gy;
-    bool inside;
+    int b, l, tx, ty;
 };
 
-__device__ __forceinline__ EnvPixel env_pixel_of_thread(const Levels& lv, const EnvTiles& et)
+__device__ __forceinline__ EnvTileOf env_tile_of_block(const Levels& lv, const EnvTiles& et)
 {
     const int per_view = et.prefix[lv.num];
-    EnvPixel e;
+    EnvTileOf e;
     e.b   = (int)blockIdx.x / per_view;
     int r = (int)blockIdx.x - e.b * per_view;
     e.l   = 0;
@@ -122,79 +139,116 @@ __device__ __forceinline__ EnvPixel env_pixel_of_thread(const Levels& lv, const 
     for (int k = 1; k < ADOP_MAX_LAYERS; ++k)
         if (k < lv.num && r >= et.prefix[k]) e.l = k;
     r -= et.prefix[e.l];
-    const int ty = r / et.tiles_x[e.l], tx = r - ty * et.tiles_x[e.l];
-    e.gx     = tx * kEnvTile + ((int)threadIdx.x & (kEnvTile - 1));
-    e.gy     = ty * kEnvTile + ((int)threadIdx.x >> 4);
-    e.inside = e.gx < lv.l[e.l].w && e.gy < lv.l[e.l].h;
+    e.ty = r / et.tiles_x[e.l];
+    e.tx = r - e.ty * et.tiles_x[e.l];
     return e;
 }
 
-// The view constants of the workgroup's view, computed by one thread (poses_se3 is f64, the intrinsics row up to 24
+// The constants of the workgroup's view and level, computed by one thread (poses_se3 is f64, the intrinsics row up to 24
 // floats: 256 threads each doing this for themselves cost more than the sampling).
-__device__ __forceinline__ const ViewConst& env_view_const(ViewConst* s_vc, const ViewChunk& chunk, int b,
-                                                           const double* __restrict__ poses,
-                                                           const float* __restrict__ intrinsics, int cols)
+__device__ __forceinline__ const EnvView& env_view_const(EnvView* s_v, const ViewChunk& chunk, int b, int level,
+                                                         const double* __restrict__ poses,
+                                                         const float* __restrict__ intrinsics, int cols)
 {
-    if (threadIdx.x == 0) *s_vc = make_view_const(chunk.v[b], poses, intrinsics, cols);
+    if (threadIdx.x == 0) set_env_view(s_v, make_view_const(chunk.v[b], poses, intrinsics, cols), level);
     __syncthreads();
-    return *s_vc;
+    return *s_v;
 }
 
+// CT: channels as a constant (0: lv.C).  A workgroup waits once for the constants of its view, which one thread computes, and then
+// has four pixels per thread to do, whose masks are requested beforehand; the channels of a pixel are read together:
+// 8 fisheye views of 2200 x 1500, 27 M sampled pixels, 1043 -> 909 us (of which 0.66 ms are vector instructions: the divisions and square
+// roots of the ray); a view of 1365 x 911: 42 -> 38.5 us.
+template <int CT>
 __global__ __launch_bounds__(kBlock) void env_sample_kernel(ViewChunk chunk, const double* __restrict__ poses,
                                                             const float* __restrict__ intrinsics, Levels lv,
                                                             EnvLevels ev, EnvTiles et, const float* __restrict__ tex,
                                                             int eh, int ew, int add_to_out, int cols)
 {
-    __shared__ ViewConst s_vc;
-    const EnvPixel e    = env_pixel_of_thread(lv, et);
-    const ViewConst& vc = env_view_const(&s_vc, chunk, e.b, poses, intrinsics, cols);
-    if (!e.inside) return;
-    const int l = e.l, b = e.b;
+    __shared__ EnvView s_v;
+    const EnvTileOf e = env_tile_of_block(lv, et);
+    const int l = e.l, b = e.b, C = CT ? CT : lv.C;
     const LevelArg& L = lv.l[l];
-    const int p       = e.gy * L.w + e.gx;
     const size_t hw   = (size_t)L.w * L.h;
-    float sc          = 1;
-    for (int k = 0; k < l; ++k) sc /= 2;
-    float bgw = 1.f;
-    if (add_to_out && L.mask) bgw = 1.f - L.mask[(size_t)b * hw + p];
-    if (add_to_out && bgw == 0.f)
+    const int gx      = e.tx * kEnvWide + ((int)threadIdx.x & (kEnvWide - 1));
+    const int gy0     = e.ty * kEnvRows + (int)threadIdx.x / kEnvWide;
+    float weight[kEnvPer];
+#pragma unroll
+    for (int k = 0; k < kEnvPer; ++k)
     {
-        // a rendered pixel: the composition does not sample it (and its uv is not written); out of place it is a copy
-        if (add_to_out == 2)
-            for (int c = 0; c < lv.C; ++c)
-            {
-                const size_t o = ((size_t)b * lv.C + c) * hw + p;
-                ev.env[l][o]   = L.out[o];
-            }
-        else if (ev.env[l])
-            for (int c = 0; c < lv.C; ++c) ev.env[l][((size_t)b * lv.C + c) * hw + p] = 0.f;
-        return;
+        const int gy = gy0 + k * (kBlock / kEnvWide);
+        weight[k]    = 1.f;
+        if (add_to_out && L.mask && gx < L.w && gy < L.h) weight[k] = 1.f - L.mask[(size_t)b * hw + (size_t)gy * L.w + gx];
     }
-    bool need = ev.uv[l] || ev.env[l] || add_to_out;
-    if (!need) return;
-    V2 uv = spherical_uv(vc, intrinsics, sc, e.gx, e.gy);
-    if (ev.uv[l])
+    const EnvView& v = env_view_const(&s_v, chunk, b, l, poses, intrinsics, cols);
+    if (!(ev.uv[l] || ev.env[l] || add_to_out)) return;
+#pragma unroll 1
+    for (int k = 0; k < kEnvPer; ++k)
     {
-        *(float2*)(ev.uv[l] + ((size_t)b * hw + p) * 2) = make_float2(uv.x, uv.y);
-    }
-    if (!ev.env[l] && !(add_to_out && bgw != 0.f)) return;
-    Bilinear s = bilinear_setup(uv, ew, eh);
-    for (int c = 0; c < lv.C; ++c)
-    {
-        const float* tc = tex + (size_t)c * eh * ew;
-        float a         = 0;
-        a += tc[(size_t)s.y0 * ew + s.x0] * s.w00;
-        if (s.x1ok) a += tc[(size_t)s.y0 * ew + s.x0 + 1] * s.w01;
-        if (s.y1ok) a += tc[(size_t)(s.y0 + 1) * ew + s.x0] * s.w10;
-        if (s.x1ok && s.y1ok) a += tc[(size_t)(s.y0 + 1) * ew + s.x0 + 1] * s.w11;
-        size_t o = ((size_t)b * lv.C + c) * hw + p;
-        if (add_to_out == 2)
-            ev.env[l][o] = L.out[o] + bgw * a;  // the composed image, out_l itself stays as the rasterizer left it
-        else
+        const int gy = gy0 + k * (kBlock / kEnvWide);
+        if (gx >= L.w || gy >= L.h) continue;
+        const int p      = gy * L.w + gx;
+        const size_t o   = (size_t)b * C * hw + p;  // channel c: + c * hw
+        float bgw        = weight[0];
+#pragma unroll
+        for (int q = 1; q < kEnvPer; ++q)
+            if (q == k) bgw = weight[q];
+        float image[CT ? CT : 1];
+        if (CT && add_to_out)
         {
-            if (ev.env[l]) ev.env[l][o] = a;
-            if (add_to_out) L.out[o] = L.out[o] + bgw * a;
+#pragma unroll
+            for (int c = 0; c < CT; ++c) image[c] = L.out[o + (size_t)c * hw];
         }
+        if (add_to_out && bgw == 0.f)
+        {
+            // a rendered pixel: the composition does not sample it (and its uv is not written); out of place it is a copy
+            if (add_to_out == 2 || ev.env[l])
+            {
+                if (CT)
+                {
+#pragma unroll
+                    for (int c = 0; c < CT; ++c) ev.env[l][o + (size_t)c * hw] = add_to_out == 2 ? image[c] : 0.f;
+                }
+                else
+                    for (int c = 0; c < C; ++c) ev.env[l][o + (size_t)c * hw] = add_to_out == 2 ? L.out[o + (size_t)c * hw] : 0.f;
+            }
+            continue;
+        }
+        const V2 uv = spherical_uv(v, intrinsics, gx, gy);
+        if (ev.uv[l]) *(float2*)(ev.uv[l] + ((size_t)b * hw + p) * 2) = make_float2(uv.x, uv.y);
+        if (!ev.env[l] && !add_to_out) continue;
+        const Bilinear s = bilinear_setup(uv, ew, eh);
+        auto sample = [&](int c)
+        {
+            const float* tc = tex + (size_t)c * eh * ew + (size_t)s.y0 * ew + s.x0;
+            float a         = 0;
+            a += tc[0] * s.w00;
+            if (s.x1ok) a += tc[1] * s.w01;
+            if (s.y1ok) a += tc[ew] * s.w10;
+            if (s.x1ok && s.y1ok) a += tc[ew + 1] * s.w11;
+            return a;
+        };
+        auto put = [&](int c, float a, float under)
+        {
+            const size_t at = o + (size_t)c * hw;
+            if (add_to_out == 2)
+                ev.env[l][at] = under + bgw * a;  // the composed image, out_l itself stays as the rasterizer left it
+            else
+            {
+                if (ev.env[l]) ev.env[l][at] = a;
+                if (add_to_out) L.out[at] = under + bgw * a;
+            }
+        };
+        if (CT)
+        {
+            float a[CT ? CT : 1];
+#pragma unroll
+            for (int c = 0; c < CT; ++c) a[c] = sample(c);
+#pragma unroll
+            for (int c = 0; c < CT; ++c) put(c, a[c], add_to_out ? image[c] : 0.f);
+        }
+        else
+            for (int c = 0; c < C; ++c) put(c, sample(c), add_to_out ? L.out[o + (size_t)c * hw] : 0.f);
     }
 }
 
@@ -214,7 +268,7 @@ __global__ __launch_bounds__(kBlock) void env_backward_kernel(ViewChunk chunk, c
                                                               EnvLevels ev, EnvTiles et, float* __restrict__ genv, int eh,
                                                               int ew, int cols)
 {
-    __shared__ ViewConst s_vc;
+    __shared__ EnvView s_v;
     __shared__ unsigned long long s_acc[kEnvAccEntries];
     // window of the tile's active pixels in the texture: min / max of y0, of x0, and of x0 shifted by half the width
     // (modulo the width: a tile on the seam of the map is narrow there)
@@ -224,18 +278,23 @@ __global__ __launch_bounds__(kBlock) void env_backward_kernel(ViewChunk chunk, c
         s_box[0] = s_box[2] = s_box[4] = 0x7FFFFFFF;
         s_box[1] = s_box[3] = s_box[5] = -1;
     }
-    const EnvPixel e    = env_pixel_of_thread(lv, et);
-    const ViewConst& vc = env_view_const(&s_vc, chunk, e.b, poses, intrinsics, cols);  // (barrier: s_box is set)
+    const EnvTileOf e = env_tile_of_block(lv, et);
     const int l = e.l, b = e.b, C = lv.C;
+    const int gx = e.tx * kEnvTile + ((int)threadIdx.x & (kEnvTile - 1)), gy = e.ty * kEnvTile + ((int)threadIdx.x >> 4);
     const int half    = ew / 2;
     const LevelArg& L = lv.l[l];
-    const int p       = e.gy * L.w + e.gx;
+    const bool inside = gx < L.w && gy < L.h;
+    const int p       = gy * L.w + gx;
     const size_t hw   = (size_t)L.w * L.h;
-    float sc          = 1;
-    for (int k = 0; k < l; ++k) sc /= 2;
+    // (the constants of the view only where the rays are computed again)
+    const bool kept = ev.uv[l] != nullptr;  // workgroup-uniform
+    if (kept)
+        __syncthreads();  // s_box is set
+    else
+        env_view_const(&s_v, chunk, b, l, poses, intrinsics, cols);  // (its barrier too)
     float bgw = 0.f;
-    if (e.inside) bgw = L.mask ? 1.f - L.mask[(size_t)b * hw + p] : 1.f;
-    const bool active = e.inside && bgw != 0.f;
+    if (inside) bgw = L.mask ? 1.f - L.mask[(size_t)b * hw + p] : 1.f;
+    const bool active = inside && bgw != 0.f;
     Bilinear s;
     s.x0 = s.y0 = 0;
     s.w00 = s.w01 = s.w10 = s.w11 = 0.f;
@@ -243,13 +302,13 @@ __global__ __launch_bounds__(kBlock) void env_backward_kernel(ViewChunk chunk, c
     if (active)
     {
         V2 uv;
-        if (ev.uv[l])  // kept from the forward call
+        if (kept)  // from the forward call
         {
             const float2 t = *(const float2*)(ev.uv[l] + ((size_t)b * hw + p) * 2);
             uv             = {t.x, t.y};
         }
         else
-            uv = spherical_uv(vc, intrinsics, sc, e.gx, e.gy);
+            uv = spherical_uv(s_v, intrinsics, gx, gy);
         s = bilinear_setup(uv, ew, eh);
     }
     // (reduced inside the wavefront first: 64 lanes on one LDS address are served one after the other)
@@ -382,7 +441,7 @@ __global__ void apply_tangent_kernel(double* __restrict__ tangent, double* __res
 }
 
 
-static EnvTiles env_tiles(const Levels& lv)
+static EnvTiles env_tiles(const Levels& lv, int tile_w, int tile_h)
 {
     EnvTiles et;
     int acc = 0;
@@ -392,8 +451,8 @@ static EnvTiles env_tiles(const Levels& lv)
         et.tiles_x[l] = 1;
         if (l < lv.num)
         {
-            et.tiles_x[l] = (lv.l[l].w + kEnvTile - 1) / kEnvTile;
-            acc += et.tiles_x[l] * ((lv.l[l].h + kEnvTile - 1) / kEnvTile);
+            et.tiles_x[l] = (lv.l[l].w + tile_w - 1) / tile_w;
+            acc += et.tiles_x[l] * ((lv.l[l].h + tile_h - 1) / tile_h);
         }
     }
     et.prefix[ADOP_MAX_LAYERS] = acc;
@@ -404,18 +463,25 @@ static EnvTiles env_tiles(const Levels& lv)
 void launch_env_sample(const ViewChunk& chunk, const double* poses, const float* intrinsics, const Levels& lv,
                        const EnvLevels& ev, const float* tex, int eh, int ew, int add_to_out, int cols, hipStream_t st)
 {
-    static_assert(kEnvTile * kEnvTile == kBlock, "one thread per pixel of a tile");
-    const EnvTiles et = env_tiles(lv);
+    const EnvTiles et = env_tiles(lv, kEnvWide, kEnvRows);
     const int grid    = et.prefix[lv.num] * lv.B;
-    if (grid > 0)
-        hipLaunchKernelGGL(env_sample_kernel, dim3(grid), dim3(kBlock), 0, st, chunk, poses, intrinsics, lv, ev, et, tex,
-                           eh, ew, add_to_out, cols);
+    if (grid <= 0) return;
+    if (lv.C == 4)
+        hipLaunchKernelGGL(env_sample_kernel<4>, dim3(grid), dim3(kBlock), 0, st, chunk, poses, intrinsics, lv, ev, et, tex, eh,
+                           ew, add_to_out, cols);
+    else if (lv.C == 8)
+        hipLaunchKernelGGL(env_sample_kernel<8>, dim3(grid), dim3(kBlock), 0, st, chunk, poses, intrinsics, lv, ev, et, tex, eh,
+                           ew, add_to_out, cols);
+    else
+        hipLaunchKernelGGL(env_sample_kernel<0>, dim3(grid), dim3(kBlock), 0, st, chunk, poses, intrinsics, lv, ev, et, tex, eh,
+                           ew, add_to_out, cols);
 }
 
 void launch_env_backward(const ViewChunk& chunk, const double* poses, const float* intrinsics, const Levels& lv,
                          const EnvLevels& ev, float* genv, int eh, int ew, int cols, hipStream_t st)
 {
-    const EnvTiles et = env_tiles(lv);
+    static_assert(kEnvTile * kEnvTile == kBlock, "one thread per pixel of a tile");
+    const EnvTiles et = env_tiles(lv, kEnvTile, kEnvTile);
     const int grid    = et.prefix[lv.num] * lv.B;
     if (grid > 0)
         hipLaunchKernelGGL(env_backward_kernel, dim3(grid), dim3(kBlock), 0, st, chunk, poses, intrinsics, lv, ev, et,
