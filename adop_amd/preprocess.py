@@ -23,6 +23,14 @@ def _checked_position(position):
     return position.contiguous()
 
 
+def _check_normal(normal, position):
+    """The kernels take the address of the normals as it is: a tensor of another device, or one of fewer rows than there are
+    points, is refused here."""
+    if normal is not None and (normal.device != position.device or normal.dim() < 1 or normal.shape[0] < position.shape[0]):
+        raise RuntimeError(f"normal must be a tensor of at least {position.shape[0]} rows on {position.device}, "
+                           f"not {tuple(normal.shape)} on {normal.device}")
+
+
 _RADIUS_BLOCK = 256  # the block size of adop_radius_blocks
 
 
@@ -228,6 +236,7 @@ def PreprocessPointCloud(position, normal=None, rank=4, block_size=256, seed=0):
     gen = torch.Generator(device="cpu").manual_seed(int(seed))
     gen_dev = torch.Generator(device=position.device).manual_seed(int(seed))  # the per-point numbers are drawn on the device
     position = _checked_position(position)
+    _check_normal(normal, position)
     n = int(position.shape[0])
     if block_size != _RADIUS_BLOCK or (normal is not None and (normal.dtype != torch.int32 or normal.numel() != n)):
         order = ReorderMorton64(position)
