@@ -42,6 +42,25 @@ torch::Tensor Workspace(size_t bytes, const torch::Tensor& like)
 {
     return torch::empty({(int64_t)(bytes > 0 ? bytes : 1)}, like.options().dtype(torch::kUInt8));
 }
+// rows[index] for rows of 4 floats.  (torch's own gather of rows of 16 bytes raises at 2^26 rows, and of more it returns
+// wrong ones without an error.)
+torch::Tensor GatherPoints(const torch::Tensor& rows, const torch::Tensor& index)
+{
+    auto out = torch::empty({index.size(0), 4}, rows.options());
+    Check(adop_gather_points(rows.data_ptr<float>(), (int32_t)rows.size(0), index.data_ptr<int64_t>(),
+                             (int32_t)index.size(0), out.data_ptr<float>(), Stream()));
+    return out;
+}
+
+// rows[index] for rows of any size, in parts that torch's gather can take
+torch::Tensor GatherRows(const torch::Tensor& rows, const torch::Tensor& index)
+{
+    const int64_t part = (int64_t)1 << 25;
+    if (index.size(0) <= part) return rows.index({index});
+    std::vector<torch::Tensor> parts;
+    for (const auto& i : index.split(part)) parts.push_back(rows.index({i}));
+    return torch::cat(parts);
+}
 }  // namespace
 
 torch::Tensor KNearestNeighbourDistance(torch::Tensor position, int n)
@@ -168,7 +187,7 @@ torch::Tensor FilterPointCloud(torch::Tensor position, torch::Tensor poses_se3, 
     // (per point: erasing other points does not change it)
     auto cam  = PointDistanceToCamera(position, poses_se3, intrinsics, frames);
     auto keep = RemoveLonelyPoints(position, cam, lonely_n, lonely_th);
-    position  = position.index({keep}).contiguous();
+    position  = GatherPoints(position, keep.nonzero().squeeze(1).contiguous());
     cam       = cam.index({keep});
     ids       = ids.index({keep});
     keep      = RemoveClosePoints(position, cam, close_th);
@@ -183,14 +202,14 @@ PreprocessedCloud PreprocessPointCloud(torch::Tensor position, torch::Tensor nor
     dev_gen.set_current_seed((uint64_t)seed);
     auto order = ReorderMorton64(position);
     order      = order.index({RandomBlockShuffle(position.size(0), block_size, host_gen, position.device())});
-    position   = position.index({order}).contiguous();
+    position   = GatherPoints(position, order);
     auto data  = ComputeRadius(position, n, dev_gen);
     auto by_radius = SortBlocksByRadius(data.select(1, 3), block_size);
     PreprocessedCloud out;
     out.order    = order.index({by_radius});
-    out.position = position.index({by_radius}).clone();
-    out.data     = data.index({by_radius}).contiguous();
+    out.position = GatherPoints(position, by_radius);
+    out.data     = GatherPoints(data, by_radius);
     out.position.select(1, 3).copy_(out.data.select(1, 3));
-    if (normal.defined()) out.normal = normal.index({out.order}).contiguous();
+    if (normal.defined()) out.normal = GatherRows(normal, out.order).contiguous();
     return out;
 }
