@@ -135,7 +135,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(PPT > 2 
                 frame_p[k] = {0.f, 0.f};
                 frame_z[k] = 0.f;
                 if (base + k * kBlock < pc.n)
-                    project_frame(vc, pc.intrinsics, pos, nrm, rp.check_normal != 0, rp.dist_cutoff, &frame_p[k], &frame_z[k],
+                    project_frame<true>(vc, pc.intrinsics, pos, nrm, rp.check_normal != 0, rp.dist_cutoff, &frame_p[k], &frame_z[k],
                                   &view_p);
             }
         }

@@ -787,8 +787,8 @@ def test_every_tuning_variant_gives_the_same_results(oracle_mod, variant, forwar
 @pytest.mark.parametrize("model", ["pinhole", "ocam"])
 @pytest.mark.parametrize("scale", [1.0, 1e-9, 1e6])
 def test_back_face_test_at_grazing_angles(oracle_mod, model, scale):
-    """Normals nearly perpendicular to the line of sight: the kernels take the sign of the back-face test in world
-    coordinates where it is beyond doubt and evaluate the reference's form elsewhere.  Whatever the size of the scene, the
+    """Normals nearly perpendicular to the line of sight: the first binning pass takes the sign of the back-face test in
+    world coordinates where it is beyond doubt and evaluates the reference's form elsewhere, the direct path always.  Whatever the size of the scene, the
     points culled are the checker's: packed depth and weights bit for bit."""
     from adop_amd import scenes
 
