@@ -114,9 +114,8 @@ __device__ __forceinline__ Bilinear bilinear_setup(V2 uv, int ew, int eh)
 
 
 // Both kernels work on tiles of one level of one view: workgroup -> (view, level, tile).
-constexpr int kEnvTile = 16;                          // gradient: tiles of 16 x 16 pixels, one per thread
-constexpr int kEnvWide = 64, kEnvRows = 16;           // sampling: tiles of 64 x 16 pixels, four per thread
-constexpr int kEnvPer  = kEnvWide * kEnvRows / kBlock;
+constexpr int kEnvTile = 16;                                // gradient: tiles of 16 x 16 pixels, one per thread
+constexpr int kEnvWide = 64, kEnvRows = kBlock / kEnvWide;  // sampling: tiles of 64 x 4 pixels, one per thread
 struct EnvTiles
 {
     int prefix[ADOP_MAX_LAYERS + 1];  // tiles of the levels before l (one view)
@@ -155,10 +154,12 @@ __device__ __forceinline__ const EnvView& env_view_const(EnvView* s_v, const Vie
     return *s_v;
 }
 
-// CT: channels as a constant (0: lv.C).  A workgroup waits once for the constants of its view, which one thread computes, and then
-// has four pixels per thread to do, whose masks are requested beforehand; the channels of a pixel are read together:
-// 8 fisheye views of 2200 x 1500, 27 M sampled pixels, 1043 -> 909 us (of which 0.66 ms are vector instructions: the divisions and square
-// roots of the ray); a view of 1365 x 911: 42 -> 38.5 us.
+// CT: channels as a constant (0: lv.C).  A workgroup waits once for the constants of its view, which one thread computes; the
+// mask is requested beforehand, the channels of a pixel are read together, and a wavefront lies in one row of the image, so
+// that what it reads and writes of a channel are whole lines.  Tiles of 16 x 16 pixels / of 64 x 16 with four pixels per
+// thread / of 64 x 4 (taken), fp32: 8 fisheye views of 2200 x 1500 1042 / 910 / 859 us (most of it the divisions and square
+// roots of the rays), one 127 / 117 / 108, a view of 1365 x 911 42 / 38 / 36, with 8 channels 89 / 90 / 58, of 457 x 162
+// (fisheye) 13 / 29 / 11: four pixels per thread leave a small image with fewer workgroups than the GPU has CUs.
 template <int CT>
 __global__ __launch_bounds__(kBlock) void env_sample_kernel(ViewChunk chunk, const double* __restrict__ poses,
                                                             const float* __restrict__ intrinsics, Levels lv,
@@ -170,86 +171,70 @@ __global__ __launch_bounds__(kBlock) void env_sample_kernel(ViewChunk chunk, con
     const int l = e.l, b = e.b, C = CT ? CT : lv.C;
     const LevelArg& L = lv.l[l];
     const size_t hw   = (size_t)L.w * L.h;
-    const int gx      = e.tx * kEnvWide + ((int)threadIdx.x & (kEnvWide - 1));
-    const int gy0     = e.ty * kEnvRows + (int)threadIdx.x / kEnvWide;
-    float weight[kEnvPer];
-#pragma unroll
-    for (int k = 0; k < kEnvPer; ++k)
-    {
-        const int gy = gy0 + k * (kBlock / kEnvWide);
-        weight[k]    = 1.f;
-        if (add_to_out && L.mask && gx < L.w && gy < L.h) weight[k] = 1.f - L.mask[(size_t)b * hw + (size_t)gy * L.w + gx];
-    }
+    const int gx = e.tx * kEnvWide + ((int)threadIdx.x & (kEnvWide - 1)), gy = e.ty * kEnvRows + (int)threadIdx.x / kEnvWide;
+    const bool inside = gx < L.w && gy < L.h;
+    const int p       = gy * L.w + gx;
+    const size_t o    = (size_t)b * C * hw + p;  // channel c: + c * hw
+    float bgw         = 1.f;
+    if (add_to_out && L.mask && inside) bgw = 1.f - L.mask[(size_t)b * hw + p];
     const EnvView& v = env_view_const(&s_v, chunk, b, l, poses, intrinsics, cols);
-    if (!(ev.uv[l] || ev.env[l] || add_to_out)) return;
-#pragma unroll 1
-    for (int k = 0; k < kEnvPer; ++k)
+    if (!inside || !(ev.uv[l] || ev.env[l] || add_to_out)) return;
+    float image[CT ? CT : 1];
+    if (CT && add_to_out)
     {
-        const int gy = gy0 + k * (kBlock / kEnvWide);
-        if (gx >= L.w || gy >= L.h) continue;
-        const int p      = gy * L.w + gx;
-        const size_t o   = (size_t)b * C * hw + p;  // channel c: + c * hw
-        float bgw        = weight[0];
 #pragma unroll
-        for (int q = 1; q < kEnvPer; ++q)
-            if (q == k) bgw = weight[q];
-        float image[CT ? CT : 1];
-        if (CT && add_to_out)
-        {
-#pragma unroll
-            for (int c = 0; c < CT; ++c) image[c] = L.out[o + (size_t)c * hw];
-        }
-        if (add_to_out && bgw == 0.f)
-        {
-            // a rendered pixel: the composition does not sample it (and its uv is not written); out of place it is a copy
-            if (add_to_out == 2 || ev.env[l])
-            {
-                if (CT)
-                {
-#pragma unroll
-                    for (int c = 0; c < CT; ++c) ev.env[l][o + (size_t)c * hw] = add_to_out == 2 ? image[c] : 0.f;
-                }
-                else
-                    for (int c = 0; c < C; ++c) ev.env[l][o + (size_t)c * hw] = add_to_out == 2 ? L.out[o + (size_t)c * hw] : 0.f;
-            }
-            continue;
-        }
-        const V2 uv = spherical_uv(v, intrinsics, gx, gy);
-        if (ev.uv[l]) *(float2*)(ev.uv[l] + ((size_t)b * hw + p) * 2) = make_float2(uv.x, uv.y);
-        if (!ev.env[l] && !add_to_out) continue;
-        const Bilinear s = bilinear_setup(uv, ew, eh);
-        auto sample = [&](int c)
-        {
-            const float* tc = tex + (size_t)c * eh * ew + (size_t)s.y0 * ew + s.x0;
-            float a         = 0;
-            a += tc[0] * s.w00;
-            if (s.x1ok) a += tc[1] * s.w01;
-            if (s.y1ok) a += tc[ew] * s.w10;
-            if (s.x1ok && s.y1ok) a += tc[ew + 1] * s.w11;
-            return a;
-        };
-        auto put = [&](int c, float a, float under)
-        {
-            const size_t at = o + (size_t)c * hw;
-            if (add_to_out == 2)
-                ev.env[l][at] = under + bgw * a;  // the composed image, out_l itself stays as the rasterizer left it
-            else
-            {
-                if (ev.env[l]) ev.env[l][at] = a;
-                if (add_to_out) L.out[at] = under + bgw * a;
-            }
-        };
-        if (CT)
-        {
-            float a[CT ? CT : 1];
-#pragma unroll
-            for (int c = 0; c < CT; ++c) a[c] = sample(c);
-#pragma unroll
-            for (int c = 0; c < CT; ++c) put(c, a[c], add_to_out ? image[c] : 0.f);
-        }
-        else
-            for (int c = 0; c < C; ++c) put(c, sample(c), add_to_out ? L.out[o + (size_t)c * hw] : 0.f);
+        for (int c = 0; c < CT; ++c) image[c] = L.out[o + (size_t)c * hw];
     }
+    if (add_to_out && bgw == 0.f)
+    {
+        // a rendered pixel: the composition does not sample it (and its uv is not written); out of place it is a copy
+        if (add_to_out == 2 || ev.env[l])
+        {
+            if (CT)
+            {
+#pragma unroll
+                for (int c = 0; c < CT; ++c) ev.env[l][o + (size_t)c * hw] = add_to_out == 2 ? image[c] : 0.f;
+            }
+            else
+                for (int c = 0; c < C; ++c) ev.env[l][o + (size_t)c * hw] = add_to_out == 2 ? L.out[o + (size_t)c * hw] : 0.f;
+        }
+        return;
+    }
+    const V2 uv = spherical_uv(v, intrinsics, gx, gy);
+    if (ev.uv[l]) *(float2*)(ev.uv[l] + ((size_t)b * hw + p) * 2) = make_float2(uv.x, uv.y);
+    if (!ev.env[l] && !add_to_out) return;
+    const Bilinear s = bilinear_setup(uv, ew, eh);
+    auto sample = [&](int c)
+    {
+        const float* tc = tex + (size_t)c * eh * ew + (size_t)s.y0 * ew + s.x0;
+        float a         = 0;
+        a += tc[0] * s.w00;
+        if (s.x1ok) a += tc[1] * s.w01;
+        if (s.y1ok) a += tc[ew] * s.w10;
+        if (s.x1ok && s.y1ok) a += tc[ew + 1] * s.w11;
+        return a;
+    };
+    auto put = [&](int c, float a, float under)
+    {
+        const size_t at = o + (size_t)c * hw;
+        if (add_to_out == 2)
+            ev.env[l][at] = under + bgw * a;  // the composed image, out_l itself stays as the rasterizer left it
+        else
+        {
+            if (ev.env[l]) ev.env[l][at] = a;
+            if (add_to_out) L.out[at] = under + bgw * a;
+        }
+    };
+    if (CT)
+    {
+        float a[CT ? CT : 1];
+#pragma unroll
+        for (int c = 0; c < CT; ++c) a[c] = sample(c);
+#pragma unroll
+        for (int c = 0; c < CT; ++c) put(c, a[c], add_to_out ? image[c] : 0.f);
+    }
+    else
+        for (int c = 0; c < C; ++c) put(c, sample(c), add_to_out ? L.out[o + (size_t)c * hw] : 0.f);
 }
 
 // Gradient of the texture.  The pixels of a tile land in a small window of the texture (a texel takes hundreds of

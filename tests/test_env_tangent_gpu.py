@@ -230,6 +230,24 @@ def test_env_random_scenes(oracle_mod, seed):
     assert_norm_close(g_env_uv.cpu().numpy(), tex.grad.numpy(), 2e-5, "grad env texture (uv from the forward call)")
 
 
+@pytest.mark.parametrize("channels", [3, 4, 8])
+@pytest.mark.parametrize("w,h", [(1, 9), (63, 3), (64, 4), (65, 5), (130, 8)])
+def test_env_at_the_edges_of_a_tile(oracle_mod, w, h, channels):
+    """Images around the 64 x 4 pixels of a workgroup of the sampling kernel, two views, channel counts of each variant."""
+    from adop_amd import scenes
+
+    announce(f"environment map, {w}x{h}, {channels} channels")
+    hs = scenes.config2(n=3_000, w=w, h=h, levels=1, batch=2, seed=w)
+    g = np.random.default_rng(w)
+    hs.texture = g.random((channels, hs.num_points), dtype=np.float32)
+    hs.background = g.random(channels, dtype=np.float32)
+    hs.env_texture = g.random((channels, 33, 61), dtype=np.float32)
+    hs.params.output_background_mask = 1
+    hs.params.output_background_mask_value = 0.0
+    hs.dropout = scenes.bernoulli_mask(w, 2, hs.num_points, 0.9)
+    _check_sampling_and_composition(oracle_mod, hs, min_empty=0)
+
+
 def test_env_rejects_unknown_model_and_bad_rows():
     import ctypes as C
     from adop_amd import _capi, scenes
