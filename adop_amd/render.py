@@ -130,7 +130,7 @@ class NeuralRenderInfo:
 
 class PointRendererCache:
     """Buffer lifecycle of the render stage; reallocates only when {C,N,L,B,h,w} changes
-    (PointRenderer.cu:952-1037)."""
+    (PointRenderer.cu:952-1037), or the stream."""
 
     def __init__(self):
         self.lib = _capi.load_library()
@@ -156,13 +156,32 @@ class PointRendererCache:
         if forward:
             self.InitializeData(forward)
 
+    def take_workspace(self, info):
+        """Scratch memory for a pass of ``info`` on the current stream: what the last pass had, if that was of the same
+        size and on the same stream.  Nothing in it outlives the passes queued on its stream, so it is shared by passes
+        that run one after the other and by no others: another stream gets its own, and so does every captured pass (the
+        graph goes on writing what it recorded).  Returns the key of buffers that may be used again under the same
+        conditions, None under capture."""
+        fd, scene = info.images[0], info.scene
+        key = (int(scene.texture.shape[0]), scene.point_cloud_cuda.Size(), info.num_layers, len(info.images), fd.h, fd.w,
+               int(info.workspace_flags), scene.texture.device, _raw_stream(), scene.poses_se3.shape[0],
+               tuple(scene.intrinsics.shape))
+        if torch.cuda.is_current_stream_capturing():
+            key = None
+        if key is None or key != self._workspace_key:
+            s = scene.struct()
+            nbytes = self.lib.adop_workspace_size_for(C.byref(s), len(info.images), info.num_layers, fd.w, fd.h,
+                                                      int(info.workspace_flags))
+            self.workspace = None  # (given back before the next one is taken)
+            self.workspace = torch.empty(max(int(nbytes), 256), dtype=torch.uint8, device=scene.texture.device)
+            self._workspace_key = key
+        return key
+
     def Allocate(self, info, forward):
         fd = info.images[0]
-        scene = info.scene
-        dev = scene.texture.device
-        new_size = (int(scene.texture.shape[0]), scene.point_cloud_cuda.Size(), info.num_layers, self.num_batches,
-                    fd.h, fd.w, int(info.workspace_flags))
-        if new_size == self.cache_size:
+        dev = info.scene.texture.device
+        key = self.take_workspace(info)
+        if key is not None and key == self.cache_size:
             return
         B = self.num_batches
         self.layers_cuda = []
@@ -177,19 +196,8 @@ class PointRendererCache:
             w //= 2
             h //= 2
             scale *= 0.5
-        # The workspace is scratch memory: nothing in it outlives the passes queued on its stream, so it stays while
-        # they take the same amount of it on the same stream.  (A pass that is captured takes its own: the graph keeps it.)
-        stream = _raw_stream()
-        key = (new_size, dev, stream, scene.poses_se3.shape[0], tuple(scene.intrinsics.shape))
-        capturing = torch.cuda.is_current_stream_capturing()
-        if capturing or key != self._workspace_key:
-            s = scene.struct()
-            nbytes = self.lib.adop_workspace_size_for(C.byref(s), B, info.num_layers, fd.w, fd.h, int(info.workspace_flags))
-            self.workspace = None  # (given back before the next one is taken)
-            self.workspace = torch.empty(max(int(nbytes), 256), dtype=torch.uint8, device=dev)
-            self._workspace_key = None if capturing else key
         self._stats = None
-        self.cache_size = new_size
+        self.cache_size = key
 
     @property
     def stats(self):
@@ -342,6 +350,7 @@ def BlendPointCloudBackward(ctx, info, image_gradients, needs=(True, True, True)
 
     cache.num_batches = len(info.images)
     cache.info = info
+    cache.take_workspace(info)
     s = scene.struct()
     stats = C.c_void_p(cache.stats.data_ptr()) if info.collect_stats else None
     info.params.workspace_flags = int(info.workspace_flags)
