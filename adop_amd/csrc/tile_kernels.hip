@@ -734,10 +734,9 @@ static hipError_t launch_tile_blend_t(const CloudArg& pc, const Levels& lv, cons
 #define ADOP_TILE_K(K, STATS)                                                                                            \
     launch_tile_blend_k<CT, HALF, K, LT, STATS>(pc, lv, rp, bin, num_tiles, accum, S, background, write_mask, mask_value, \
                                                 identity_index, stats, st)
-    if (stats) return ADOP_TILE_K(1, true);  // (a counter pass: one variant)
-    if (k == 1) return ADOP_TILE_K(1, false);
-    if (k == 4) return ADOP_TILE_K(4, false);
-    return ADOP_TILE_K(2, false);
+    if (k == 1) return stats ? ADOP_TILE_K(1, true) : ADOP_TILE_K(1, false);
+    if (k == 4) return stats ? ADOP_TILE_K(4, true) : ADOP_TILE_K(4, false);
+    return stats ? ADOP_TILE_K(2, true) : ADOP_TILE_K(2, false);
 #undef ADOP_TILE_K
 }
 

@@ -784,6 +784,20 @@ def test_every_tuning_variant_gives_the_same_results(oracle_mod, variant, forwar
             _fwd_bwd(scene, oracle_mod, collect_stats=False, poison=True)
 
 
+@pytest.mark.parametrize("channels", [3, 4, 8])
+@pytest.mark.parametrize("tile_k", [1, 2, 4])
+def test_counter_passes_of_every_batch_size(oracle_mod, forward_path, tile_k, channels):
+    """The counters are those of the kernel variant the tuning set asks for: every batch size of the tile blend counts."""
+    from adop_amd import _capi, scenes
+
+    if forward_path != 2:
+        pytest.skip("the tile path only")
+    announce(f"counter pass, tile_k={tile_k}, C={channels}: 60k pts 200x120 L4")
+    hs = scenes.config3(n=60_000, w=200, h=120, channels=channels, seed=12)
+    with _capi.tuning(tile_k=tile_k):
+        _fwd_bwd(hs, oracle_mod, collect_stats=True)
+
+
 @pytest.mark.parametrize("model", ["pinhole", "ocam"])
 @pytest.mark.parametrize("scale", [1.0, 1e-9, 1e6])
 def test_back_face_test_at_grazing_angles(oracle_mod, model, scale):
