@@ -72,7 +72,10 @@ __global__ __launch_bounds__(kBlock) void clear_kernel(Levels lv, int first_leve
 // pixel, one lane per distinct pixel takes the minimum of its group from LDS and issues the 64-bit atomicMin:
 // clouds stored in Morton-ordered blocks collide heavily at the coarse levels, and a device-scope atomic costs one
 // memory transaction whatever it carries.
-template <int PPT, bool STATS>
+// The counters are a branch at run time, not a variant as in the other kernels: with the shorter code of a variant more
+// wavefronts read a depth before the first of them has lowered it, and they issue redundant atomics (1.4 M points on a few
+// hundred pixels, fisheye: 255 us with the branch, 267 without; 100 M points on 1920 x 1080 do not differ).
+template <int PPT>
 __global__ __launch_bounds__(kBlock) void prepass_kernel(CloudArg pc, const ViewConst* __restrict__ views, Levels lv,
                                                          ParamArg rp, int group_from, adop_stats* stats, Gate gate)
 {
@@ -80,6 +83,7 @@ __global__ __launch_bounds__(kBlock) void prepass_kernel(CloudArg pc, const View
     if (gate_closed(gate)) return;
     __shared__ unsigned long long s_gmask[kBlock];
     __shared__ uint32_t s_gkey[kBlock];
+    const bool STATS = stats != nullptr;  // counter pass (uniform branch)
     const int lane   = threadIdx.x & 63;
     const int wbase  = threadIdx.x & ~63;
     unsigned long long* pk_w    = s_pk + wbase;
@@ -611,23 +615,14 @@ void launch_prepass(const CloudArg& pc, const ViewConst* views, const Levels& lv
     const int group_from = tn.prepass_group_from;
     const int ppt        = prepass_ppt(pc.n, tn.prepass_ppt);
     const dim3 grid((pc.n + kBlock * ppt - 1) / (kBlock * ppt));
-#define ADOP_PREPASS(PPT)                                                                                               \
-    if (stats)                                                                                                           \
-        hipLaunchKernelGGL((prepass_kernel<PPT, true>), grid, dim3(kBlock), 0, st, pc, views, lv, rp, group_from, stats, gate); \
-    else                                                                                                                 \
-        hipLaunchKernelGGL((prepass_kernel<PPT, false>), grid, dim3(kBlock), 0, st, pc, views, lv, rp, group_from, stats, gate);
+#define ADOP_PREPASS(PPT) \
+    hipLaunchKernelGGL((prepass_kernel<PPT>), grid, dim3(kBlock), 0, st, pc, views, lv, rp, group_from, stats, gate)
     if (ppt == 4)
-    {
-        ADOP_PREPASS(4)
-    }
+        ADOP_PREPASS(4);
     else if (ppt == 2)
-    {
-        ADOP_PREPASS(2)
-    }
+        ADOP_PREPASS(2);
     else
-    {
-        ADOP_PREPASS(1)
-    }
+        ADOP_PREPASS(1);
 #undef ADOP_PREPASS
 }
 
