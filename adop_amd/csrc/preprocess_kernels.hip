@@ -616,10 +616,71 @@ __global__ __launch_bounds__(kBlock) void knn_coarse_kernel(const float4* __rest
     }
 }
 
-// Stage 4: stray points far from everything (no cube of a few shells of either grid settles them): one workgroup per point
-// goes through all points (a wavefront per point, 1 M points of a Gaussian cloud: 1.5 ms; a workgroup of 16: 0.25 ms - there
-// are fewer strays than the GPU has wavefronts).
-constexpr int kBruteBlock = 1024;
+// Stage 4: stray points far from everything (no cube of a few shells of either grid settles them): one workgroup goes through
+// all points for one of them, or for kBruteStrays together where there are more strays than workgroups.  (A wavefront per
+// stray, 1 M points of a Gaussian cloud: 1.5 ms; a workgroup of 16: 0.25 ms - there are fewer strays than the GPU has
+// wavefronts.)  With thousands of strays the points come from the last cache over and over, 5 TB/s of them, so strays share
+// a pass; of the thousands of points a thread sees few get into its lists, so a round of kBruteRound points is looked at as a
+// whole before any of it goes in.  6 M points of a Gaussian cloud, rank 4 / 8 (some 1500 / 4000 strays): one stray per pass
+// 29.8 / 77.5 ms, four 6.2 / 14.3.
+constexpr int kBruteBlock  = 1024;
+constexpr int kBruteStrays = 4;
+constexpr int kBruteRound  = 4;
+
+template <int K, int S>
+__device__ __forceinline__ void brute_pass(const float4* __restrict__ points, int n, const uint32_t* __restrict__ list,
+                                           uint32_t first, uint32_t count, float (*s_best)[kBruteBlock / 64][K],
+                                           float* __restrict__ out)
+{
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    float4 p[S];
+    float best[S][K];
+#pragma unroll
+    for (int s = 0; s < S; ++s)
+    {
+        p[s] = points[list[first + s < count ? first + s : count - 1]];
+#pragma unroll
+        for (int k = 0; k < K; ++k) best[s][k] = 3.0e38f;
+    }
+    for (size_t q0 = threadIdx.x; q0 < (size_t)n; q0 += kBruteRound * kBruteBlock)
+    {
+        float4 o[kBruteRound];
+#pragma unroll
+        for (int u = 0; u < kBruteRound; ++u)
+        {
+            const size_t q = q0 + u * kBruteBlock;
+            o[u]           = points[q < (size_t)n ? q : (size_t)n - 1];
+        }
+#pragma unroll
+        for (int s = 0; s < S; ++s)
+        {
+            float d2[kBruteRound], nearest = 3.0e38f;
+#pragma unroll
+            for (int u = 0; u < kBruteRound; ++u)
+            {
+                d2[u]   = q0 + u * kBruteBlock < (size_t)n ? distance2(p[s], o[u]) : 3.0e38f;
+                nearest = fminf(nearest, d2[u]);
+            }
+            if (nearest < best[s][K - 1])
+            {
+#pragma unroll
+                for (int u = 0; u < kBruteRound; ++u) keep_smallest<K>(best[s], d2[u]);
+            }
+        }
+    }
+#pragma unroll
+    for (int s = 0; s < S; ++s) wave_kth<K>(best[s], s_best[s][wave]);
+    __syncthreads();
+    if (wave < S && first + wave < count)  // the wavefronts' lists of one stray, one per lane
+    {
+        float all[K];
+#pragma unroll
+        for (int k = 0; k < K; ++k) all[k] = lane < kBruteBlock / 64 ? s_best[wave][lane][k] : 3.0e38f;
+        const float kth = wave_kth<K>(all);
+        if (lane == 0) out[__float_as_uint(points[list[first + wave]].w)] = sqrtf(kth);
+    }
+    __syncthreads();  // s_best has been read
+}
 
 template <int K>
 __global__ __launch_bounds__(kBruteBlock) void knn_brute_kernel(const float4* __restrict__ points, int n,
@@ -627,28 +688,16 @@ __global__ __launch_bounds__(kBruteBlock) void knn_brute_kernel(const float4* __
                                                                 const uint32_t* __restrict__ list_count,
                                                                 float* __restrict__ out)
 {
-    __shared__ float s_best[kBruteBlock / 64][K];
-    const uint32_t count = *list_count;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    for (uint32_t e = blockIdx.x; e < count; e += gridDim.x)
+    __shared__ float s_best[kBruteStrays][kBruteBlock / 64][K];
+    static_assert(kBruteStrays <= kBruteBlock / 64, "one wavefront per stray at the end");
+    const uint32_t count = *list_count;  // (all branches on it are uniform over the grid)
+    if (count <= gridDim.x)
     {
-        const float4 p = points[list[e]];
-        float best[K];
-#pragma unroll
-        for (int k = 0; k < K; ++k) best[k] = 3.0e38f;
-#pragma unroll 4
-        for (int q = threadIdx.x; q < n; q += kBruteBlock) keep_smallest<K>(best, distance2(p, points[q]));
-        wave_kth<K>(best, s_best[wave]);
-        __syncthreads();
-        if (wave == 0)  // the wavefronts' lists, one per lane
-        {
-#pragma unroll
-            for (int k = 0; k < K; ++k) best[k] = lane < kBruteBlock / 64 ? s_best[lane][k] : 3.0e38f;
-            const float kth = wave_kth<K>(best);
-            if (lane == 0) out[__float_as_uint(p.w)] = sqrtf(kth);
-        }
-        __syncthreads();  // s_best has been read
+        if (blockIdx.x < count) brute_pass<K, 1>(points, n, list, blockIdx.x, count, s_best, out);
     }
+    else
+        for (uint32_t e = blockIdx.x * kBruteStrays; e < count; e += gridDim.x * kBruteStrays)
+            brute_pass<K, kBruteStrays>(points, n, list, e, count, s_best, out);
 }
 
 // The neighbour distance of `samples` points evenly spaced in the order of the coarse grid, one wavefront per point (the

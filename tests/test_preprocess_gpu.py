@@ -324,6 +324,41 @@ def test_knn_distance_of_large_clouds(kind):
         assert torch.equal(got[torch.from_numpy(sample).cuda()].view(torch.int32), want.view(torch.int32)), (kind, rank)
 
 
+def _strays(ws):
+    """Points the last search left to the scan over all points: the third list counter of the workspace."""
+    import torch
+
+    return int(ws[256 + 256 + 4 * 1024:][:16].view(torch.int32)[2].item())
+
+
+@pytest.mark.parametrize("rank", [1, 4, 8])
+@pytest.mark.parametrize("n,few", [(20_000, True), ((1 << 17) + 77, False)], ids=["a_workgroup_each", "four_per_workgroup"])
+def test_knn_distance_of_strays(n, few, rank):
+    """Points far from everything are searched for in the whole cloud, one by a workgroup or four together where there are
+    more of them than workgroups (512).  The points farthest out and a sample of the others bit for bit against all
+    distances."""
+    import torch
+    from adop_amd import preprocess as pp
+
+    announce(f"knn distance of strays, N={n}, rank {rank}")
+    g = np.random.default_rng(2)
+    p = np.zeros((n, 4), np.float32)
+    p[:, :3] = g.standard_normal((n, 3)) * np.exp((1.5 if few else 2.0) * g.standard_normal((n, 1)))
+    dev = torch.from_numpy(p).cuda()
+    ws = pp._knn_workspace(dev)
+    got = pp._knn_distance(dev, rank, pp._bbox(dev), ws)
+    strays = _strays(ws)
+    print(f"[info] {strays} strays", flush=True)
+    assert (1 <= strays <= 512) if few else strays > 512 + 4
+    far = np.argsort(-np.abs(p[:, :3]).max(1))[:4000]
+    check = torch.from_numpy(np.concatenate([far, g.integers(0, n, 200)])).cuda()
+    for part in check.split(500):
+        q = dev[part, :3]
+        d = [q[:, k, None] - dev[None, :, k] for k in range(3)]
+        want = ((d[0] * d[0] + d[1] * d[1]) + d[2] * d[2]).kthvalue(rank + 1, dim=1).values.sqrt()
+        assert torch.equal(got[part].view(torch.int32), want.view(torch.int32))
+
+
 def test_filter_refuses_a_cloud_it_empties():
     import torch
     from adop_amd import preprocess, scenes
