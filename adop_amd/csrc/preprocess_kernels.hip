@@ -1073,12 +1073,16 @@ void launch_knn_first_grid(const float4* position, int n, const KnnGrid& box, Kn
 // candidates (their number goes with the square of the cell on a surface, with the cube in a volume) and more points that the
 // cube of 27 cells does not settle.  1.5 measured best over surfaces and volumes (search of 10 M points on 1000 patches,
 // 3 M in a volume, whole call: 2.0: 1365, 786 us; 1.5: 1264, 574; 1.2: 1283, 1015).  Where the samples are taken in every
-// s-th point, their nearest neighbour there stands in for the s-th in the cloud, and d_R = d_s (R / s)^(1 / D) for a
-// cloud of dimension D: 2.5 is within 14 % for surfaces and volumes alike.
+// s-th point, their nearest neighbour there stands in for the s-th in the cloud, and d_R = d_s (R / s)^(1 / D) for a cloud of
+// dimension D.  D = 2.5 is 32 % above a surface's value at R = 1, s = 16 and 17 % below a volume's, and cells too small by
+// that much leave a tenth of a volume's points unsettled; the distance to the nearest neighbour also spreads more about its
+// median than that to the 8th.  R + 1.25 in the place of R takes care of both where it matters and costs surfaces nothing
+// (6 M points in a volume, rank 1 / 2 / 4 / 8: with R 2.03, 1.87, 1.35, 1.30 ms,
+// with R + 1.25 1.05, 1.06, 1.13, 1.36; 10 M points on patches 2.07 and 2.08).
 void launch_knn_refine_grid(const float* sample, int samples, int rank, int stride, const KnnGrid* first, KnnGrid* g,
                             uint32_t budget, uint32_t* list_counts, hipStream_t st)
 {
-    const float factor = 1.5f * (stride > 1 ? powf((float)rank / (float)stride, 0.4f) : 1.0f);
+    const float factor = 1.5f * (stride > 1 ? powf(((float)rank + 1.25f) / (float)stride, 0.4f) : 1.0f);
     hipLaunchKernelGGL(knn_refine_grid_kernel, dim3(1), dim3(1024), 0, st, sample, samples, factor, first, g, budget,
                        list_counts);
 }
