@@ -938,7 +938,14 @@ __global__ __launch_bounds__(kBlock) void camera_distance_sorted_kernel(const fl
 // the rounding of four operations, which the widened reach covers (1e-4 of the radius; 1e-20 where its square
 // underflows).  The radii of the filter are a hundredth of a cell: one row of one or two cells in place of the 27 around the
 // point (3 M points in random order: 730 -> 177 us, most of it the states and radii, which are gathered by id).
+// A scene in a unit of its own has radii of many cells (the radius grows as the unit, the cells shrink): then the kernel waits
+// for the rows it looks up, one load after the other.  One flat loop over candidates, rows and bricks, so that a wavefront
+// takes as many turns as its longest lane needs of all of them together and not the longest of every row; where the ball
+// spans a brick in x the rows of a layer are one run; candidates and their states come in fours.  Whole call, cells row by
+// row / flat: 1 M points on patches, radii of 4 cells 7.0 / 4.8 ms, of a Gaussian cloud 10.7 / 8.2, on a plane and a sphere
+// 15.8 / 14.3; 3 M points with radii of a hundredth of a cell 252 / 231 us in this kernel.
 constexpr int kStateUndecided = 0, kStateKept = 1, kStateErased = 2;
+constexpr int kCloseUnroll    = 4;
 
 __global__ __launch_bounds__(kBlock) void close_points_kernel(KnnView kv, int n, const float* __restrict__ radius,
                                                               int32_t* state, uint32_t* round_count, int round)
@@ -959,29 +966,76 @@ __global__ __launch_bounds__(kBlock) void close_points_kernel(KnnView kv, int n,
             const int3 lo   = grid_cell(g, p.x - reach, p.y - reach, p.z - reach);
             const int3 hi   = grid_cell(g, p.x + reach, p.y + reach, p.z + reach);
             int result = kStateKept;
-            for (int cz = lo.z; cz <= hi.z && result != kStateErased; ++cz)
-                for (int cy = lo.y; cy <= hi.y && result != kStateErased; ++cy)
-                    for (int part = lo.x >> kBrickX; part <= hi.x >> kBrickX && result != kStateErased; ++part)
+            const int3 b0 = {lo.x >> kBrickX, lo.y >> kBrickY, lo.z >> kBrickZ}, b1 = {hi.x >> kBrickX, hi.y >> kBrickY, hi.z >> kBrickZ};
+            int3 b        = {b0.x - 1, b0.y, b0.z};  // (no brick yet)
+            int xa = 0, xb = 0, ya = 0, yb = 0, zb = -1, cy = 0, cz = 0;
+            uint32_t slot = kNoBrick, q = 0, e = 0;
+            for (;;)
+            {
+                if (q < e)
+                {
+                    float4 o[kCloseUnroll];
+#pragma unroll
+                    for (int u = 0; u < kCloseUnroll; ++u) o[u] = kv.sorted[min(q + u, e - 1)];
+                    // (the states of all candidates that count are requested before the first is looked at; the state of the
+                    // point itself, which is undecided and stands in for the others, is not looked at)
+                    bool near[kCloseUnroll], any = false;
+#pragma unroll
+                    for (int u = 0; u < kCloseUnroll; ++u)
                     {
-                        const uint32_t slot = kv.slot[brick_row(g, cy, cz) + (uint32_t)part];
-                        if (slot == kNoBrick) continue;
-                        uint32_t q, e;
-                        brick_range(kv, slot, max(lo.x, part << kBrickX), min(hi.x, part << kBrickX | 7), cy, cz, &q, &e);
-                        for (; q < e; ++q)
+                        near[u] = q + u < e && __float_as_uint(o[u].w) < i && distance2(p, o[u]) < r2;
+                        any |= near[u];
+                    }
+                    if (any)
+                    {
+                        int32_t sj[kCloseUnroll];
+#pragma unroll
+                        for (int u = 0; u < kCloseUnroll; ++u)
+                            sj[u] = __atomic_load_n(&state[near[u] ? __float_as_uint(o[u].w) : i], __ATOMIC_RELAXED);
+#pragma unroll
+                        for (int u = 0; u < kCloseUnroll; ++u)
                         {
-                            const float4 o   = kv.sorted[q];
-                            const uint32_t j = __float_as_uint(o.w);
-                            if (j >= i) continue;
-                            if (!(distance2(p, o) < r2)) continue;
-                            const int sj = __atomic_load_n(&state[j], __ATOMIC_RELAXED);
-                            if (sj == kStateKept)
-                            {
-                                result = kStateErased;
-                                break;
-                            }
-                            if (sj == kStateUndecided) result = kStateUndecided;
+                            if (near[u] && sj[u] == kStateKept) result = kStateErased;
+                            if (near[u] && sj[u] == kStateUndecided && result != kStateErased) result = kStateUndecided;
                         }
                     }
+                    if (result == kStateErased) break;
+                    q += kCloseUnroll;
+                }
+                else if (cz <= zb)  // the next row or layer of the brick
+                {
+                    const int ye        = xb - xa == 7 ? yb : cy;
+                    const uint32_t* row = kv.cell_start + ((size_t)slot << 7);
+                    q                   = row[brick_local(xa, cy, cz)];
+                    e                   = row[brick_local(xb, ye, cz) + 1];
+                    cy                  = ye + 1;
+                    if (cy > yb)
+                    {
+                        cy = ya;
+                        ++cz;
+                    }
+                }
+                else  // the next brick of the box
+                {
+                    if (++b.x > b1.x)
+                    {
+                        b.x = b0.x;
+                        if (++b.y > b1.y)
+                        {
+                            b.y = b0.y;
+                            if (++b.z > b1.z) break;
+                        }
+                    }
+                    slot = kv.slot[brick_row(g, b.y << kBrickY, b.z << kBrickZ) + (uint32_t)b.x];
+                    xa   = max(lo.x, b.x << kBrickX);
+                    xb   = min(hi.x, b.x << kBrickX | 7);
+                    ya   = max(lo.y, b.y << kBrickY);
+                    yb   = min(hi.y, b.y << kBrickY | 3);
+                    cy   = ya;
+                    cz   = max(lo.z, b.z << kBrickZ);
+                    zb   = slot == kNoBrick ? -1 : min(hi.z, b.z << kBrickZ | 3);
+                }
+            }
             if (result != kStateUndecided) __atomic_store_n(&state[i], result, __ATOMIC_RELAXED);
             pending = result == kStateUndecided;
         }
@@ -1075,7 +1129,7 @@ void launch_knn_first_grid(const float4* position, int n, const KnnGrid& box, Kn
 // 3 M in a volume, whole call: 2.0: 1365, 786 us; 1.5: 1264, 574; 1.2: 1283, 1015).  Where the samples are taken in every
 // s-th point, their nearest neighbour there stands in for the s-th in the cloud, and d_R = d_s (R / s)^(1 / D) for a cloud of
 // dimension D.  D = 2.5 is 32 % above a surface's value at R = 1, s = 16 and 17 % below a volume's, and cells too small by
-// that much leave a tenth of a volume's points unsettled; the distance to the nearest neighbour also spreads more about its
+// that much leave a seventh of a volume's points unsettled; the distance to the nearest neighbour also spreads more about its
 // median than that to the 8th.  R + 1.25 in the place of R takes care of both where it matters and costs surfaces nothing
 // (6 M points in a volume, rank 1 / 2 / 4 / 8: with R 2.03, 1.87, 1.35, 1.30 ms,
 // with R + 1.25 1.05, 1.06, 1.13, 1.36; 10 M points on patches 2.07 and 2.08).

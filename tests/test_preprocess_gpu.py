@@ -185,6 +185,34 @@ def test_remove_close_points_equals_the_sequential_sweep(name):
         assert want.sum() == 1
 
 
+@pytest.mark.parametrize("largest", [0.004, 0.03, 0.1, 0.4, float("inf")])
+@pytest.mark.parametrize("kind", ["volume", "surface", "crowded"])
+def test_remove_close_points_with_balls_of_many_cells(kind, largest):
+    """Radii from a hundredth of a cell of the search grid to the whole cloud: balls inside a brick, across bricks along every
+    axis, spanning bricks whole, and out of the grid on every side; crowded: 300 points in one cell."""
+    import torch
+    import oracle.preprocess as op
+    from adop_amd import preprocess
+
+    n = 5000
+    g = np.random.default_rng(31)
+    p = np.zeros((n, 4), np.float32)
+    p[:, :3] = g.random((n, 3)) - 0.5
+    if kind == "surface":
+        p[:, 1] = 0.25
+    if kind == "crowded":
+        p[::16, :3] = g.random((len(p[::16]), 3)) * 1e-3
+    radius = (g.uniform(0.0, 1.0, n) ** 4 * min(largest, 0.4)).astype(np.float32)
+    radius[g.choice(n, 20, replace=False)] = largest
+    announce(f"close points, {kind}, radii up to {largest}")
+    cam = torch.from_numpy(1.0 / np.maximum(radius, 1e-30)).cuda()
+    used = (1.0 / cam).float().cpu().numpy()
+    got = preprocess.RemoveClosePoints(torch.from_numpy(p).cuda(), cam, dis_th=1.0).cpu().numpy()
+    want = op.remove_close_points(p, used)
+    assert np.array_equal(got, want), int((got != want).sum())
+    assert 0 < want.sum() < n or largest < 0.01  # (radii that small take points of the crowded cloud only)
+
+
 def test_remove_lonely_points():
     import torch
     import oracle.preprocess as op
