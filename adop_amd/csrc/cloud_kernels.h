@@ -75,18 +75,37 @@ __global__ __launch_bounds__(kBlock) void box_partial_kernel(const float4* __res
     box_of_block(box, partial + 6 * (size_t)blockIdx.x);
 }
 
+// out[0..5]: the box; out[6..11]: the mean of the partial boxes.  A far outlier stretches the box but only one of the partial
+// ones: the two together say whether the box stands for the cloud.
 __global__ __launch_bounds__(kBlock) void box_final_kernel(const float* __restrict__ partial, int blocks,
                                                            float* __restrict__ out)
 {
-    Box6 box = empty_box();
+    __shared__ float s_sum[kBlock / 64][6];
+    Box6 box     = empty_box();
+    float sum[6] = {0, 0, 0, 0, 0, 0};
     for (int i = threadIdx.x; i < blocks; i += kBlock)
 #pragma unroll
         for (int k = 0; k < 3; ++k)
         {
-            box.lo[k] = min_nan(box.lo[k], partial[6 * i + k]);
-            box.hi[k] = max_nan(box.hi[k], partial[6 * i + 3 + k]);
+            const float lo = partial[6 * i + k], hi = partial[6 * i + 3 + k];
+            box.lo[k] = min_nan(box.lo[k], lo);
+            box.hi[k] = max_nan(box.hi[k], hi);
+            sum[k] += lo;
+            sum[3 + k] += hi;
         }
-    box_of_block(box, out);
+#pragma unroll
+    for (int k = 0; k < 6; ++k)
+    {
+        sum[k] = wave_sum(sum[k]);
+        if ((threadIdx.x & 63) == 0) s_sum[threadIdx.x >> 6][k] = sum[k];
+    }
+    box_of_block(box, out);  // (its barrier is behind s_sum too)
+    if (threadIdx.x < 6)
+    {
+        float all = 0.f;
+        for (int w = 0; w < kBlock / 64; ++w) all += s_sum[w][threadIdx.x];
+        out[6 + threadIdx.x] = all / (float)blocks;
+    }
 }
 
 // ---- permutations -----------------------------------------------------------------------------------------------
@@ -253,14 +272,14 @@ __global__ __launch_bounds__(kBlock) void radius_blocks_kernel(const float4* __r
 // ------------------------------------------------------------------------------------------------
 // launchers
 // ------------------------------------------------------------------------------------------------
-size_t bounding_box_floats() { return 6 * (size_t)(kBoxBlocks + 1); }
+size_t bounding_box_floats() { return 6 * (size_t)(kBoxBlocks + 2); }
 
 void launch_bounding_box(const float4* position, int n, float* box, hipStream_t st)
 {
     const int want   = (n + kBlock * 4 - 1) / (kBlock * 4);
     const int blocks = want < 1 ? 1 : (want < kBoxBlocks ? want : kBoxBlocks);
-    hipLaunchKernelGGL(box_partial_kernel, dim3(blocks), dim3(kBlock), 0, st, position, n, box + 6);
-    hipLaunchKernelGGL(box_final_kernel, dim3(1), dim3(kBlock), 0, st, box + 6, blocks, box);
+    hipLaunchKernelGGL(box_partial_kernel, dim3(blocks), dim3(kBlock), 0, st, position, n, box + 12);
+    hipLaunchKernelGGL(box_final_kernel, dim3(1), dim3(kBlock), 0, st, box + 12, blocks, box);
 }
 
 static int gather_blocks(int n) { return (int)(((size_t)n + kBlock * kGatherPer - 1) / (kBlock * kGatherPer)); }

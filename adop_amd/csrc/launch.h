@@ -59,7 +59,7 @@ void launch_camera_distance_sorted(const float4* sorted, int n, const ViewConst*
                                    hipStream_t st);
 void launch_close_points(const KnnView& view, int n, const float* radius, int32_t* state, uint32_t* round_count, int round,
                          hipStream_t st);
-size_t bounding_box_floats();  // the box and the partial boxes behind it
+size_t bounding_box_floats();  // the box, the mean partial box and the partial boxes
 void launch_bounding_box(const float4* position, int n, float* box, hipStream_t st);
 void launch_gather_rows(const float4* src, int rows, const long long* index, int n, float4* dst, hipStream_t st);
 void launch_shuffle_gather(const float4* position, const int32_t* normal, const long long* order, const long long* perm,

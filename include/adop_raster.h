@@ -366,7 +366,8 @@ adop_status adop_morton_ties(const int32_t* sorted_keys, int64_t* order, const u
 
 /* The passes of SceneData's initial processing (SceneData.cpp:101-104) that move the cloud.
  * adop_bounding_box: box [adop_bounding_box_size() bytes, device] starts with min x, y, z, max x, y, z (not a number on an
- * axis where a coordinate is not), scratch behind them.
+ * axis where a coordinate is not), then the mean of the same six over up to 2048 parts of the cloud that lie all over it (a far
+ * outlier stretches the box and one part's, hardly the mean), scratch behind them.
  * adop_gather_points: out_position[i] = position[index[i]], rows of 4 floats; an index that names no point gives zeros.
  * adop_shuffle_points: the cloud along `order` (a permutation of its N points) with its blocks of block_size points
  * shuffled (RandomBlockShuffle, :102): point i of the result is point order[block_order[i / block_size] * block_size +

@@ -447,4 +447,49 @@ def test_morton_order_from_short_keys(kind, n):
     dev = torch.from_numpy(np.ascontiguousarray(p)).cuda()
     box = pp._bbox(dev)
     want = torch.sort(pp._morton_codes(dev, box), stable=True).indices
-    assert torch.equal(pp._morton_order(dev, box, key_sort_from=1)(), want)
+    assert torch.equal(pp._morton_order(dev, box, by_keys=True)(), want)
+
+
+@pytest.mark.parametrize("n", [3, 1024, 300_001])
+def test_bounding_box_of_the_parts(n):
+    """How far the box exceeds that of a part: little for clouds that fill it, stored in any order, much where one point
+    lies far out; the route of the Morton order is taken by it."""
+    import torch
+    from adop_amd import preprocess as pp
+
+    announce(f"bounding box and its stretch, N={n}")
+    g = torch.Generator(device="cuda").manual_seed(n)
+    p = torch.rand(n, 4, generator=g, device="cuda")
+    assert 1.0 <= pp._box_and_stretch(p)[1] < 1.01 + 4000.0 / n
+    sorted_by_x = p[torch.argsort(p[:, 0])].contiguous()
+    box, stretch = pp._box_and_stretch(sorted_by_x)
+    assert stretch < pp._KEY_SORT_STRETCH
+    assert np.array_equal(np.float32(list(box[0]) + list(box[1])), torch.cat([p.amin(0)[:3], p.amax(0)[:3]]).cpu().numpy())
+    p[n // 2, 1] = -3.0e4
+    assert pp._box_and_stretch(p)[1] > pp._KEY_SORT_STRETCH or n <= 1024  # (one part: its box is the box)
+    assert pp._sorts_by_keys(1 << 20, 1.0) and pp._sorts_by_keys(1 << 24, 4.0)
+    assert not pp._sorts_by_keys((1 << 20) - 1, 1.0) and not pp._sorts_by_keys((1 << 24) + 1, 1.0)
+    assert not pp._sorts_by_keys(1 << 22, 4.01)
+
+
+@pytest.mark.parametrize("kind", ["volume", "outlier", "tails"])
+def test_preparation_of_a_large_cloud_by_either_sort(kind):
+    """From 2^20 points on the order comes from keys or from whole codes: the same either way."""
+    import torch
+    from adop_amd import preprocess as pp
+
+    n = (1 << 20) + 5
+    announce(f"PreprocessPointCloud, {kind}, N={n}")
+    g = torch.Generator(device="cuda").manual_seed(8)
+    p = torch.rand(n, 4, generator=g, device="cuda")
+    if kind == "outlier":
+        p[77, :3] = 5.0e3
+    if kind == "tails":
+        p[:, :3] = torch.empty(n, 3, device="cuda").cauchy_(generator=g)
+    box, stretch = pp._box_and_stretch(p)
+    assert pp._sorts_by_keys(n, stretch) == (kind == "volume"), stretch
+    order = pp.PreprocessPointCloud(p, None, seed=7)[3]
+    want = pp.ReorderMorton64(p)[pp.RandomBlockShuffle(n, 256, torch.Generator().manual_seed(7))]
+    whole = n // 256 * 256
+    assert torch.equal(order[:whole].reshape(-1, 256).sort(1).values, want[:whole].reshape(-1, 256).sort(1).values)
+    assert torch.equal(order[whole:], want[whole:])

@@ -23,9 +23,9 @@ def stub(monkeypatch):
     lib = _Recorder()
     monkeypatch.setattr(_capi, "load_library", lambda: lib)
     monkeypatch.setattr(pp, "_checked_position", lambda p: p.contiguous())
-    monkeypatch.setattr(pp, "_bbox", lambda p: (None, None))
+    monkeypatch.setattr(pp, "_box_and_stretch", lambda p: ((None, None), 1.0))
     monkeypatch.setattr(pp, "_stream_ptr", lambda: None)
-    monkeypatch.setattr(pp, "_morton_order", lambda p, box: lambda: torch.arange(p.shape[0]))
+    monkeypatch.setattr(pp, "_morton_order", lambda p, box, by_keys: lambda: torch.arange(p.shape[0]))
     monkeypatch.setattr(pp, "_knn_distance", lambda p, *a: torch.zeros(p.shape[0]))
     return lib
 
