@@ -226,6 +226,13 @@ int main()
         EXPECT(adop_point_distance_to_camera_static(&s, v.data(), 40, nullptr, nullptr) == ADOP_INVALID_ARG, "no output buffer");
         std::vector<adop_view> lots = make_views(1025, 64, 64, ADOP_CAMERA_PINHOLE_DISTORTION);
         EXPECT(adop_point_distance_to_camera_static(&s, lots.data(), 1025, (float*)fake(97), nullptr) == ADOP_INVALID_ARG, "1025 frames for the static scratch array");
+        EXPECT(adop_point_distance_to_camera_grid(&s, v.data(), 40, (float*)fake(97), fake(92), (size_t)1 << 40, fake(93), 1024, nullptr) == ADOP_WORKSPACE_TOO_SMALL, "camera distances from a search workspace of 1 KB");
+        EXPECT(adop_bounding_box((const float*)fake(1), INT_MIN, (float*)fake(91), nullptr) == ADOP_INVALID_ARG, "bounding box of INT_MIN points");
+        EXPECT(adop_gather_points((const float*)fake(1), INT_MAX, (const int64_t*)fake(91), INT_MIN, (float*)fake(92), nullptr) == ADOP_INVALID_ARG, "gather of INT_MIN points");
+        EXPECT(adop_shuffle_points((const float*)fake(1), nullptr, (const int64_t*)fake(91), (const int64_t*)fake(92), INT_MAX, INT_MIN, (float*)fake(93), nullptr, (int32_t*)fake(94), nullptr) == ADOP_INVALID_ARG, "shuffle in blocks of INT_MIN");
+        EXPECT(adop_radius_blocks((const float*)fake(1), nullptr, (const int32_t*)fake(91), (const float*)fake(92), (const double*)fake(93), INT_MIN, (float*)fake(94), nullptr, (float*)fake(95), (int64_t*)fake(96), nullptr) == ADOP_INVALID_ARG, "radii of INT_MIN points");
+        EXPECT(adop_morton_keys((const float*)fake(1), 1000, nan_lo, box_hi, (uint64_t*)fake(93), (int32_t*)fake(94), nullptr) == ADOP_INVALID_ARG, "short keys in a bounding box with a NaN corner");
+        EXPECT(adop_morton_ties((const int32_t*)fake(1), (int64_t*)fake(91), (const uint64_t*)fake(92), INT_MIN, (int32_t*)fake(93), nullptr) == ADOP_INVALID_ARG, "ties of INT_MIN points");
         EXPECT(adop_apply_tangent(nullptr, nullptr, 5, nullptr) == ADOP_INVALID_ARG, "ApplyTangent without buffers");
         EXPECT(adop_apply_tangent((double*)fake(98), (double*)fake(99), 0, nullptr) == ADOP_OK, "ApplyTangent of no poses");
     }

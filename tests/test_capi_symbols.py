@@ -176,3 +176,57 @@ def test_preprocessing_entry_points_reject_bad_arguments_before_any_launch():
     s.intrinsics_cols = 10
     views[0].camera_model_type = _capi.CAMERA_PINHOLE_DISTORTION
     assert lib.adop_point_distance_to_camera(C.byref(s), views, 1, fake, fake, big, None) != 0 and "13 columns" in message()
+
+
+def test_whole_cloud_entry_points_reject_bad_arguments_before_any_launch():
+    """The entry points that move whole clouds, the short Morton keys and the camera distances in grid order."""
+    lib = _capi.load_library()
+    lo, hi = (C.c_float * 3)(0, 0, 0), (C.c_float * 3)(1, 1, 1)
+    nan_hi, inf_hi = (C.c_float * 3)(1, float("nan"), 1), (C.c_float * 3)(1, 1, float("inf"))
+    p = C.c_void_p(256)  # never dereferenced: every call below fails its checks first, or has nothing to do
+    INVALID, TOO_SMALL = _capi.ADOP_INVALID_ARG, _capi.ADOP_WORKSPACE_TOO_SMALL
+
+    assert lib.adop_bounding_box_size() >= 12 * 4
+    assert lib.adop_bounding_box(None, 10, p, None) == INVALID and lib.adop_bounding_box(p, 10, None, None) == INVALID
+    for n in (0, -1):
+        assert lib.adop_bounding_box(p, n, p, None) == INVALID
+
+    for args in ((None, 10, p, 10, p), (p, 10, None, 10, p), (p, 10, p, 10, None), (p, -1, p, 10, p), (p, 10, p, -1, p)):
+        assert lib.adop_gather_points(*args, None) == INVALID, args
+    assert lib.adop_gather_points(p, 10, p, 0, p, None) == _capi.ADOP_OK  # nothing to gather
+
+    good = [p, p, p, p, 1000, 256, p, p, p]  # position, normal, order, block_order, n, block, out_position, out_normal, out_id
+    for k, bad in ((0, None), (1, None), (2, None), (3, None), (4, 0), (4, -5), (5, 0), (5, -256), (6, None), (7, None), (8, None)):
+        args = list(good)
+        args[k] = bad
+        assert lib.adop_shuffle_points(*args, None) == INVALID, (k, bad)  # (a normal without its output is refused too)
+
+    good = [p, p, p, p, p, 1000, p, p, p, p]  # position, normal, id, distance, uniform, n, four outputs
+    for k, bad in ((0, None), (1, None), (2, None), (3, None), (4, None), (5, 0), (5, -1), (6, None), (7, None), (8, None), (9, None)):
+        args = list(good)
+        args[k] = bad
+        assert lib.adop_radius_blocks(*args, None) == INVALID, (k, bad)
+
+    for args in ((None, 10, lo, hi, p, p), (p, 10, None, hi, p, p), (p, 10, lo, None, p, p), (p, 10, lo, hi, None, p),
+                 (p, 10, lo, hi, p, None), (p, -1, lo, hi, p, p), (p, 10, lo, nan_hi, p, p), (p, 10, lo, inf_hi, p, p),
+                 (p, 10, hi, lo, p, p)):
+        assert lib.adop_morton_keys(*args, None) == INVALID
+    assert lib.adop_morton_keys(p, 0, lo, hi, p, p, None) == _capi.ADOP_OK
+    for args in ((None, p, p, 10, p), (p, None, p, 10, p), (p, p, None, 10, p), (p, p, p, 10, None), (p, p, p, -1, p)):
+        assert lib.adop_morton_ties(*args, None) == INVALID, args
+
+    s = _capi.Scene()
+    s.position, s.num_points = 256, 1000
+    s.poses_se3, s.num_poses, s.intrinsics, s.num_cameras, s.intrinsics_cols = 256, 2, 256, 1, 13
+    v = (_capi.View * 1)()
+    v[0].w, v[0].h, v[0].camera_model_type = 64, 48, _capi.CAMERA_PINHOLE_DISTORTION
+    frames, knn = lib.adop_frames_workspace_size(1), lib.adop_knn_workspace_size(1000)
+
+    def grid(frames_ws=p, frames_bytes=frames, knn_ws=p, knn_bytes=knn, out=p, count=1):
+        return lib.adop_point_distance_to_camera_grid(C.byref(s), v, count, out, frames_ws, frames_bytes, knn_ws, knn_bytes, None)
+
+    assert grid(frames_ws=None) == TOO_SMALL and grid(frames_bytes=frames - 1) == TOO_SMALL
+    assert grid(knn_ws=None) == TOO_SMALL and grid(knn_bytes=knn - 1) == TOO_SMALL
+    assert grid(out=None) == INVALID and grid(count=0) == INVALID
+    s.num_points = 0
+    assert grid() == INVALID
