@@ -47,8 +47,9 @@ __device__ __forceinline__ void entry_tiles(const Levels& lv, const ParamArg& rp
         {
             if (rp.drop_by_radius && radius_pixels < rp.drop_threshold) alive = false;  // break, :261-264
             if (alive) *nlev = l + 1;
-            // (levels are not nested, but nearly all points of the image are in it at level 0: the pixels of the levels from
-            // 2 on are computed only where a lane of the wavefront needs them, or all of them are counted)
+            // (levels are not nested, but nearly all points of the image are in it at level 0: the pixels of the
+            // levels from 2 on are computed only where a lane of the wavefront needs them, or all of them are
+            // counted)
             if (l == 2) rest = in_out != nullptr || __ballot(alive && !*any_in) != 0;
             if (l < 2 || rest)
             {
@@ -82,15 +83,17 @@ __device__ __forceinline__ uint32_t shard_of(uint32_t point, int shard_shift)
 }
 
 // First pass over the points: projection (kept in the point cache) and the number of entries per tile.  A thread
-// handles PPT points whose loads are all issued before anything waits.
-// Scalar registers decide the number of its instructions: what does not fit them is parked in lanes of vector registers, one
-// v_writelane / v_readlane per value, and they count against the vector issue this kernel is bound by.  Hence the counter
-// pass as a variant of its own, the projections of all points before the first of them is binned (the view's constants are
-// done with then) and up to 96 scalar registers, which 8 wavefronts per SIMD allow (the compiler stops at 80 when it is asked for 8
+// handles PPT points whose loads are all issued before anything waits. Scalar registers decide the number of its
+// instructions: what does not fit them is parked in lanes of vector registers, one v_writelane / v_readlane per
+// value, and they count against the vector issue this kernel is bound by.  Hence the counter pass as a variant of its
+// own, the projections of all points before the first of them is binned (the view's constants are done with then) and
+// up to 96 scalar registers, which 8 wavefronts per SIMD allow (the compiler stops at 80 when it is asked for 8
 // wavefronts): 1462 vector and 1132 scalar instructions, 197 of them parking, become 1215, 773 and 44.  16 crops of
 // 10 M points: 356 -> 305 us; one view of 12 M: 85 -> 80 us.
 template <int PPT, bool STATS>
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(PPT > 2 ? 5 : 7, PPT > 2 ? 5 : 8), amdgpu_num_sgpr(96))) void bin_count_kernel(CloudArg pc, const ViewConst* __restrict__ views, Levels lv,
+__global__ __launch_bounds__(kBlock)
+__attribute__((amdgpu_waves_per_eu(PPT > 2 ? 5 : 7, PPT > 2 ? 5 : 8), amdgpu_num_sgpr(96)))
+void bin_count_kernel(CloudArg pc, const ViewConst* __restrict__ views, Levels lv,
                                                            ParamArg rp, BinArg bin, adop_stats* stats)
 {
     const int lane   = threadIdx.x & 63;
@@ -135,8 +138,8 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(PPT > 2 
                 frame_p[k] = {0.f, 0.f};
                 frame_z[k] = 0.f;
                 if (base + k * kBlock < pc.n)
-                    project_frame<true>(vc, pc.intrinsics, pos, nrm, rp.check_normal != 0, rp.dist_cutoff, &frame_p[k], &frame_z[k],
-                                  &view_p);
+                    project_frame<true>(vc, pc.intrinsics, pos, nrm, rp.check_normal != 0, rp.dist_cutoff, &frame_p[k],
+                                        &frame_z[k], &view_p);
             }
         }
 #pragma unroll
@@ -227,13 +230,13 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(PPT > 2 
 }
 
 // The order in which the tile kernels take the tiles: order[i] = (tile, first entry, end, 0), the fullest bins first.
-// The bins of a view differ by two orders of magnitude (a surface seen at a grazing angle beside empty sky), a tile is one
-// workgroup from its first entry to its last, and the hardware starts workgroups in the order of their index: with the
-// tiles in image order a full bin may start late and run on alone (config 3: tile_blend_kernel 129 -> 102 us).
-// Computed by the first order_groups(T) workgroups of the bin_scatter launch, beside the scatter (nothing waits for it
-// before the tile kernels): workgroup g classes the tiles g, g + G, g + 2G, ... by entries / 128 (classes of equal cost
-// in batches of the tile kernels) and puts the r-th of them, fullest class first, at order[g + G * r].  Inside a class the
-// order is whatever the LDS atomics make it, which changes no result.
+// The bins of a view differ by two orders of magnitude (a surface seen at a grazing angle beside empty sky), a tile
+// is one workgroup from its first entry to its last, and the hardware starts workgroups in the order of their index:
+// with the tiles in image order a full bin may start late and run on alone (config 3: tile_blend_kernel 129 -> 102
+// us). Computed by the first order_groups(T) workgroups of the bin_scatter launch, beside the scatter (nothing waits
+// for it before the tile kernels): workgroup g classes the tiles g, g + G, g + 2G, ... by entries / 128 (classes of
+// equal cost in batches of the tile kernels) and puts the r-th of them, fullest class first, at order[g + G * r].
+// Inside a class the order is whatever the LDS atomics make it, which changes no result.
 constexpr int kOrderClasses       = 64;
 constexpr int kOrderTilesPerGroup = 1024;
 

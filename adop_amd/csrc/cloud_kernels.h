@@ -1,7 +1,8 @@
-// cloud_kernels.h — (part of preprocess_kernels.hip) moving whole clouds: bounding box, permutations of the points, radii and order of the 256-point
-// blocks (gfx950).  The counterpart of the loops of SceneData.cpp:101-104 and :441-484, 671-684 that touch every point
-// once; what they compute per point is next to nothing, so these kernels are bound by memory: random 64-byte lines where
-// they gather, the bandwidth of a copy where they do not.
+// cloud_kernels.h — included by preprocess_kernels.hip alone: moving whole clouds (gfx950): bounding box,
+// permutations of the points, radii and order of the 256-point blocks.  The counterpart of the loops of
+// SceneData.cpp:101-104 and :441-484, 671-684 that touch every point once; what they compute per point is next to
+// nothing, so these kernels are bound by memory: random 64-byte lines where they gather, the bandwidth of a copy
+// where they do not.
 #pragma once
 #include "common.h"
 #include "launch.h"
@@ -75,8 +76,8 @@ __global__ __launch_bounds__(kBlock) void box_partial_kernel(const float4* __res
     box_of_block(box, partial + 6 * (size_t)blockIdx.x);
 }
 
-// out[0..5]: the box; out[6..11]: the mean of the partial boxes.  A far outlier stretches the box but only one of the partial
-// ones: the two together say whether the box stands for the cloud.
+// out[0..5]: the box; out[6..11]: the mean of the partial boxes.  A far outlier stretches the box but only one of the
+// partial ones: the two together say whether the box stands for the cloud.
 __global__ __launch_bounds__(kBlock) void box_final_kernel(const float* __restrict__ partial, int blocks,
                                                            float* __restrict__ out)
 {
@@ -111,7 +112,8 @@ __global__ __launch_bounds__(kBlock) void box_final_kernel(const float* __restri
 // ---- permutations -----------------------------------------------------------------------------------------------
 // One row of 16 bytes per lane, four rows per thread: all index loads, then all gathers are in flight before anything
 // waits.  What bounds it is the number of 64-byte lines the random rows touch: 10 M random rows take 0.3 ms, where
-// torch's gather of the same rows, one row per wavefront's share of 16 bytes, takes 2.1 ms.  An index that names no row gives zeros.
+// torch's gather of the same rows, one row per wavefront's share of 16 bytes, takes 2.1 ms.  An index that names no
+// row gives zeros.
 constexpr int kGatherPer = 4;
 
 __global__ __launch_bounds__(kBlock) void gather_rows_kernel(const float4* __restrict__ src, int rows,
@@ -198,11 +200,11 @@ __global__ __launch_bounds__(kBlock) void shuffle_gather_kernel(const float4* __
 
 // ---- radii and the order inside the blocks ----------------------------------------------------------------------
 // ComputeRadius (SceneData.cpp:462-483) from the neighbour distance and the uniform number of every point, then
-// SortBlocksByRadius (:671-684) for blocks of kBlock points, one workgroup each: the (radius, slot) keys of a block are
-// sorted in registers, 33 of the 36 steps of the bitonic network between lanes of a wavefront, 3 through LDS, and the
-// rows of the block are written in that order.  10 M points: 146 us for 840 MB, 5.8 TB/s, in place of a segmented sort
-// (464 us), two gathers and eight elementwise passes.  The slot in the low word makes the sort stable; a radius that is not a
-// number comes last.  The points behind the last whole block keep their order.
+// SortBlocksByRadius (:671-684) for blocks of kBlock points, one workgroup each: the (radius, slot) keys of a block
+// are sorted in registers, 33 of the 36 steps of the bitonic network between lanes of a wavefront, 3 through LDS, and
+// the rows of the block are written in that order.  10 M points: 146 us for 840 MB, 5.8 TB/s, in place of a segmented
+// sort (464 us), two gathers and eight elementwise passes.  The slot in the low word makes the sort stable; a radius
+// that is not a number comes last.  The points behind the last whole block keep their order.
 __global__ __launch_bounds__(kBlock) void radius_blocks_kernel(const float4* __restrict__ position,
                                                                const int32_t* __restrict__ normal,
                                                                const int32_t* __restrict__ id,

@@ -324,18 +324,18 @@ __device__ __forceinline__ V3 ocam_unproject(const float* aff, const float* poly
     return {cxn * cs, cyn * cs, -sn};
 }
 
-// Head of the three reference point kernels (PointRenderer.cu:227-256, 334-359, 409-438), in two parts.
-// First part, the same for every crop of one frame (pose and camera model): ProjectPointPinhole / ProjectPointOcam
-// (PointRendererHelper.h:49-106) up to the point in the uncropped image.  Returns false when the point is culled
-// (z == 0).
+// Head of the three reference point kernels (PointRenderer.cu:227-256, 334-359, 409-438), in two parts. First part,
+// the same for every crop of one frame (pose and camera model): ProjectPointPinhole / ProjectPointOcam
+// (PointRendererHelper.h:49-106) up to the point in the uncropped image.  Returns false when the point is culled (z
+// == 0).
 //
-// FACE_FIRST: the back-face test (dot(V p, V n) > 0, PointRendererHelper.h:60-66, 103) by its sign in world coordinates,
-// dot(p - c, n), before anything else, where that is beyond doubt: the rounding of both forms is below 3e-6 of
-// (|p| + |c|) |n|, |n|^2 <= 3.  Only the points between take the form of the reference with its second rotation.  For a
-// kernel that is bound by its vector instructions: wavefronts of Morton-ordered points are mostly culled as a whole.
-// First binning pass, before / after: 8 fisheye views of 20 M points 1184 / 908 us, 16 pinhole crops of 10 M 300 / 294.
-// Not for the prepass, which waits for its early-z reads and atomics: 2.8 M unordered points on 416 x 151 pixels, fisheye,
-// 310 us without, 377 with it; 1.4 M points without normals 77 / 86.
+// FACE_FIRST: the back-face test (dot(V p, V n) > 0, PointRendererHelper.h:60-66, 103) by its sign in world
+// coordinates, dot(p - c, n), before anything else, where that is beyond doubt: the rounding of both forms is below
+// 3e-6 of (|p| + |c|) |n|, |n|^2 <= 3.  Only the points between take the form of the reference with its second
+// rotation.  For a kernel that is bound by its vector instructions: wavefronts of Morton-ordered points are mostly
+// culled as a whole. First binning pass, before / after: 8 fisheye views of 20 M points 1184 / 908 us, 16 pinhole
+// crops of 10 M 300 / 294. Not for the prepass, which waits for its early-z reads and atomics: 2.8 M unordered points
+// on 416 x 151 pixels, fisheye, 310 us without, 377 with it; 1.4 M points without normals 77 / 86.
 template <bool FACE_FIRST = false>
 __device__ __forceinline__ bool project_frame(const ViewConst& vc, const float* __restrict__ intrinsics, V3 pos, V3 nrm,
                                               bool check_normal, float dist_cutoff, V2* image_p_out, float* z_out,

@@ -143,8 +143,8 @@ __device__ __forceinline__ EnvTileOf env_tile_of_block(const Levels& lv, const E
     return e;
 }
 
-// The constants of the workgroup's view and level, computed by one thread (poses_se3 is f64, the intrinsics row up to 24
-// floats: 256 threads each doing this for themselves cost more than the sampling).
+// The constants of the workgroup's view and level, computed by one thread (poses_se3 is f64, the intrinsics row up to
+// 24 floats: 256 threads each doing this for themselves cost more than the sampling).
 __device__ __forceinline__ const EnvView& env_view_const(EnvView* s_v, const ViewChunk& chunk, int b, int level,
                                                          const double* __restrict__ poses,
                                                          const float* __restrict__ intrinsics, int cols)
@@ -154,12 +154,13 @@ __device__ __forceinline__ const EnvView& env_view_const(EnvView* s_v, const Vie
     return *s_v;
 }
 
-// CT: channels as a constant (0: lv.C).  A workgroup waits once for the constants of its view, which one thread computes; the
-// mask is requested beforehand, the channels of a pixel are read together, and a wavefront lies in one row of the image, so
-// that what it reads and writes of a channel are whole lines.  Tiles of 16 x 16 pixels / of 64 x 16 with four pixels per
-// thread / of 64 x 4 (taken), fp32: 8 fisheye views of 2200 x 1500 1042 / 910 / 859 us (most of it the divisions and square
-// roots of the rays), one 127 / 117 / 108, a view of 1365 x 911 42 / 38 / 36, with 8 channels 89 / 90 / 58, of 457 x 162
-// (fisheye) 13 / 29 / 11: four pixels per thread leave a small image with fewer workgroups than the GPU has CUs.
+// CT: channels as a constant (0: lv.C).  A workgroup waits once for the constants of its view, which one thread
+// computes; the mask is requested beforehand, the channels of a pixel are read together, and a wavefront lies in one
+// row of the image, so that what it reads and writes of a channel are whole lines.  Tiles of 16 x 16 pixels / of 64 x
+// 16 with four pixels per thread / of 64 x 4 (taken), fp32: 8 fisheye views of 2200 x 1500 1042 / 910 / 859 us (most
+// of it the divisions and square roots of the rays), one 127 / 117 / 108, a view of 1365 x 911 42 / 38 / 36, with 8
+// channels 89 / 90 / 58, of 457 x 162 (fisheye) 13 / 29 / 11: four pixels per thread leave a small image with fewer
+// workgroups than the GPU has CUs.
 template <int CT>
 __global__ __launch_bounds__(kBlock) void env_sample_kernel(ViewChunk chunk, const double* __restrict__ poses,
                                                             const float* __restrict__ intrinsics, Levels lv,
@@ -319,7 +320,8 @@ __global__ __launch_bounds__(kBlock) void env_backward_kernel(ViewChunk chunk, c
     }
     __syncthreads();
     if (s_box[1] < 0) return;  // no empty pixel in the tile (workgroup-uniform)
-    // the narrower of the two windows; window column tx is texel column (bx + tx) (- half, modulo the width, if shifted)
+    // the narrower of the two windows; window column tx is texel column (bx + tx) (- half, modulo the width, if
+    // shifted)
     const bool shifted = s_box[5] - s_box[4] < s_box[3] - s_box[2];
     const int by = s_box[0], bx = shifted ? s_box[4] : s_box[2];
     const int bw = (shifted ? s_box[5] : s_box[3]) - bx + 2, bh = s_box[1] - by + 2;  // the taps reach one texel further

@@ -66,15 +66,15 @@ __global__ __launch_bounds__(kBlock) void clear_kernel(Levels lv, int first_leve
 }
 
 // DepthPrepassMulti (PointRenderer.cu:203-301) on the packed buffer the reference keeps as "old rendering"
-// (LayerCuda::depth_index_tensor, PackIndex): min over (depth bits << 32 | point id).
-// Every thread handles PPT points (all their loads are issued before anything waits: the kernel is bound by memory
-// latency, not by arithmetic).  Per level and 64-point run the lanes that survive the early-z read are grouped by
-// pixel, one lane per distinct pixel takes the minimum of its group from LDS and issues the 64-bit atomicMin:
-// clouds stored in Morton-ordered blocks collide heavily at the coarse levels, and a device-scope atomic costs one
-// memory transaction whatever it carries.
-// The counters are a branch at run time, not a variant as in the other kernels: with the shorter code of a variant more
-// wavefronts read a depth before the first of them has lowered it, and they issue redundant atomics (1.4 M points on a few
-// hundred pixels, fisheye: 255 us with the branch, 267 without; 100 M points on 1920 x 1080 do not differ).
+// (LayerCuda::depth_index_tensor, PackIndex): min over (depth bits << 32 | point id). Every thread handles PPT points
+// (all their loads are issued before anything waits: the kernel is bound by memory latency, not by arithmetic).  Per
+// level and 64-point run the lanes that survive the early-z read are grouped by pixel, one lane per distinct pixel
+// takes the minimum of its group from LDS and issues the 64-bit atomicMin: clouds stored in Morton-ordered blocks
+// collide heavily at the coarse levels, and a device-scope atomic costs one memory transaction whatever it carries.
+// The counters are a branch at run time, not a variant as in the other kernels: with the shorter code of a variant
+// more wavefronts read a depth before the first of them has lowered it, and they issue redundant atomics (1.4 M
+// points on a few hundred pixels, fisheye: 255 us with the branch, 267 without; 100 M points on 1920 x 1080 do not
+// differ).
 template <int PPT>
 __global__ __launch_bounds__(kBlock) void prepass_kernel(CloudArg pc, const ViewConst* __restrict__ views, Levels lv,
                                                          ParamArg rp, int group_from, adop_stats* stats, Gate gate)

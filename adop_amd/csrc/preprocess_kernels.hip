@@ -1,18 +1,18 @@
-// preprocess_kernels.hip — point-cloud preprocessing that decides how well the rasterizer runs (gfx950):
-// the distance of every point to its n-th nearest neighbour (SceneData::ComputeRadius, SceneData.cpp:441-484: a
-// kd-tree k-nearest-neighbour search per point on the host) and the Morton code of every point (the key of
-// ReorderMorton64, SceneData.cpp:101).
+// preprocess_kernels.hip — point-cloud preprocessing that decides how well the rasterizer runs (gfx950): the distance
+// of every point to its n-th nearest neighbour (SceneData::ComputeRadius, SceneData.cpp:441-484: a kd-tree
+// k-nearest-neighbour search per point on the host) and the Morton code of every point (the key of ReorderMorton64,
+// SceneData.cpp:101).
 //
-// Nearest neighbours: the points are put into the cells of a uniform grid, stored cell after cell, and every point then
-// walks the cube of cells around its own until the n-th best distance cannot be beaten from outside the cube.  The
-// distances are formed as sqrt((dx*dx + dy*dy) + dz*dz) in fp32; the result is the n-th smallest of them over all other
-// points, whatever the search order and whatever the grid, so a brute-force search over the same arithmetic gives the
-// same bits.
-// The cost is the number of candidates, which the cell size decides, and the right cell size depends on how the cloud
-// fills space (scans are surfaces: a grid sized by volume puts hundreds of points into the few cells that have any).
-// So the search grid is sized on the device (no host round trip) from the neighbour distances of 1024 sample points,
-// measured in a part of the cloud (every 16th point) on a coarse grid sized by volume.  The coarse grid over the whole cloud is
-// built only when the search grid leaves points undecided (sparse parts of the cloud), which the device finds out.
+// Nearest neighbours: the points are put into the cells of a uniform grid, stored cell after cell, and every point
+// then walks the cube of cells around its own until the n-th best distance cannot be beaten from outside the cube.
+// The distances are formed as sqrt((dx*dx + dy*dy) + dz*dz) in fp32; the result is the n-th smallest of them over all
+// other points, whatever the search order and whatever the grid, so a brute-force search over the same arithmetic
+// gives the same bits. The cost is the number of candidates, which the cell size decides, and the right cell size
+// depends on how the cloud fills space (scans are surfaces: a grid sized by volume puts hundreds of points into the
+// few cells that have any). So the search grid is sized on the device (no host round trip) from the neighbour
+// distances of 1024 sample points, measured in a part of the cloud (every 16th point) on a coarse grid sized by
+// volume.  The coarse grid over the whole cloud is built only when the search grid leaves points undecided (sparse
+// parts of the cloud), which the device finds out.
 #include "cloud_kernels.h"
 #include "common.h"
 #include "launch.h"
@@ -21,12 +21,12 @@
 
 namespace adop
 {
-// The search grid is stored in bricks of 8 x 4 x 4 cells: the points brick after brick and, inside a brick, cell after
-// cell with x fastest.  A cloud of 10 M points asks for 100 M cells and more, nearly all of them empty: the bricks are
-// counted in one dense table (a 128th of the cells) and only the bricks that hold points have a row in the table of the
-// cells' first points.  (A dense table of cells took 650 us to clear and sum up for 10 M points on 1000 patches, and
-// its 10 M atomics on single cells 720 us; the bricks and the sort inside them take 235 us in all.)  A wavefront of consecutive points stays inside a brick or two, and so do
-// the cells it searches.
+// The search grid is stored in bricks of 8 x 4 x 4 cells: the points brick after brick and, inside a brick, cell
+// after cell with x fastest.  A cloud of 10 M points asks for 100 M cells and more, nearly all of them empty: the
+// bricks are counted in one dense table (a 128th of the cells) and only the bricks that hold points have a row in the
+// table of the cells' first points.  (A dense table of cells took 650 us to clear and sum up for 10 M points on 1000
+// patches, and its 10 M atomics on single cells 720 us; the bricks and the sort inside them take 235 us in all.)  A
+// wavefront of consecutive points stays inside a brick or two, and so do the cells it searches.
 constexpr int kBrickX = 3, kBrickY = 2, kBrickZ = 2;  // log2 of the cells per brick
 static_assert(kBrickX + kBrickY + kBrickZ == 7 && (1 << 7) == kBrickCells, "128 cells");
 constexpr uint32_t kNoBrick = 0xFFFFFFFFu;
@@ -57,8 +57,8 @@ __device__ __forceinline__ uint32_t brick_local(int cx, int cy, int cz)
 }
 static_assert(kBrickY == 2 && kBrickZ == 2 && kBrickX == 3, "masks of brick_local");
 
-// The points [first, end) of the cells x0..x1 of row (cy, cz) that lie in the brick of x0 (part 0) or in the brick of x1
-// where that is another one (part 1; x1 - x0 < 8 cells, so there is no third).
+// The points [first, end) of the cells xa..xb of row (cy, cz) of the brick in `slot` (xa and xb lie in that brick; a
+// longer row is taken brick by brick).
 __device__ __forceinline__ void brick_range(const KnnView& k, uint32_t slot, int xa, int xb, int cy, int cz,
                                             uint32_t* first, uint32_t* end)
 {
@@ -96,7 +96,8 @@ __global__ __launch_bounds__(kBlock) void knn_count_kernel(const float4* __restr
     {
         const bool valid = base + k * kBlock < (size_t)n;
         const int3 c     = grid_cell(g, p[k].x, p[k].y, p[k].z);
-        const uint32_t b = !valid ? kNoBrick : (BRICKS ? brick_row(g, c.y, c.z) + (uint32_t)(c.x >> kBrickX) : grid_index(g, c.x, c.y, c.z));
+        uint32_t b       = kNoBrick;
+        if (valid) b = BRICKS ? brick_row(g, c.y, c.z) + (uint32_t)(c.x >> kBrickX) : grid_index(g, c.x, c.y, c.z);
         const uint32_t prev = (uint32_t)__shfl_up((int)b, 1, 64);
         const bool starts   = lane == 0 || prev != b;
         const unsigned long long heads = __ballot(starts);
@@ -161,9 +162,9 @@ __global__ __launch_bounds__(kBlock) void knn_clear_kernel(uint32_t* __restrict_
         __builtin_nontemporal_store(0u, count + i);
 }
 
-// Exclusive prefix sums over the bins in two launches: sums of chunks of 8192 bins, then the sums inside every chunk on top of
-// those of the chunks before it (at most 1024 chunks, which every workgroup sums up for itself).  BRICKS: the bins that
-// hold points are numbered in the same pass (slots), in the high half of a 64-bit sum.
+// Exclusive prefix sums over the bins in two launches: sums of chunks of 8192 bins, then the sums inside every chunk
+// on top of those of the chunks before it (at most 1024 chunks, which every workgroup sums up for itself).  BRICKS:
+// the bins that hold points are numbered in the same pass (slots), in the high half of a 64-bit sum.
 constexpr int kScanChunk  = 8192;
 constexpr int kScanChunks = 1024;
 
@@ -314,7 +315,8 @@ __global__ __launch_bounds__(kBlock) void knn_brick_sort_kernel(const float4* __
     const int lane      = threadIdx.x & 63;
     const KnnGrid g     = *gp;
     const uint32_t all  = *num_slots;
-    for (uint32_t s = blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6); s < all; s += gridDim.x * (kBlock / 64))  // wavefront-uniform
+    // (s is uniform over the wavefront)
+    for (uint32_t s = blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6); s < all; s += gridDim.x * (kBlock / 64))
     {
         const uint32_t b = slot_brick[s], first = start[b], num = count[b];
         wave_lds_sync();
@@ -488,8 +490,8 @@ __global__ __launch_bounds__(kBlock) void knn_search_kernel(KnnView kv, int n, f
     wave_push(t < n && !settled, (uint32_t)t, list, list_count);
 }
 
-// K-th smallest of the union of the lanes' ascending lists (destroys them): K rounds of taking the smallest head.  all != null
-// receives the K smallest.
+// K-th smallest of the union of the lanes' ascending lists (destroys them): K rounds of taking the smallest head.
+// all != null receives the K smallest.
 template <int K>
 __device__ __forceinline__ float wave_kth(float* best, float* all = nullptr)
 {
@@ -514,9 +516,10 @@ __device__ __forceinline__ float wave_kth(float* best, float* all = nullptr)
     return kth;
 }
 
-// Stage 2: the points stage 1 left, cubes of 2 and 3 shells of the same grid, one wavefront per point: the lanes share the
-// rows of the cube (a thread per point waits for 25 to 49 rows one after the other, and few points are left: 250 us for a
-// list that a wavefront per point works off in 15).  A larger cube is searched from scratch; the rest goes to list2.
+// Stage 2: the points stage 1 left, cubes of 2 and 3 shells of the same grid, one wavefront per point: the lanes
+// share the rows of the cube (a thread per point waits for 25 to 49 rows one after the other, and few points are
+// left: 250 us for a list that a wavefront per point works off in 15).  A larger cube is searched from scratch; the
+// rest goes to list2.
 template <int K>
 __global__ __launch_bounds__(kBlock) void knn_shells_kernel(KnnView kv, const uint32_t* __restrict__ list,
                                                             const uint32_t* __restrict__ list_count,
@@ -561,9 +564,9 @@ __global__ __launch_bounds__(kBlock) void knn_shells_kernel(KnnView kv, const ui
     }
 }
 
-// The K-th smallest squared distance of point p on the coarse grid: cubes of 1 to 4 shells, by one wavefront (every lane takes
-// its share of the candidates of a row and keeps the K best of them).  False: 4 shells do not settle it.  Uniform over the
-// wavefront.
+// The K-th smallest squared distance of point p on the coarse grid: cubes of 1 to 4 shells, by one wavefront (every
+// lane takes its share of the candidates of a row and keeps the K best of them).  False: 4 shells do not settle it.
+// Uniform over the wavefront.
 template <int K>
 __device__ __forceinline__ bool coarse_cubes(const float4 p, const KnnGrid& g, const float4* __restrict__ sorted,
                                              const uint32_t* __restrict__ start, float* kth)
@@ -588,8 +591,8 @@ __device__ __forceinline__ bool coarse_cubes(const float4 p, const KnnGrid& g, c
     return false;
 }
 
-// Stage 3: what is left (points in sparse parts of the cloud), on the coarse grid over all points, at most 4 shells, one
-// wavefront per point; the rest goes to list3.
+// Stage 3: what is left (points in sparse parts of the cloud), on the coarse grid over all points, at most 4 shells,
+// one wavefront per point; the rest goes to list3.
 template <int K>
 __global__ __launch_bounds__(kBlock) void knn_coarse_kernel(const float4* __restrict__ points,
                                                             const uint32_t* __restrict__ list,
@@ -616,13 +619,13 @@ __global__ __launch_bounds__(kBlock) void knn_coarse_kernel(const float4* __rest
     }
 }
 
-// Stage 4: stray points far from everything (no cube of a few shells of either grid settles them): one workgroup goes through
-// all points for one of them, or for kBruteStrays together where there are more strays than workgroups.  (A wavefront per
-// stray, 1 M points of a Gaussian cloud: 1.5 ms; a workgroup of 16: 0.25 ms - there are fewer strays than the GPU has
-// wavefronts.)  With thousands of strays the points come from the last cache over and over, 5 TB/s of them, so strays share
-// a pass; of the thousands of points a thread sees few get into its lists, so a round of kBruteRound points is looked at as a
-// whole before any of it goes in.  6 M points of a Gaussian cloud, rank 4 / 8 (some 1500 / 4000 strays): one stray per pass
-// 29.8 / 77.5 ms, four 6.2 / 14.3.
+// Stage 4: stray points far from everything (no cube of a few shells of either grid settles them): one workgroup goes
+// through all points for one of them, or for kBruteStrays together where there are more strays than workgroups.  (A
+// wavefront per stray, 1 M points of a Gaussian cloud: 1.5 ms; a workgroup of 16: 0.25 ms - there are fewer strays
+// than the GPU has wavefronts.)  With thousands of strays the points come from the last cache over and over, 5 TB/s
+// of them, so strays share a pass; of the thousands of points a thread sees few get into its lists, so a round of
+// kBruteRound points is looked at as a whole before any of it goes in.  6 M points of a Gaussian cloud, rank 4 / 8
+// (some 1500 / 4000 strays): one stray per pass 29.8 / 77.5 ms, four 6.2 / 14.3.
 constexpr int kBruteBlock  = 1024;
 constexpr int kBruteStrays = 4;
 constexpr int kBruteRound  = 4;
@@ -700,10 +703,10 @@ __global__ __launch_bounds__(kBruteBlock) void knn_brute_kernel(const float4* __
             brute_pass<K, kBruteStrays>(points, n, list, e, count, s_best, out);
 }
 
-// The neighbour distance of `samples` points evenly spaced in the order of the coarse grid, one wavefront per point (the
-// lanes share the candidates, every lane keeps the K best of its share).  out[s] = distance of sample s, 3e38 for a sample
-// that 4 shells do not settle (a stray point: it shall not size the grid).  All branches on r, the bound and the
-// result are uniform over the wavefront.
+// The neighbour distance of `samples` points evenly spaced in the order of the coarse grid, one wavefront per point
+// (the lanes share the candidates, every lane keeps the K best of its share).  out[s] = distance of sample s, 3e38
+// for a sample that 4 shells do not settle (a stray point: it shall not size the grid).  All branches on r, the bound
+// and the result are uniform over the wavefront.
 template <int K>
 __global__ __launch_bounds__(kBlock) void knn_sample_kernel(const float4* __restrict__ sorted, int n,
                                                             const KnnGrid* __restrict__ gp,
@@ -882,13 +885,13 @@ __global__ __launch_bounds__(kBlock) void camera_distance_kernel(const float4* _
     out[i] = sqrtf(best);
 }
 
-// The same for points in the order of the search grid: a wavefront's points lie close together, so most frames are ruled out for
-// all of them at once.  Per 64 frames, every lane takes one: a bound below the distance of its camera to any point of
-// the wavefront's bounding sphere, or none if the whole sphere lies behind the camera.  The frames then come nearest first,
-// until the next bound is above what every lane has found.  The minimum over the frames
-// that see a point does not depend on their order, and the bound leaves 1e-5 of the coordinates for rounding.
-// 3 M points of a sphere on a plane, 100 frames: 708 -> 307 us (the corners of the plane
-// are in few images, and a point no frame sees takes all of them).
+// The same for points in the order of the search grid: a wavefront's points lie close together, so most frames are
+// ruled out for all of them at once.  Per 64 frames, every lane takes one: a bound below the distance of its camera
+// to any point of the wavefront's bounding sphere, or none if the whole sphere lies behind the camera.  The frames
+// then come nearest first, until the next bound is above what every lane has found.  The minimum over the frames that
+// see a point does not depend on their order, and the bound leaves 1e-5 of the coordinates for rounding. 3 M points
+// of a sphere on a plane, 100 frames: 708 -> 307 us (the corners of the plane are in few images, and a point no frame
+// sees takes all of them).
 __global__ __launch_bounds__(kBlock) void camera_distance_sorted_kernel(const float4* __restrict__ sorted, int n,
                                                                         const ViewConst* __restrict__ views, int num_frames,
                                                                         float* __restrict__ out)
@@ -911,7 +914,8 @@ __global__ __launch_bounds__(kBlock) void camera_distance_sorted_kernel(const fl
             const ViewConst& vc = views[f0 + lane];
             const V3 r = quat_rotate(vc.qx, vc.qy, vc.qz, vc.qw, c);
             const V3 v = {r.x + vc.tx, r.y + vc.ty, r.z + vc.tz};
-            const float slack = radius * 1.0001f + 1.0e-5f * (fabsf(c.x) + fabsf(c.y) + fabsf(c.z) + radius + fabsf(vc.tx) + fabsf(vc.ty) + fabsf(vc.tz));
+            const float size  = fabsf(c.x) + fabsf(c.y) + fabsf(c.z) + radius + fabsf(vc.tx) + fabsf(vc.ty) + fabsf(vc.tz);
+            const float slack = radius * 1.0001f + 1.0e-5f * size;
             const float reach = sqrtf(dot3(v, v)) - slack;
             if (!(v.z + slack <= 0.f)) bound = reach > 0.f ? reach * reach * 0.9999f : 0.f;
         }
@@ -930,20 +934,20 @@ __global__ __launch_bounds__(kBlock) void camera_distance_sorted_kernel(const fl
 // SceneData::RemoveClosePoints (SceneData.cpp:598-642) walks the points in order and erases point i when a point it
 // has kept before lies within radius[i] of it: state[i] = kept unless a kept j < i is that close.  Here the points
 // are decided in rounds: a point whose earlier neighbours are all decided is decided; states only ever go from
-// undecided to kept / erased, so reading a neighbour's state of this round instead of the last one is as good.
-// One thread per point in cell order; count[round] receives the points still undecided after this round, and a round
-// that finds count[round - 1] == 0 has nothing to do.
-// The cells a ball can reach are those of the corners of its bounding cube: the cell of a coordinate never decreases
-// with it, in fp32 as in real numbers, and a point counts only if every |difference of coordinates| is below the radius up to
-// the rounding of four operations, which the widened reach covers (1e-4 of the radius; 1e-20 where its square
-// underflows).  The radii of the filter are a hundredth of a cell: one row of one or two cells in place of the 27 around the
-// point (3 M points in random order: 730 -> 177 us, most of it the states and radii, which are gathered by id).
-// A scene in a unit of its own has radii of many cells (the radius grows as the unit, the cells shrink): then the kernel waits
-// for the rows it looks up, one load after the other.  One flat loop over candidates, rows and bricks, so that a wavefront
-// takes as many turns as its longest lane needs of all of them together and not the longest of every row; where the ball
-// spans a brick in x the rows of a layer are one run; candidates and their states come in fours.  Whole call, cells row by
-// row / flat: 1 M points on patches, radii of 4 cells 7.0 / 4.8 ms, of a Gaussian cloud 10.7 / 8.2, on a plane and a sphere
-// 15.8 / 14.3; 3 M points with radii of a hundredth of a cell 252 / 231 us in this kernel.
+// undecided to kept / erased, so reading a neighbour's state of this round instead of the last one is as good. One
+// thread per point in cell order; count[round] receives the points still undecided after this round, and a round that
+// finds count[round - 1] == 0 has nothing to do. The cells a ball can reach are those of the corners of its bounding
+// cube: the cell of a coordinate never decreases with it, in fp32 as in real numbers, and a point counts only if
+// every |difference of coordinates| is below the radius up to the rounding of four operations, which the widened
+// reach covers (1e-4 of the radius; 1e-20 where its square underflows).  The radii of the filter are a hundredth of a
+// cell: one row of one or two cells in place of the 27 around the point (3 M points in random order: 730 -> 177 us,
+// most of it the states and radii, which are gathered by id). A scene in a unit of its own has radii of many cells
+// (the radius grows as the unit, the cells shrink): then the kernel waits for the rows it looks up, one load after
+// the other.  One flat loop over candidates, rows and bricks, so that a wavefront takes as many turns as its longest
+// lane needs of all of them together and not the longest of every row; where the ball spans a brick in x the rows of
+// a layer are one run; candidates and their states come in fours.  Whole call, cells row by row / flat: 1 M points on
+// patches, radii of 4 cells 7.0 / 4.8 ms, of a Gaussian cloud 10.7 / 8.2, on a plane and a sphere 15.8 / 14.3; 3 M
+// points with radii of a hundredth of a cell 252 / 231 us in this kernel.
 constexpr int kStateUndecided = 0, kStateKept = 1, kStateErased = 2;
 constexpr int kCloseUnroll    = 4;
 
@@ -966,7 +970,8 @@ __global__ __launch_bounds__(kBlock) void close_points_kernel(KnnView kv, int n,
             const int3 lo   = grid_cell(g, p.x - reach, p.y - reach, p.z - reach);
             const int3 hi   = grid_cell(g, p.x + reach, p.y + reach, p.z + reach);
             int result = kStateKept;
-            const int3 b0 = {lo.x >> kBrickX, lo.y >> kBrickY, lo.z >> kBrickZ}, b1 = {hi.x >> kBrickX, hi.y >> kBrickY, hi.z >> kBrickZ};
+            const int3 b0 = {lo.x >> kBrickX, lo.y >> kBrickY, lo.z >> kBrickZ};
+            const int3 b1 = {hi.x >> kBrickX, hi.y >> kBrickY, hi.z >> kBrickZ};
             int3 b        = {b0.x - 1, b0.y, b0.z};  // (no brick yet)
             int xa = 0, xb = 0, ya = 0, yb = 0, zb = -1, cy = 0, cz = 0;
             uint32_t slot = kNoBrick, q = 0, e = 0;
@@ -977,8 +982,8 @@ __global__ __launch_bounds__(kBlock) void close_points_kernel(KnnView kv, int n,
                     float4 o[kCloseUnroll];
 #pragma unroll
                     for (int u = 0; u < kCloseUnroll; ++u) o[u] = kv.sorted[min(q + u, e - 1)];
-                    // (the states of all candidates that count are requested before the first is looked at; the state of the
-                    // point itself, which is undecided and stands in for the others, is not looked at)
+                    // (the states of all candidates that count are requested before the first is looked at; the state
+                    // of the point itself, which is undecided and stands in for the others, is not looked at)
                     bool near[kCloseUnroll], any = false;
 #pragma unroll
                     for (int u = 0; u < kCloseUnroll; ++u)
@@ -1069,17 +1074,19 @@ __global__ __launch_bounds__(kBlock) void morton_kernel(const float4* __restrict
     const float fx = fminf(fmaxf((p.x - min_x) * scale_x, 0.f), m);
     const float fy = fminf(fmaxf((p.y - min_y) * scale_y, 0.f), m);
     const float fz = fminf(fmaxf((p.z - min_z) * scale_z, 0.f), m);
-    const unsigned long long c = spread21((unsigned long long)fx) | spread21((unsigned long long)fy) << 1 | spread21((unsigned long long)fz) << 2;
+    const unsigned long long c = spread21((unsigned long long)fx) | spread21((unsigned long long)fy) << 1 |
+                                 spread21((unsigned long long)fz) << 2;
     code[i] = c;
     if (key) key[i] = (int32_t)((uint32_t)(c >> 31) ^ 0x80000000u);
 }
 
-// `order` sorts the points stably by `key`, the upper half of their codes (sorted_key: the keys in that order); the points of equal
-// keys are put in the order of their whole codes, equal codes staying as they are.  The first point of a run of equal keys does it,
-// by insertion: a run is two or three points where the cloud fills its bounding box.  A run of more than kTieRun points is left
-// alone and *too_long set: the caller then sorts by whole codes.
-// 10 M points, sort and ties: by whole codes (11 passes) 974 us, by keys (6 shorter ones) 539 us in a volume, 688 on patches, 796 on a
-// plane and a sphere (more ties); 1 M: 238 against 216 to 226; 300 k: 159 against 157, and the flag is still to be read.
+// `order` sorts the points stably by `key`, the upper half of their codes (sorted_key: the keys in that order); the
+// points of equal keys are put in the order of their whole codes, equal codes staying as they are.  The first point
+// of a run of equal keys does it, by insertion: a run is two or three points where the cloud fills its bounding box.
+// A run of more than kTieRun points is left alone and *too_long set: the caller then sorts by whole codes. 10 M
+// points, sort and ties: by whole codes (11 passes) 974 us, by keys (6 shorter ones) 539 us in a volume, 688 on
+// patches, 796 on a plane and a sphere (more ties); 1 M: 238 against 216 to 226; 300 k: 159 against 157, and the flag
+// is still to be read.
 constexpr int kTieRun = 32;
 
 __global__ __launch_bounds__(kBlock) void morton_ties_kernel(const int32_t* __restrict__ sorted_key, long long* __restrict__ order,
@@ -1123,16 +1130,16 @@ void launch_knn_first_grid(const float4* position, int n, const KnnGrid& box, Kn
     hipLaunchKernelGGL(knn_first_grid_kernel, dim3(1), dim3(1024), 0, st, position, n, box, dst);
 }
 
-// The cells of the search grid as a multiple of the median distance d_R to the R-th neighbour.  Smaller cells mean fewer
-// candidates (their number goes with the square of the cell on a surface, with the cube in a volume) and more points that the
-// cube of 27 cells does not settle.  1.5 measured best over surfaces and volumes (search of 10 M points on 1000 patches,
-// 3 M in a volume, whole call: 2.0: 1365, 786 us; 1.5: 1264, 574; 1.2: 1283, 1015).  Where the samples are taken in every
-// s-th point, their nearest neighbour there stands in for the s-th in the cloud, and d_R = d_s (R / s)^(1 / D) for a cloud of
-// dimension D.  D = 2.5 is 32 % above a surface's value at R = 1, s = 16 and 17 % below a volume's, and cells too small by
-// that much leave a seventh of a volume's points unsettled; the distance to the nearest neighbour also spreads more about its
-// median than that to the 8th.  R + 1.25 in the place of R takes care of both where it matters and costs surfaces nothing
-// (6 M points in a volume, rank 1 / 2 / 4 / 8: with R 2.03, 1.87, 1.35, 1.30 ms,
-// with R + 1.25 1.05, 1.06, 1.13, 1.36; 10 M points on patches 2.07 and 2.08).
+// The cells of the search grid as a multiple of the median distance d_R to the R-th neighbour.  Smaller cells mean
+// fewer candidates (their number goes with the square of the cell on a surface, with the cube in a volume) and more
+// points that the cube of 27 cells does not settle.  1.5 measured best over surfaces and volumes (search of 10 M
+// points on 1000 patches, 3 M in a volume, whole call: 2.0: 1365, 786 us; 1.5: 1264, 574; 1.2: 1283, 1015).  Where
+// the samples are taken in every s-th point, their nearest neighbour there stands in for the s-th in the cloud, and
+// d_R = d_s (R / s)^(1 / D) for a cloud of dimension D.  D = 2.5 is 32 % above a surface's value at R = 1, s = 16 and
+// 17 % below a volume's, and cells too small by that much leave a seventh of a volume's points unsettled; the
+// distance to the nearest neighbour also spreads more about its median than that to the 8th.  R + 1.25 in the place
+// of R takes care of both where it matters and costs surfaces nothing (6 M points in a volume, rank 1 / 2 / 4 / 8:
+// with R 2.03, 1.87, 1.35, 1.30 ms, with R + 1.25 1.05, 1.06, 1.13, 1.36; 10 M points on patches 2.07 and 2.08).
 void launch_knn_refine_grid(const float* sample, int samples, int rank, int stride, const KnnGrid* first, KnnGrid* g,
                             uint32_t budget, uint32_t* list_counts, hipStream_t st)
 {

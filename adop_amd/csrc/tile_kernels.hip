@@ -269,11 +269,14 @@ __device__ __forceinline__ void add_staged(float* acc, const float* s_stage, int
     }
 }
 
-// K entries per thread and batch (BATCH = K * kBlock, a power of two).  LT as a constant and the counter pass as a variant: the
-// tile's windows took 111 scalar registers more than there are (see bin_count_kernel), now 13; 1071 -> 768 vector
-// instructions for 4 channels (a frame of 12 M points 73 -> 71 us: the kernel waits for its gathers of descriptors).
+// K entries per thread and batch (BATCH = K * kBlock, a power of two).  LT as a constant and the counter pass as a
+// variant: the tile's windows took 111 scalar registers more than there are (see bin_count_kernel), now 13; 1071 ->
+// 768 vector instructions for 4 channels (a frame of 12 M points 73 -> 71 us: the kernel waits for its gathers of
+// descriptors).
 template <int CT, bool HALF, int K, int LT, bool STATS>
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu((CT != 0 && K == 1) ? 7 : 4, 8), amdgpu_num_sgpr(96))) void tile_blend_kernel(CloudArg pc, Levels lv, ParamArg rp, BinArg bin,
+__global__ __launch_bounds__(kBlock)
+__attribute__((amdgpu_waves_per_eu((CT != 0 && K == 1) ? 7 : 4, 8), amdgpu_num_sgpr(96)))
+void tile_blend_kernel(CloudArg pc, Levels lv, ParamArg rp, BinArg bin,
                                                             float* __restrict__ accum, int S,
                                                             const float* __restrict__ background, int write_mask,
                                                             float mask_value, int identity_index, adop_stats* stats, int num_tiles)
@@ -430,7 +433,8 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu((CT != 0
                 }
                 if (miss)
                 {
-                    // coarse pixel outside the tile's window (does not happen for in-image points): blend straight to memory
+                    // coarse pixel outside the tile's window (does not happen for in-image points): blend straight to
+                    // memory
                     x = E[k].x;
                     y = E[k].y;
                     for (int l = 0; l < lv.num; ++l)
@@ -513,9 +517,9 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu((CT != 0
         }
     }
 
-    // A slice of a split bin leaves its sums for the tile's own pixels in its row; the slice that finishes last adds the
-    // K rows in their order and resolves the pixels (the coarse windows go through the global accumulators anyway).
-    // Row: per thread the C sums and the count of its first accumulator, then of its second.
+    // A slice of a split bin leaves its sums for the tile's own pixels in its row; the slice that finishes last adds
+    // the K rows in their order and resolves the pixels (the coarse windows go through the global accumulators
+    // anyway). Row: per thread the C sums and the count of its first accumulator, then of its second.
     bool resolve_own = true;
     if (slices > 1)  // (workgroup-uniform)
     {
