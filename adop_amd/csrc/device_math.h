@@ -334,8 +334,9 @@ __device__ __forceinline__ V3 ocam_unproject(const float* aff, const float* poly
 // 3e-6 of (|p| + |c|) |n|, |n|^2 <= 3.  Only the points between take the form of the reference with its second
 // rotation.  For a kernel that is bound by its vector instructions: wavefronts of Morton-ordered points are mostly
 // culled as a whole. First binning pass, before / after: 8 fisheye views of 20 M points 1184 / 908 us, 16 pinhole
-// crops of 10 M 300 / 294. Not for the prepass, which waits for its early-z reads and atomics: 2.8 M unordered points
-// on 416 x 151 pixels, fisheye, 310 us without, 377 with it; 1.4 M points without normals 77 / 86.
+// crops of 10 M 300 / 294. Not for the prepass, which waits for its early-z reads and atomics where many
+// points share few pixels: 2.8 M unordered points on 416 x 151 pixels, fisheye, 310 us without, 377 with it; 1.4 M
+// points without normals 77 / 86.
 template <bool FACE_FIRST = false>
 __device__ __forceinline__ bool project_frame(const ViewConst& vc, const float* __restrict__ intrinsics, V3 pos, V3 nrm,
                                               bool check_normal, float dist_cutoff, V2* image_p_out, float* z_out,

@@ -66,11 +66,13 @@ __global__ __launch_bounds__(kBlock) void clear_kernel(Levels lv, int first_leve
 }
 
 // DepthPrepassMulti (PointRenderer.cu:203-301) on the packed buffer the reference keeps as "old rendering"
-// (LayerCuda::depth_index_tensor, PackIndex): min over (depth bits << 32 | point id). Every thread handles PPT points
-// (all their loads are issued before anything waits: the kernel is bound by memory latency, not by arithmetic).  Per
-// level and 64-point run the lanes that survive the early-z read are grouped by pixel, one lane per distinct pixel
-// takes the minimum of its group from LDS and issues the 64-bit atomicMin: clouds stored in Morton-ordered blocks
-// collide heavily at the coarse levels, and a device-scope atomic costs one memory transaction whatever it carries.
+// (LayerCuda::depth_index_tensor, PackIndex): min over (depth bits << 32 | point id). Every thread handles PPT points,
+// all their loads issued before anything waits.  What bounds it: vector issue on a large cloud spread over the image
+// (100 M points on 1920 x 1080: 550 M instructions, 0.90 of 1.07 ms), the round trips of the early-z reads and the
+// atomics where many points share few pixels.  Per level and 64-point run the lanes that survive the early-z read are
+// grouped by pixel, one lane per distinct pixel takes the minimum of its group from LDS and issues the 64-bit
+// atomicMin: clouds stored in Morton-ordered blocks collide heavily at the coarse levels, and a device-scope atomic
+// costs one memory transaction whatever it carries.
 // The counters are a branch at run time, not a variant as in the other kernels: with the shorter code of a variant
 // more wavefronts read a depth before the first of them has lowered it, and they issue redundant atomics (1.4 M
 // points on a few hundred pixels, fisheye: 255 us with the branch, 267 without; 100 M points on 1920 x 1080 do not

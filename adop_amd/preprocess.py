@@ -4,7 +4,9 @@ blocks sorted by radius.
 
 The order of the cloud and the radii decide how the rasterizer runs (coherent wavefronts, the LOD early exit), so the
 steps sit next to it.  The distance search and the Morton codes are HIP kernels behind the C-ABI
-(``adop_knn_distance``, ``adop_morton_codes``, ``adop_point_distance_to_camera``, ``adop_close_points``); sorting and permuting go through torch.
+(``adop_knn_distance``, ``adop_morton_codes``, ``adop_point_distance_to_camera``, ``adop_close_points``), and so are the
+passes that move whole points (``adop_gather_points``, ``adop_shuffle_points``, ``adop_radius_blocks``); torch sorts and
+draws the random numbers.
 """
 import ctypes as C
 

@@ -176,9 +176,9 @@ def bench_preprocess(args):
         if name == "camera_distance_100_frames":
             cam = r
         filt[name] = round(sorted(ts)[1], 3)
-    # algorithmic bytes of the neighbour search: the cloud is read twice and written once in cell order (binning),
-    # read once more by the search, 4 bytes per point out; neighbours are read through the caches (the library bins
-    # twice, for its first and second grid: its choice, not the algorithm's)
+    # algorithmic bytes of the neighbour search, a whole call: the cloud is read twice and written once in cell order
+    # (binning), read once more by the search, 4 bytes per point out; neighbours are read through the caches (that the
+    # library bins in two steps, bricks and the cells inside them, is its choice, not the algorithm's)
     knn_bytes = N * (16 + 16 + 16 + 16 + 4)
     cpu = None
     if not args.no_cpu_baseline:
@@ -197,7 +197,7 @@ def bench_preprocess(args):
         "scaling": "weak", "vs_baseline": None, "dtype": "f32", "data": "synthetic",
         "config": {"workload": f"preprocess: 4th-nearest-neighbour distance + Morton codes, {N} points of config3 in "
                                "random order"},
-        "roofline": {"bound": "hbm", "kernel": "knn_search_kernel", "stage": "knn_distance",
+        "roofline": {"bound": "hbm", "kernel": "adop_knn_distance, all kernels of a call", "stage": "knn_distance",
                      "achieved": round(knn_bytes / (t_knn * 1e-3) / 1e9, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": round(knn_bytes / (t_knn * 1e-3) / 1e9 / HBM_PEAK_GBS, 4), "traffic": None,
                      "kernel_ms": round(t_knn, 4), "algorithmic_bytes": int(knn_bytes)},
