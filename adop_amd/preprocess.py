@@ -41,7 +41,8 @@ def _box_and_stretch(position):
     lib = _capi.load_library()
     box = torch.empty(int(lib.adop_bounding_box_size()) // 4, dtype=torch.float32, device=position.device)
     _check(lib.adop_bounding_box(_ptr(position), int(position.shape[0]), _ptr(box), _stream_ptr()), lib)
-    lo, hi, part_lo, part_hi = (box[:12].tolist()[k:k + 3] for k in (0, 3, 6, 9))
+    host = box[:12].tolist()  # (one read: the host waits in it)
+    lo, hi, part_lo, part_hi = host[:3], host[3:6], host[6:9], host[9:]
     stretch = max((b - a) / (d - c) if d > c else 1.0 for a, b, c, d in zip(lo, hi, part_lo, part_hi))
     return ((C.c_float * 3)(*lo), (C.c_float * 3)(*hi)), stretch
 

@@ -298,6 +298,7 @@ def BlendPointCloudForward(ctx, info, build=True):
         ctx.dropout_points = cache.dropout_points
         ctx.point_cache = cache.point_cache
         ctx.pixel_cache = cache.pixel_cache
+        ctx.workspace_key = cache._workspace_key
         ctx.depth_index = [L.depth_index_tensor for L in cache.layers_cuda]
         ctx.masks = list(cache.output_forward_background_mask)
     return list(cache.output_forward), list(cache.output_forward_background_mask)
@@ -350,7 +351,9 @@ def BlendPointCloudBackward(ctx, info, image_gradients, needs=(True, True, True)
 
     cache.num_batches = len(info.images)
     cache.info = info
-    cache.take_workspace(info)
+    key = getattr(ctx, "workspace_key", None)  # of the forward pass: mostly the last pass of the cache, on this stream
+    if key is None or key is not cache._workspace_key or key[8] != _raw_stream() or torch.cuda.is_current_stream_capturing():
+        cache.take_workspace(info)
     s = scene.struct()
     stats = C.c_void_p(cache.stats.data_ptr()) if info.collect_stats else None
     info.params.workspace_flags = int(info.workspace_flags)
