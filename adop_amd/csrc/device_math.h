@@ -337,7 +337,7 @@ __device__ __forceinline__ V3 ocam_unproject(const float* aff, const float* poly
 // crops of 10 M 300 / 294. Not for the prepass, which waits for its early-z reads and atomics where many
 // points share few pixels: 2.8 M unordered points on 416 x 151 pixels, fisheye, 310 us without, 377 with it; 1.4 M
 // points without normals 77 / 86.
-template <bool FACE_FIRST = false>
+template <bool FACE_FIRST>
 __device__ __forceinline__ bool project_frame(const ViewConst& vc, const float* __restrict__ intrinsics, V3 pos, V3 nrm,
                                               bool check_normal, float dist_cutoff, V2* image_p_out, float* z_out,
                                               V3* view_p_out)
@@ -464,7 +464,9 @@ __device__ __forceinline__ bool project_point(const ViewConst& vc, const float* 
 {
     V2 image_p;
     *radius_pixels = 0;
-    if (!project_frame(vc, intrinsics, pos, nrm, check_normal, dist_cutoff, &image_p, z_out, view_p_out)) return false;
+    // (blend and gradient kernels look at points that mostly face the camera: the early test spares them the second
+    // rotation; spatial gradients of 390 k unordered points in 3 views, 3 channels: 88 us without, 79 with it)
+    if (!project_frame<true>(vc, intrinsics, pos, nrm, check_normal, dist_cutoff, &image_p, z_out, view_p_out)) return false;
     project_crop(vc, image_p, *z_out, radius, w0, ip, radius_pixels);
     return true;
 }

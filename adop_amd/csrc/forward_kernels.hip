@@ -130,7 +130,9 @@ __global__ __launch_bounds__(kBlock) void prepass_kernel(CloudArg pc, const View
             V3 view_p;
             V2 frame_p = {0.f, 0.f};
             float z    = 0.f;
-            if (valid) project_frame(vc, pc.intrinsics, pos, nrm, rp.check_normal != 0, rp.dist_cutoff, &frame_p, &z, &view_p);
+            if (valid)
+                project_frame<false>(vc, pc.intrinsics, pos, nrm, rp.check_normal != 0, rp.dist_cutoff, &frame_p, &z,
+                                     &view_p);
             const bool ok = z != 0;
             if (ok) ip = k_apply(vc.crop, frame_p);
             // a crop sees a small part of the cloud: most runs of 64 points are nowhere near it and skip the levels
