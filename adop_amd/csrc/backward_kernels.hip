@@ -291,7 +291,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(CT != 0 
                 V3 nrm   = {0, 0, 0};
                 if (valid && pc.normal) nrm = unpack_normal10(pc.normal[i]);
                 V3 view_p;
-                ok = valid && project_point(vc, pc.intrinsics, pos, nrm, P.w, rp.check_normal != 0, rp.dist_cutoff, lv.l[0].w,
+                ok = valid && project_point<false>(vc, pc.intrinsics, pos, nrm, P.w, rp.check_normal != 0, rp.dist_cutoff, lv.l[0].w,
                                             &ip, &z, &radius_pixels, &view_p);
             }
             ok = ok && tex_in_range;

@@ -458,6 +458,7 @@ __device__ __forceinline__ bool outside_every_level(const ImageBox& box, V2 ip)
     return ip.x < box.lo || ip.x > box.hi_x || ip.y < box.lo || ip.y > box.hi_y;
 }
 
+template <bool FACE_FIRST = true>
 __device__ __forceinline__ bool project_point(const ViewConst& vc, const float* __restrict__ intrinsics, V3 pos,
                                               V3 nrm, float radius, bool check_normal, float dist_cutoff, int w0,
                                               V2* ip, float* z_out, float* radius_pixels, V3* view_p_out)
@@ -465,8 +466,10 @@ __device__ __forceinline__ bool project_point(const ViewConst& vc, const float* 
     V2 image_p;
     *radius_pixels = 0;
     // (blend and gradient kernels look at points that mostly face the camera: the early test spares them the second
-    // rotation; spatial gradients of 390 k unordered points in 3 views, 3 channels: 88 us without, 79 with it)
-    if (!project_frame<true>(vc, intrinsics, pos, nrm, check_normal, dist_cutoff, &image_p, z_out, view_p_out)) return false;
+    // rotation; spatial gradients of 390 k unordered points in 3 views, 3 channels: 88 us without, 79 with it.  Not the
+    // descriptor pass, which has no register for it: 186 MB of parked registers more for 16 crops of 10 M points)
+    if (!project_frame<FACE_FIRST>(vc, intrinsics, pos, nrm, check_normal, dist_cutoff, &image_p, z_out, view_p_out))
+        return false;
     project_crop(vc, image_p, *z_out, radius, w0, ip, radius_pixels);
     return true;
 }
