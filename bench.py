@@ -48,18 +48,18 @@ KERNEL_OF_STAGE = {"BinCount": "bin_count_kernel", "BinScatter": "bin_scatter_ke
 # x 1.0 after calibration with plain device copies of known size), per workload.  "sources" is kernel_sources_state() of
 # the tree the profile was taken on (python bench.py --print-sources-state): the figures are quoted for that state only.
 MEASURED_TRAFFIC = {
-    "config3": {"sources": "107acb526a89", "profile": "profiles/config3_tile_path_fwd_bwd_kernels_traffic_instructions.md",
-                "bytes": {"RenderBackward/descriptor": 860.1e6, "RenderBackward/spatial": 572.1e6, "TileBlend": 525.3e6, "BinCount": 430.3e6, "BinScatter": 197.4e6, "CombineAndFillBackward": 220.8e6, "TileDepth": 101.5e6, "Post Process Gradient": 0.5e6, "CombineAndFill": 23.6e6, "Initialize": 11.8e6}},
-    "config1": {"sources": "107acb526a89", "profile": "profiles/config1_direct_path_forward_kernels_traffic_instructions.md",
+    "config3": {"sources": "ae821088fc52", "profile": "profiles/config3_tile_path_fwd_bwd_kernels_traffic_instructions.md",
+                "bytes": {"RenderBackward/descriptor": 860.1e6, "RenderBackward/spatial": 569.8e6, "TileBlend": 525.3e6, "BinCount": 430.3e6, "BinScatter": 197.4e6, "CombineAndFillBackward": 220.8e6, "TileDepth": 101.5e6, "Post Process Gradient": 0.5e6, "CombineAndFill": 23.5e6, "Initialize": 11.8e6}},
+    "config1": {"sources": "ae821088fc52", "profile": "profiles/config1_direct_path_forward_kernels_traffic_instructions.md",
                 "bytes": {"DepthPrepass": 13.1e6, "RenderForward": 8.5e6, "CombineAndFill": 5.6e6, "Initialize": 3.5e6}},
-    "config2": {"sources": "107acb526a89", "profile": "profiles/config2_fwd_bwd_kernels_traffic_instructions.md",
-                "bytes": {"RenderBackward/descriptor": 200.7e6, "TileBlend": 162.3e6, "RenderBackward/spatial": 146.2e6, "BinScatter": 67.5e6, "BinCount": 64.4e6, "CombineAndFillBackward": 67.3e6, "TileDepth": 37.9e6, "Post Process Gradient": 15.1e6, "Initialize": 3.4e6, "CombineAndFill": 6.6e6}},
-    "config4": {"sources": "107acb526a89", "profile": "profiles/config4_direct_path_forward_kernels_traffic_instructions.md",
-                "bytes": {"DepthPrepass": 5081.6e6, "RenderForward": 1547.2e6, "CombineAndFill": 176.8e6, "Initialize": 110.5e6}},
+    "config2": {"sources": "ae821088fc52", "profile": "profiles/config2_fwd_bwd_kernels_traffic_instructions.md",
+                "bytes": {"RenderBackward/descriptor": 200.7e6, "TileBlend": 162.1e6, "RenderBackward/spatial": 146.2e6, "BinScatter": 67.5e6, "BinCount": 64.4e6, "CombineAndFillBackward": 67.3e6, "TileDepth": 37.9e6, "Post Process Gradient": 15.1e6, "Initialize": 3.4e6, "CombineAndFill": 6.6e6}},
+    "config4": {"sources": "ae821088fc52", "profile": "profiles/config4_direct_path_forward_kernels_traffic_instructions.md",
+                "bytes": {"DepthPrepass": 5081.8e6, "RenderForward": 1546.3e6, "CombineAndFill": 176.8e6, "Initialize": 110.5e6}},
     "config5": {"sources": "107acb526a89", "profile": "profiles/config5_ocam_envmap_fwd_bwd_kernels_traffic_instructions.md",
                 "bytes": {"RenderBackward/spatial": 5753.2e6, "TileBlend": 5062.6e6, "EnvironmentMapBackward": 2242.7e6, "RenderBackward/descriptor": 4092.3e6, "EnvironmentMap": 2213.4e6, "BinCount": 2191.2e6, "BinScatter": 3331.7e6, "TileDepth": 1622.9e6, "CombineAndFillBackward": 1869.7e6, "Post Process Gradient": 484.7e6, "CombineAndFill": 177.1e6, "Initialize": 83.1e6}},
-    "crops": {"sources": "107acb526a89", "profile": "profiles/training_batch_16_crops_fwd_bwd_kernels_traffic_instructions.md",
-                "bytes": {"RenderBackward/descriptor": 1580.0e6, "RenderBackward/spatial": 1242.0e6, "BinCount": 587.0e6, "TileBlend": 1208.0e6, "BinScatter": 764.7e6, "CombineAndFillBackward": 446.2e6, "TileDepth": 249.2e6, "Post Process Gradient": 120.3e6, "CombineAndFill": 47.9e6, "Initialize": 23.7e6}},
+    "crops": {"sources": "ae821088fc52", "profile": "profiles/training_batch_16_crops_fwd_bwd_kernels_traffic_instructions.md",
+                "bytes": {"RenderBackward/descriptor": 1579.9e6, "RenderBackward/spatial": 1223.1e6, "BinCount": 587.0e6, "TileBlend": 1208.3e6, "BinScatter": 764.7e6, "CombineAndFillBackward": 446.2e6, "TileDepth": 249.2e6, "Post Process Gradient": 120.3e6, "CombineAndFill": 47.9e6, "Initialize": 23.7e6}},
 }
 
 
